@@ -508,7 +508,7 @@ def tolerance(case):
             return {"rel": 2.0e-2}  # r1..r6: differences of rounded velocities
         if case["storage"] == "fp16":
             return {"rel": 8.0e-3}
-        if case.get("q", True):
+        if case.get("q", True) or case.get("topo"):
             return {"rel": 6.0e-4}
     return {"rel": 1.0e-5}
 
