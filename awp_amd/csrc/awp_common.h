@@ -63,7 +63,7 @@ __device__ __forceinline__ int awp_xcd_remap(int b, int nblocks) {
 
 static inline int awp_cdiv(int a, int b) { return (a + b - 1) / b; }
 
-// k-run width of the (k, j)-tiled kernels: a wave covers 64 consecutive k of
+// k-run width of the plasticity kernels: a wave covers 64 consecutive k of
 // one j row, or 32 consecutive k of each of two j rows when that leaves at
 // least 16 fewer lanes idle per column of n levels (n = 96 fills 2 x 64
 // lanes to 75 % but 3 x 32 to 100 %).  forced: 32 or 64 from the tuning,
@@ -72,6 +72,53 @@ static inline int awp_pick_kw(int n, int forced) {
   if (forced == 32 || forced == 64) return forced;
   const int idle64 = awp_cdiv(n, 64) * 64 - n, idle32 = awp_cdiv(n, 32) * 32 - n;
   return idle64 - idle32 >= 16 ? 32 : 64;
+}
+
+// (k, j) tile of the marching Cartesian kernels: a workgroup of `lanes` lanes
+// covers `rows` j rows of `width` consecutive k each, lane t being row
+// t / width and level t % width, `nkt` tiles down a column of n levels.
+// The width is the one that leaves the fewest lanes idle: a column that is
+// not a multiple of 64 is cut into equal runs and the lanes they free take
+// further rows (n = 101: 2 runs of 51 levels of 5 rows, 505 of 512 lanes,
+// against 404 with 64-level runs of 4 rows).  Runs stay at 32 levels (one
+// 128-byte line) or more; equal counts go to the width nearest 64, so
+// columns of 64 m levels keep whole-line waves of one row each.  Where rows
+// are whole lines (yline a multiple of 32 floats) only widths that are too
+// are taken, unless they cost 12 % more lanes: a run's edge line is then
+// fetched by two tiles.
+struct AwpTile {
+  int width, rows, nkt, mul;  // mul: t / width = t * mul >> 20 for t < 1024
+};
+static inline AwpTile awp_pick_tile(int n, int lanes, int yline, int forced) {
+  AwpTile best = {64, lanes / 64, awp_cdiv(n, 64), 0};
+  if (forced == 32 || forced == 64) {
+    best.width = forced;
+    best.rows = lanes / forced;
+    best.nkt = awp_cdiv(n, forced);
+  } else {
+    float cost = 1e30f;
+    const int most = lanes < 256 ? lanes : 256;
+    for (int nkt = awp_cdiv(n, most); nkt <= awp_cdiv(n, 32); ++nkt)
+      for (int al = 0; al < 2; ++al) {
+        int w = awp_cdiv(n, nkt);
+        if (al) w = awp_cdiv(w, 32) * 32;
+        if (w < 32) w = 32;
+        if (w > most) continue;
+        const int rows = lanes / w, nt = awp_cdiv(n, w);
+        float c = (float)(nt * lanes) / (float)(n * rows);
+        if (yline % 32 == 0 && w % 32 != 0) c *= 1.12f;
+        const int d = w < 64 ? 64 - w : w - 64, db = best.width < 64 ? 64 - best.width
+                                                                     : best.width - 64;
+        if (c < cost * 0.999f || (c < cost * 1.001f && d < db)) {
+          cost = c;
+          best.width = w;
+          best.rows = rows;
+          best.nkt = nt;
+        }
+      }
+  }
+  best.mul = ((1 << 20) + best.width - 1) / best.width;
+  return best;
 }
 
 // The reference's (float)(c / (double)x) for binary32 c and x.  Rounding the

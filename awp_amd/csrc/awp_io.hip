@@ -8,15 +8,16 @@
 #include "awp_tuning.h"
 #include "../../include/awp_hip.h"
 
-// Defaults from sweeps on MI355X at 512x512x256: velocity 4 rows x 2 i-chunks
-// (all workgroups resident), stress 16 rows x ~32-plane i-chunks; the
+// Defaults from sweeps on MI355X: velocity and stress workgroups of 4 waves in
+// the chunks of awp_split_march (16-wave stress workgroups, of which a CU
+// holds one, took 951 against 832 us at 384x384x256 in bfloat16 storage); the
 // curvilinear velocity update as three launches (0.985 against 1.043 ms for
 // one launch at 384x384x192), its strain-rate pass as three (normal rates,
 // xy, xz and yz: 2.056 -> 2.006 -> 1.948 ms per stress update for one, two,
 // three launches), the velocity waves ordering their LDS at wave scope
 // (1.002 -> 0.971 ms); the adjoint kernels' blocks in groups of 8 j tiles over
 // all planes (adj_stress_local 551 -> 533 us at 256x256x128).
-static AwpTuning g_tuning = {4, 16, 1024, 2048, 0, 0, 1, 1, 8, 16, 1, 32, 2048, 0, 0, 0, 1, 8, 2, 0, 8, 1, 0};
+static AwpTuning g_tuning = {4, 4, 10240, 10240, 0, 0, 1, 1, 8, 16, 1, 32, 2048, 0, 0, 0, 1, 8, 2, 0, 8, 1, 0};
 AwpTuning& awp_tuning() { return g_tuning; }
 
 namespace {

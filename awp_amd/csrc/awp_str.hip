@@ -11,6 +11,7 @@
 // Operation order and literal types follow the reference (double-literal
 // sub-expressions are evaluated in double), built with -ffp-contract=off.
 #include "awp_common.h"
+#include "awp_math.h"
 #include "awp_store.h"
 #include "awp_tuning.h"
 #include "../../include/awp_hip.h"
@@ -20,35 +21,32 @@ namespace {
 struct StrLaunch {
   int kb, k0, k1, j0, j1, i0;  // kb: k of lane 0 in tile 0; [k0, k1] active
   int nkt, njt, ichunk, ni, nblocks, remap, jfast;
+  AwpTile tile;
   int yline;
   long long slice;
   float c1, c2, dth, dh1, DT;
 };
 
-// Production Q weight (kernel.cu:978-1045).
-__device__ __forceinline__ float qw_prod(float q, float ca, float cb, float wwo) {
-  float w;
-  const double q2 = (double)q * 2.0;
-  if (1. / q2 <= 200.0)
-    w = (float)((double)ca * (2. * (double)q) * (2. * (double)q) + (double)cb * (2. * (double)q));
-  else
-    w = 2.0f * wwo * q;
-  return w / wwo;
+// Production Q weight (kernel.cu:978-1045), y = awp_rcp(wwo).  Both branches
+// are cheaper than a divergent branch around either, so they are selected.
+__device__ __forceinline__ float qw_prod(float q, float ca, float cb, float wwo, float y) {
+  const double t = 2. * (double)q;
+  const float quad = (float)((double)ca * t * t + (double)cb * t);
+  return awp_div_by(awp_q_low64(q) ? quad : 2.0f * wwo * q, wwo, y);
 }
 
 // dstrqc_new's Q weights (kernel.cu:505-604): float test; qpa keeps a double
 // quadratic, the others are float.
-__device__ __forceinline__ float qw_new(float q, float ca, float cb, float wwo, bool dbl) {
-  float w;
-  if (1.0f / (q * 2.0f) <= 200.0f) {
-    if (dbl)
-      w = (float)((double)ca * (2. * (double)q) * (2. * (double)q) + (double)cb * (2. * (double)q));
-    else
-      w = ca * (2.0f * q) * (2.0f * q) + cb * (2.0f * q);
+__device__ __forceinline__ float qw_new(float q, float ca, float cb, float wwo, float y,
+                                        bool dbl) {
+  float quad;
+  if (dbl) {
+    const double t = 2. * (double)q;
+    quad = (float)((double)ca * t * t + (double)cb * t);
   } else {
-    w = 2.0f * wwo * q;
+    quad = ca * (2.0f * q) * (2.0f * q) + cb * (2.0f * q);
   }
-  return w / wwo;
+  return awp_div_by(awp_q_low32(q) ? quad : 2.0f * wwo * q, wwo, y);
 }
 
 // OOP: the stresses before the step are read from s0 (xx yy zz xy xz yz) and
@@ -76,8 +74,7 @@ struct TexTable {
   int xls, yls, nj, nzt;         // TEX_RULE only
 };
 
-// KW: k-run width (awp_pick_kw); with KW = 32 a wave covers two j rows.
-template <int BJ, bool NEWLIT, bool OOP, class ST, int TEX = TEX_ARRAYS, int KW = 64>
+template <int BJ, bool NEWLIT, bool OOP, class ST, int TEX = TEX_ARRAYS>
 __global__ __launch_bounds__(64 * BJ) void dstrqc_kernel(
     typename ST::T* __restrict__ xx, typename ST::T* __restrict__ yy,
     typename ST::T* __restrict__ zz, typename ST::T* __restrict__ xy,
@@ -94,21 +91,23 @@ __global__ __launch_bounds__(64 * BJ) void dstrqc_kernel(
     const float* __restrict__ vx2, const int* __restrict__ ww, const float* __restrict__ wwo,
     const StrLaunch L, const WaveScales SC, const TexTable TT) {
   __shared__ float s_coeff[16];
-  __shared__ float s_tex[24];
-  const int tid = threadIdx.y * 64 + threadIdx.x;
+  __shared__ float s_tex[32];  // vx1[8], vx2[8], wwo[8], 1/wwo[8]
+  const int tid = (int)threadIdx.x;
   if (tid < 16) s_coeff[tid] = coeff[tid];
-  if (TEX != TEX_ARRAYS && tid < 24)
-    s_tex[tid] = tid < 8 ? TT.vx1[tid] : tid < 16 ? TT.vx2[tid - 8] : TT.wwo[tid - 16];
+  if (TEX != TEX_ARRAYS && tid < 32)
+    s_tex[tid] = tid < 8    ? TT.vx1[tid]
+                 : tid < 16 ? TT.vx2[tid - 8]
+                 : tid < 24 ? TT.wwo[tid - 16]
+                            : awp_rcp(TT.wwo[tid - 24]);
   __syncthreads();
 
   const int b = L.remap ? awp_xcd_remap(blockIdx.x, L.nblocks) : (int)blockIdx.x;
   int kt, jt, ic;
   awp_tile3(b, L.nkt, L.njt, L.jfast, kt, jt, ic);
-  constexpr int RW = 64 / KW;  // j rows per wave
-  const int lane = (int)threadIdx.x;
-  const int k = L.kb + kt * KW + (KW == 64 ? lane : lane % KW);
-  const int j = L.j0 + (jt * BJ + (int)threadIdx.y) * RW + (KW == 64 ? 0 : lane / KW);
-  if (k < L.k0 || k > L.k1 || j > L.j1) return;
+  const int lr = tid * L.tile.mul >> 20;  // row of this lane in the tile (awp_pick_tile)
+  const int k = L.kb + kt * L.tile.width + (tid - lr * L.tile.width);
+  const int j = L.j0 + jt * L.tile.rows + lr;
+  if (lr >= L.tile.rows || k < L.k0 || k > L.k1 || j > L.j1) return;
   const int ia = L.i0 + ic * L.ichunk;
   int nsteps = L.ni - ic * L.ichunk;
   if (nsteps > L.ichunk) nsteps = L.ichunk;
@@ -166,11 +165,12 @@ __global__ __launch_bounds__(64 * BJ) void dstrqc_kernel(
     const float w_jp1 = ST::ld(wp, o + Y, sw), w_jp2 = ST::ld(wp, o + 2 * Y, sw), w_jm1 = ST::ld(wp, o - Y, sw);
 
     const long long p = pl + o;
-    float f_vx1, f_vx2, f_wwo;
+    float f_vx1, f_vx2, f_wwo, r_wwo;  // r_wwo: 1 / wwo
     int f_ww;
     if (TEX == TEX_ARRAYS) {
       f_vx1 = vx1[p]; f_vx2 = vx2[p]; f_wwo = wwo[p];
       f_ww = ww[p];
+      r_wwo = awp_rcp(f_wwo);
     } else {
       if (TEX == TEX_TABLE) {
         f_ww = ww[p];
@@ -181,6 +181,7 @@ __global__ __launch_bounds__(64 * BJ) void dstrqc_kernel(
       }
       const int t = (f_ww - 1) & 7;
       f_vx1 = s_tex[t]; f_vx2 = s_tex[8 + t]; f_wwo = s_tex[16 + t];
+      r_wwo = s_tex[24 + t];
     }
     const float ca = s_coeff[(f_ww * 2 - 2) & 15], cb = s_coeff[(f_ww * 2 - 1) & 15];
     const float f_dcrj = dcrjx[i] * dy * dz;
@@ -189,41 +190,34 @@ __global__ __launch_bounds__(64 * BJ) void dstrqc_kernel(
     const float sm8 = mc + Mc + mjm + Mjm + mkm + Mkm + mjk + Mjk;
     const float sp8 = pc + Pc + pjm + Pjm + pkm + Pkm + pjk + Pjk;
     const float ss8 = sc + Sc + sjm + Sjm + skm + Skm + sjk + Sjk;
-    float xl, xm, xmu1, xmu2, xmu3, qpa, h, h1, h2, h3, qpaw, hw, h1w, h2w, h3w;
+    float xm = awp_pow2_div(16.0f, sm8);
+    float xl = awp_pow2_div(8.0f, sl8) + xm;
+    float xmu1 = awp_pow2_div(2.0f, mc + mkm);
+    float xmu2 = awp_pow2_div(2.0f, mc + mjm);
+    float xmu3 = awp_pow2_div(2.0f, mc + Mc);
+    float qpa, h, h1, h2, h3, qpaw, hw, h1w, h2w, h3w;
     if (!NEWLIT) {
-      xl = awp_quot(8.0f, sl8);
-      xm = awp_quot(16.0f, sm8);
-      xmu1 = awp_quot(2.0f, mc + mkm);
-      xmu2 = awp_quot(2.0f, mc + mjm);
-      xmu3 = awp_quot(2.0f, mc + Mc);
-      xl = xl + xm;
       qpa = 0.0625f * sp8;
-      qpaw = qw_prod(qpa, ca, cb, f_wwo);
+      qpaw = qw_prod(qpa, ca, cb, f_wwo, r_wwo);
       h = 0.0625f * ss8;
-      hw = qw_prod(h, ca, cb, f_wwo);
+      hw = qw_prod(h, ca, cb, f_wwo, r_wwo);
       h1 = 0.250f * (sc + skm);
-      h1w = qw_prod(h1, ca, cb, f_wwo);
+      h1w = qw_prod(h1, ca, cb, f_wwo, r_wwo);
       h2 = 0.250f * (sc + sjm);
-      h2w = qw_prod(h2, ca, cb, f_wwo);
+      h2w = qw_prod(h2, ca, cb, f_wwo, r_wwo);
       h3 = 0.250f * (sc + Sc);
-      h3w = qw_prod(h3, ca, cb, f_wwo);
+      h3w = qw_prod(h3, ca, cb, f_wwo, r_wwo);
     } else {
-      xl = 8.0f / sl8;
-      xm = 16.0f / sm8;
-      xmu1 = 2.0f / (mc + mkm);
-      xmu2 = awp_quot(2.0f, mc + mjm);
-      xmu3 = awp_quot(2.0f, mc + Mc);
-      xl = xl + xm;
       qpa = 0.0625f * sp8;
-      qpaw = qw_new(qpa, ca, cb, f_wwo, true);
+      qpaw = qw_new(qpa, ca, cb, f_wwo, r_wwo, true);
       h = 0.0625f * ss8;
-      hw = qw_new(h, ca, cb, f_wwo, false);
+      hw = qw_new(h, ca, cb, f_wwo, r_wwo, false);
       h1 = 0.250f * (sc + skm);
-      h1w = qw_new(h1, ca, cb, f_wwo, false);
+      h1w = qw_new(h1, ca, cb, f_wwo, r_wwo, false);
       h2 = 0.250f * (sc + sjm);
-      h2w = qw_new(h2, ca, cb, f_wwo, false);
+      h2w = qw_new(h2, ca, cb, f_wwo, r_wwo, false);
       h3 = 0.250f * (sc + Sc);
-      h3w = qw_new(h3, ca, cb, f_wwo, false);
+      h3w = qw_new(h3, ca, cb, f_wwo, r_wwo, false);
     }
     h = -xm * hw * dh1;
     h1 = -xmu1 * h1w * dh1;
@@ -417,35 +411,26 @@ void dstrqc_common(const char* W, void* const* f15, const CStress6& S0, float* l
   L.jfast = awp_tuning().str_jfast;
   if (L.k1 < L.k0) return;
   const int bj = awp_tuning().str_bj;
-  const int kw = awp_pick_kw(L.k1 - L.kb + 1, awp_tuning().kw);
-  L.nkt = awp_cdiv(L.k1 - L.kb + 1, kw);
-  L.njt = awp_cdiv(L.j1 - L.j0 + 1, bj * (64 / kw));
+  L.tile = awp_pick_tile(L.k1 - L.kb + 1, 64 * bj, g.yline, awp_tuning().kw);
+  L.nkt = L.tile.nkt;
+  L.njt = awp_cdiv(L.j1 - L.j0 + 1, L.tile.rows);
   int nic, ichunk;
-  awp_split_i(L.ni, L.nkt * L.njt, awp_tuning().str_ichunk, awp_tuning().str_target_wgs, &nic, &ichunk);
+  awp_split_march(L.ni, L.nkt * L.njt, awp_tuning().str_ichunk, awp_tuning().str_target_wgs, &nic,
+                  &ichunk);
   L.ichunk = ichunk;
   L.nblocks = L.nkt * L.njt * nic;
 #define AWP_STR_ARGS                                                                          \
   A[0], A[1], A[2], A[3], A[4], A[5], S0, A[6], A[7], A[8], A[9], A[10], A[11], A[12], A[13], \
       A[14], lam, mu, qp, coeff, qs, dcrjx, dcrjy, dcrjz, vx1, vx2, ww, wwo, L, SC, TT
-#define AWP_STR_LAUNCH(B, KW)                                                               \
-  hipLaunchKernelGGL((dstrqc_kernel<B, NEWLIT, OOP, ST, TEX, KW>), dim3(L.nblocks), dim3(64, B), \
+#define AWP_STR_LAUNCH(B)                                                                    \
+  hipLaunchKernelGGL((dstrqc_kernel<B, NEWLIT, OOP, ST, TEX>), dim3(L.nblocks), dim3(64 * B), \
                      0, St, AWP_STR_ARGS)
-  if (kw == 32) {
-    switch (bj) {
-      case 1: AWP_STR_LAUNCH(1, 32); break;
-      case 2: AWP_STR_LAUNCH(2, 32); break;
-      case 4: AWP_STR_LAUNCH(4, 32); break;
-      case 8: AWP_STR_LAUNCH(8, 32); break;
-      default: AWP_STR_LAUNCH(16, 32); break;
-    }
-  } else {
-    switch (bj) {
-      case 1: AWP_STR_LAUNCH(1, 64); break;
-      case 2: AWP_STR_LAUNCH(2, 64); break;
-      case 4: AWP_STR_LAUNCH(4, 64); break;
-      case 8: AWP_STR_LAUNCH(8, 64); break;
-      default: AWP_STR_LAUNCH(16, 64); break;
-    }
+  switch (bj) {
+    case 1: AWP_STR_LAUNCH(1); break;
+    case 2: AWP_STR_LAUNCH(2); break;
+    case 8: AWP_STR_LAUNCH(8); break;
+    case 16: AWP_STR_LAUNCH(16); break;
+    default: AWP_STR_LAUNCH(4); break;
   }
 #undef AWP_STR_LAUNCH
 #undef AWP_STR_ARGS

@@ -21,13 +21,34 @@ struct AwpTuning {
   int topo_vel_split;   // 1: the curvilinear velocity update as one launch per component
   int adj_jgroup;       // adjoint kernels' block order: 0 plane by plane, else j tiles per group
   int topo_str_split;   // strain-rate pass: 0 one launch, 1 two (normal, shear), 2 three (normal, xy, xz+yz)
-  int kw;               // k-run width of the Cartesian kernels: 0 by the idle-lane rule, 32, 64
+  int kw;               // k-run width of the Cartesian kernels: 0 by the idle-lane rules, 32, 64
   int topo_nseg;        // curvilinear stress kernel: waves per k chunk at most (1: one-wave segments)
   int topo_wsync;       // curvilinear kernels: 1 wave-scope LDS sync where a wave reads only its own
   int topo_rj;          // curvilinear stress kernel: > 0 forces the j rows per workgroup
 };
 
 AwpTuning& awp_tuning();
+
+// The same for the Cartesian velocity and stress kernels: chunks of 4 to 16
+// planes towards `target` workgroups of 4 waves (10240 = 40 per CU).  Longer
+// chunks re-read fewer planes at their ends but leave the last round of
+// workgroups nearly empty: at 243x187x101 chunks of 4 against 16 planes took
+// the stress update (per-cell texture) 194 against 216 us, at 400x300x200
+// 8 against 32 took 860 against 938 us; at 512x512x256 16 and longer are level
+// (1.99 ms).  A grid too small for one round of 1280 workgroups (5 per CU) at
+// 4 planes takes fewer.
+static inline void awp_split_march(int ni, int nkj, int forced, int target, int* nic,
+                                   int* ichunk) {
+  const long long planes = (long long)ni * nkj;
+  long long c = planes / target;
+  if (c < 4) c = 4;
+  if (c > 16) c = 16;
+  if (c > planes / 1280) c = planes / 1280;
+  if (forced > 0) c = forced;
+  if (c < 1) c = 1;
+  *ichunk = (int)c;
+  *nic = (ni + (int)c - 1) / (int)c;
+}
 
 // Number of i-chunks and chunk length for a march over ni planes when the
 // (k, j) tiling gives nkj workgroups per chunk.

@@ -11,6 +11,7 @@
 // -ffp-contract=off), so results are reproducible bit for bit on any
 // IEEE-754 binary32 implementation of the same operations.
 #include "awp_common.h"
+#include "awp_math.h"
 #include "awp_store.h"
 #include "awp_tuning.h"
 #include "../../include/awp_hip.h"
@@ -20,6 +21,7 @@ namespace {
 struct VelLaunch {
   int kb, k0, k1, j0, j1, i0;  // kb: k of lane 0 in tile 0; [k0, k1] active
   int nkt, njt, ichunk, ni, nblocks, remap, jfast;
+  AwpTile tile;
   int yline;
   long long slice;
   float c1, c2, dth;
@@ -32,9 +34,9 @@ struct VelLaunch {
 // the 4th-order update skips there) applies dvelc2's 2nd-order update
 // (kernel.cu:2289-2356) from the operands it has loaded anyway, so one
 // launch does dvelcx_H_opt + dvelc2_H.
-// KW: k-run width (awp_pick_kw); with KW = 32 a wave covers two j rows, and
-// the second row's offset rides in the per-lane byte offsets.
-template <int BJ, bool OOP, class ST, bool DM2 = false, int KW = 64>
+// The tile's first row (awp_pick_tile) is wave-uniform; a lane's row within
+// the tile rides in its byte offsets.
+template <int BJ, bool OOP, class ST, bool DM2 = false>
 __global__ __launch_bounds__(64 * BJ) void dvelcx_kernel(
     typename ST::T* __restrict__ u1, typename ST::T* __restrict__ v1,
     typename ST::T* __restrict__ w1, const typename ST::T* __restrict__ u0,
@@ -48,14 +50,12 @@ __global__ __launch_bounds__(64 * BJ) void dvelcx_kernel(
   const int b = L.remap ? awp_xcd_remap(blockIdx.x, L.nblocks) : (int)blockIdx.x;
   int kt, jt, ic;
   awp_tile3(b, L.nkt, L.njt, L.jfast, kt, jt, ic);
-  // one wave per j row (KW = 64) or per two rows (KW = 32): the wave's first
-  // row jw is wave-uniform, k is the lane (mod KW)
-  constexpr int RW = 64 / KW;
-  const int lane = (int)threadIdx.x;
-  const int lr = KW == 64 ? 0 : lane / KW;  // row of this lane in the wave
-  const int jw = L.j0 + (jt * BJ + __builtin_amdgcn_readfirstlane((int)threadIdx.y)) * RW;
+  const int t = (int)threadIdx.x;
+  const int lr = t * L.tile.mul >> 20;  // row of this lane in the tile
+  const int jw = L.j0 + jt * L.tile.rows;
   const int j = jw + lr;
-  const int k = L.kb + kt * KW + (KW == 64 ? lane : lane % KW);
+  const int k = L.kb + kt * L.tile.width + (t - lr * L.tile.width);
+  if (lr >= L.tile.rows) return;
   if (j > L.j1) return;
   const bool dm2 = DM2 && k == AWP_ALIGN + 2;
   if ((k < L.k0 && !dm2) || k > L.k1) return;
@@ -128,9 +128,9 @@ __global__ __launch_bounds__(64 * BJ) void dvelcx_kernel(
     float f_d1 = 0.25f * (dc + djm + dkm + djk);
     float f_d2 = 0.25f * (dc + ec + dkm + ekm);
     float f_d3 = 0.25f * (dc + ec + djm + ejm);
-    f_d1 = dth / f_d1;
-    f_d2 = dth / f_d2;
-    f_d3 = dth / f_d3;
+    f_d1 = awp_div(dth, f_d1);
+    f_d2 = awp_div(dth, f_d2);
+    f_d3 = awp_div(dth, f_d3);
 
     float un = (u + f_d1 * (c1 * (xx_0 - xx_m1) + c2 * (xx_p1 - xx_m2) + c1 * (xy_0 - xy_jm1) +
                             c2 * (xy_jp1 - xy_jm2) + c1 * (xz_0 - xz_km1) +
@@ -168,28 +168,27 @@ __global__ __launch_bounds__(64 * BJ) void dvelcx_kernel(
 #undef RP
 }
 
-template <int BJ, class ST, bool DM2 = false, int KW = 64>
+template <int BJ, class ST, bool DM2 = false>
 void launch_vel(void* const* f9, void* const* v0, float* dcrjx, float* dcrjy, float* dcrjz,
                 float* d_1, hipStream_t St, VelLaunch L, const WaveScales& SC) {
   typedef typename ST::T T;
   const int nkj = L.nkt * L.njt;
   int nic, ichunk;
-  awp_split_i(L.ni, nkj, awp_tuning().vel_ichunk, awp_tuning().vel_target_wgs, &nic, &ichunk);
+  awp_split_march(L.ni, nkj, awp_tuning().vel_ichunk, awp_tuning().vel_target_wgs, &nic, &ichunk);
   L.ichunk = ichunk;
   L.nblocks = nkj * nic;
   if (DM2)
-    hipLaunchKernelGGL((dvelcx_kernel<BJ, false, ST, true, KW>), dim3(L.nblocks), dim3(64, BJ), 0,
-                       St, (T*)f9[0], (T*)f9[1], (T*)f9[2], nullptr, nullptr, nullptr,
+    hipLaunchKernelGGL((dvelcx_kernel<BJ, false, ST, true>), dim3(L.nblocks), dim3(64 * BJ), 0, St, (T*)f9[0], (T*)f9[1], (T*)f9[2], nullptr, nullptr, nullptr,
                        (const T*)f9[3], (const T*)f9[4], (const T*)f9[5], (const T*)f9[6],
                        (const T*)f9[7], (const T*)f9[8], dcrjx, dcrjy, dcrjz, d_1, L, SC);
   else if (v0)
-    hipLaunchKernelGGL((dvelcx_kernel<BJ, true, ST, false, KW>), dim3(L.nblocks), dim3(64, BJ), 0, St,
+    hipLaunchKernelGGL((dvelcx_kernel<BJ, true, ST, false>), dim3(L.nblocks), dim3(64 * BJ), 0, St,
                        (T*)f9[0], (T*)f9[1], (T*)f9[2], (const T*)v0[0], (const T*)v0[1],
                        (const T*)v0[2], (const T*)f9[3], (const T*)f9[4], (const T*)f9[5],
                        (const T*)f9[6], (const T*)f9[7], (const T*)f9[8], dcrjx, dcrjy, dcrjz,
                        d_1, L, SC);
   else
-    hipLaunchKernelGGL((dvelcx_kernel<BJ, false, ST, false, KW>), dim3(L.nblocks), dim3(64, BJ), 0, St,
+    hipLaunchKernelGGL((dvelcx_kernel<BJ, false, ST, false>), dim3(L.nblocks), dim3(64 * BJ), 0, St,
                        (T*)f9[0], (T*)f9[1], (T*)f9[2], nullptr, nullptr, nullptr,
                        (const T*)f9[3], (const T*)f9[4], (const T*)f9[5], (const T*)f9[6],
                        (const T*)f9[7], (const T*)f9[8], dcrjx, dcrjy, dcrjz, d_1, L, SC);
@@ -233,28 +232,17 @@ void dvelcx_common(const char* W, void* const* f9, void* const* v0, float* dcrjx
   L.jfast = awp_tuning().vel_jfast;
   L.kb = awp_tuning().kalign ? (L.k0 & ~31) : L.k0;
   const int bj = awp_tuning().vel_bj;
-  const int kw = awp_pick_kw(L.k1 - L.kb + 1, awp_tuning().kw);
-  L.nkt = awp_cdiv(L.k1 - L.kb + 1, kw);
-  L.njt = awp_cdiv(L.j1 - L.j0 + 1, bj * (64 / kw));
+  L.tile = awp_pick_tile(L.k1 - L.kb + 1, 64 * bj, g.yline, awp_tuning().kw);
+  L.nkt = L.tile.nkt;
+  L.njt = awp_cdiv(L.j1 - L.j0 + 1, L.tile.rows);
   if (L.k1 < L.k0) return;
-#define AWP_VEL_LAUNCH(B, KW) \
-  launch_vel<B, ST, DM2, KW>(f9, v0, dcrjx, dcrjy, dcrjz, d_1, St, L, SC)
-  if (kw == 32) {
-    switch (bj) {
-      case 1: AWP_VEL_LAUNCH(1, 32); break;
-      case 2: AWP_VEL_LAUNCH(2, 32); break;
-      case 8: AWP_VEL_LAUNCH(8, 32); break;
-      case 16: AWP_VEL_LAUNCH(16, 32); break;
-      default: AWP_VEL_LAUNCH(4, 32); break;
-    }
-  } else {
-    switch (bj) {
-      case 1: AWP_VEL_LAUNCH(1, 64); break;
-      case 2: AWP_VEL_LAUNCH(2, 64); break;
-      case 8: AWP_VEL_LAUNCH(8, 64); break;
-      case 16: AWP_VEL_LAUNCH(16, 64); break;
-      default: AWP_VEL_LAUNCH(4, 64); break;
-    }
+#define AWP_VEL_LAUNCH(B) launch_vel<B, ST, DM2>(f9, v0, dcrjx, dcrjy, dcrjz, d_1, St, L, SC)
+  switch (bj) {
+    case 1: AWP_VEL_LAUNCH(1); break;
+    case 2: AWP_VEL_LAUNCH(2); break;
+    case 8: AWP_VEL_LAUNCH(8); break;
+    case 16: AWP_VEL_LAUNCH(16); break;
+    default: AWP_VEL_LAUNCH(4); break;
   }
 #undef AWP_VEL_LAUNCH
   awp_check_launch(W);
