@@ -74,51 +74,33 @@ static inline int awp_pick_kw(int n, int forced) {
   return idle64 - idle32 >= 16 ? 32 : 64;
 }
 
-// (k, j) tile of the marching Cartesian kernels: a workgroup of `lanes` lanes
+// (k, j) tile of the marching Cartesian kernels: a workgroup of `waves` waves
 // covers `rows` j rows of `width` consecutive k each, lane t being row
 // t / width and level t % width, `nkt` tiles down a column of n levels.
-// The width is the one that leaves the fewest lanes idle: a column that is
-// not a multiple of 64 is cut into equal runs and the lanes they free take
-// further rows (n = 101: 2 runs of 51 levels of 5 rows, 505 of 512 lanes,
-// against 404 with 64-level runs of 4 rows).  Runs stay at 32 levels (one
-// 128-byte line) or more; equal counts go to the width nearest 64, so
-// columns of 64 m levels keep whole-line waves of one row each.  Where rows
-// are whole lines (yline a multiple of 32 floats) only widths that are too
-// are taken, unless they cost 12 % more lanes: a run's edge line is then
-// fetched by two tiles.
+//   n <= 64, n a multiple of 64, n > 256: rows of 64 levels, one per wave
+//     (4 waves), so a wave's accesses are whole 128-byte lines;
+//   else: one row of all n levels, ceil(n / 64) waves.  Cut into runs, such a
+//     column has seams inside it, and where nzt + 64 is no multiple of 32
+//     every row starts inside a line: the lines at a seam are fetched by two
+//     workgroups and written in two parts.  At 400x300x200 runs of 50 levels
+//     fetched 2.51 GB and wrote 1.31 GB per stress update for 1.82 and 1.15
+//     algorithmic; one row per workgroup took it from 899 to 829 us and the
+//     velocity update from 393 to 340, idle lanes included (300x300xn: within
+//     2 % of the best of 30 shapes for n = 101 .. 230).
+// waves, width: forced by the tuning unless 0.
 struct AwpTile {
-  int width, rows, nkt, mul;  // mul: t / width = t * mul >> 20 for t < 1024
+  int width, rows, waves, nkt, mul;  // mul: t / width = t * mul >> 20 for t < 1024
 };
-static inline AwpTile awp_pick_tile(int n, int lanes, int yline, int forced) {
-  AwpTile best = {64, lanes / 64, awp_cdiv(n, 64), 0};
-  if (forced == 32 || forced == 64) {
-    best.width = forced;
-    best.rows = lanes / forced;
-    best.nkt = awp_cdiv(n, forced);
-  } else {
-    float cost = 1e30f;
-    const int most = lanes < 256 ? lanes : 256;
-    for (int nkt = awp_cdiv(n, most); nkt <= awp_cdiv(n, 32); ++nkt)
-      for (int al = 0; al < 2; ++al) {
-        int w = awp_cdiv(n, nkt);
-        if (al) w = awp_cdiv(w, 32) * 32;
-        if (w < 32) w = 32;
-        if (w > most) continue;
-        const int rows = lanes / w, nt = awp_cdiv(n, w);
-        float c = (float)(nt * lanes) / (float)(n * rows);
-        if (yline % 32 == 0 && w % 32 != 0) c *= 1.12f;
-        const int d = w < 64 ? 64 - w : w - 64, db = best.width < 64 ? 64 - best.width
-                                                                     : best.width - 64;
-        if (c < cost * 0.999f || (c < cost * 1.001f && d < db)) {
-          cost = c;
-          best.width = w;
-          best.rows = rows;
-          best.nkt = nt;
-        }
-      }
-  }
-  best.mul = ((1 << 20) + best.width - 1) / best.width;
-  return best;
+static inline AwpTile awp_pick_tile(int n, int waves, int width) {
+  AwpTile t;
+  const bool row = n > 64 && n <= 256 && n % 64 != 0;
+  t.waves = waves > 0 ? waves : row && width <= 0 ? awp_cdiv(n, 64) : 4;
+  t.width = width > 0 ? width : row ? n : 64;
+  if (t.width > 64 * t.waves) t.width = 64;
+  t.rows = 64 * t.waves / t.width;
+  t.nkt = awp_cdiv(n, t.width);
+  t.mul = ((1 << 20) + t.width - 1) / t.width;
+  return t;
 }
 
 // The reference's (float)(c / (double)x) for binary32 c and x.  Rounding the

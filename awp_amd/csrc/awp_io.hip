@@ -17,7 +17,7 @@
 // three launches), the velocity waves ordering their LDS at wave scope
 // (1.002 -> 0.971 ms); the adjoint kernels' blocks in groups of 8 j tiles over
 // all planes (adj_stress_local 551 -> 533 us at 256x256x128).
-static AwpTuning g_tuning = {4, 4, 10240, 10240, 0, 0, 1, 1, 8, 16, 1, 32, 2048, 0, 0, 0, 1, 8, 2, 0, 8, 1, 0};
+static AwpTuning g_tuning = {0, 0, 10240, 10240, 0, 0, 1, 1, 8, 16, 1, 32, 2048, 0, 0, 0, 1, 8, 2, 0, 8, 1, 0};
 AwpTuning& awp_tuning() { return g_tuning; }
 
 namespace {
@@ -184,7 +184,8 @@ extern "C" {
 int awp_set_tuning(const char* key, int value) {
   AwpTuning& t = g_tuning;
   if (!strcmp(key, "vel_bj") || !strcmp(key, "str_bj")) {
-    if (value != 1 && value != 2 && value != 4 && value != 8 && value != 16) return -1;
+    if (value != 0 && value != 1 && value != 2 && value != 4 && value != 8 && value != 16)
+      return -1;
     (!strcmp(key, "vel_bj") ? t.vel_bj : t.str_bj) = value;
   } else if (!strcmp(key, "vel_target_wgs") || !strcmp(key, "str_target_wgs")) {
     if (value < 1) return -1;

@@ -2,9 +2,8 @@
 // src/awp/kernel.cu:880-1197, and dstrqc_new :343-859), free-surface
 // velocity ghosts (:1087-1112) and stress imaging fstr (:1616-1647), gfx950.
 //
-// Mapping as in the velocity kernel: wave64 along k, BJ waves along j, an
-// i-march with register pipelines.  All four 8-cell material means
-// (lam, mu, qp, qs) keep their plane-(i+1) corners in registers, so every
+// Mapping as in the velocity kernel: lanes along k, an i-march with register
+// pipelines.  All four 8-cell material means (lam, mu, qp, qs) keep their plane-(i+1) corners in registers, so every
 // per-cell array is fetched once per march; u/v/w keep a 4-plane x window.
 // The 16 Q coefficients sit in LDS and are indexed per lane by ww.
 //
@@ -74,8 +73,8 @@ struct TexTable {
   int xls, yls, nj, nzt;         // TEX_RULE only
 };
 
-template <int BJ, bool NEWLIT, bool OOP, class ST, int TEX = TEX_ARRAYS>
-__global__ __launch_bounds__(64 * BJ) void dstrqc_kernel(
+template <int MAXW, bool NEWLIT, bool OOP, class ST, int TEX = TEX_ARRAYS>
+__global__ __launch_bounds__(64 * MAXW) void dstrqc_kernel(
     typename ST::T* __restrict__ xx, typename ST::T* __restrict__ yy,
     typename ST::T* __restrict__ zz, typename ST::T* __restrict__ xy,
     typename ST::T* __restrict__ xz, typename ST::T* __restrict__ yz, const CStress6 S0,
@@ -411,27 +410,24 @@ void dstrqc_common(const char* W, void* const* f15, const CStress6& S0, float* l
   L.jfast = awp_tuning().str_jfast;
   if (L.k1 < L.k0) return;
   const int bj = awp_tuning().str_bj;
-  L.tile = awp_pick_tile(L.k1 - L.kb + 1, 64 * bj, g.yline, awp_tuning().kw);
+  L.tile = awp_pick_tile(L.k1 - L.kb + 1, bj, awp_tuning().kw);
   L.nkt = L.tile.nkt;
   L.njt = awp_cdiv(L.j1 - L.j0 + 1, L.tile.rows);
   int nic, ichunk;
-  awp_split_march(L.ni, L.nkt * L.njt, awp_tuning().str_ichunk, awp_tuning().str_target_wgs, &nic,
-                  &ichunk);
+  awp_split_march(L.ni, L.nkt * L.njt, L.tile.waves, awp_tuning().str_ichunk,
+                  awp_tuning().str_target_wgs, &nic, &ichunk);
   L.ichunk = ichunk;
   L.nblocks = L.nkt * L.njt * nic;
 #define AWP_STR_ARGS                                                                          \
   A[0], A[1], A[2], A[3], A[4], A[5], S0, A[6], A[7], A[8], A[9], A[10], A[11], A[12], A[13], \
       A[14], lam, mu, qp, coeff, qs, dcrjx, dcrjy, dcrjz, vx1, vx2, ww, wwo, L, SC, TT
 #define AWP_STR_LAUNCH(B)                                                                    \
-  hipLaunchKernelGGL((dstrqc_kernel<B, NEWLIT, OOP, ST, TEX>), dim3(L.nblocks), dim3(64 * B), \
+  hipLaunchKernelGGL((dstrqc_kernel<B, NEWLIT, OOP, ST, TEX>), dim3(L.nblocks), dim3(64 * L.tile.waves), \
                      0, St, AWP_STR_ARGS)
-  switch (bj) {
-    case 1: AWP_STR_LAUNCH(1); break;
-    case 2: AWP_STR_LAUNCH(2); break;
-    case 8: AWP_STR_LAUNCH(8); break;
-    case 16: AWP_STR_LAUNCH(16); break;
-    default: AWP_STR_LAUNCH(4); break;
-  }
+  if (L.tile.waves > 8)
+    AWP_STR_LAUNCH(16);
+  else
+    AWP_STR_LAUNCH(8);
 #undef AWP_STR_LAUNCH
 #undef AWP_STR_ARGS
   awp_check_launch(W);

@@ -2,8 +2,8 @@
 #pragma once
 
 struct AwpTuning {
-  int vel_bj;       // j rows per velocity workgroup (64 k-lanes each)
-  int str_bj;       // j rows per stress workgroup
+  int vel_bj;       // waves per velocity workgroup (0: awp_pick_tile)
+  int str_bj;       // waves per stress workgroup (0: awp_pick_tile)
   int vel_target_wgs;  // velocity: workgroups to aim for when splitting the i march
   int str_target_wgs;  // stress: same
   int vel_ichunk;   // >0 forces the velocity i-chunk length
@@ -37,9 +37,9 @@ AwpTuning& awp_tuning();
 // 8 against 32 took 860 against 938 us; at 512x512x256 16 and longer are level
 // (1.99 ms).  A grid too small for one round of 1280 workgroups (5 per CU) at
 // 4 planes takes fewer.
-static inline void awp_split_march(int ni, int nkj, int forced, int target, int* nic,
+static inline void awp_split_march(int ni, int nkj, int waves, int forced, int target, int* nic,
                                    int* ichunk) {
-  const long long planes = (long long)ni * nkj;
+  const long long planes = (long long)ni * nkj * waves / 4;
   long long c = planes / target;
   if (c < 4) c = 4;
   if (c > 16) c = 16;

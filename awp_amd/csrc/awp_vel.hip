@@ -1,10 +1,9 @@
 // Velocity update (reference dvelcx_opt, src/awp/kernel.cu:125-268), gfx950.
 //
-// Mapping: one wave64 covers 64 consecutive k (the contiguous axis, 256 B per
-// field load), a workgroup stacks BJ waves along j, and each lane marches
-// along i over one i-chunk with register pipelines for every x-stencil and
-// for the 4-point density means, so each field plane is fetched from HBM
-// once per march.  j/k neighbours come from L1/L2; the XCD-aware tile order
+// Mapping: lanes run along k (the contiguous axis), a workgroup covers a few j
+// rows or one whole row (awp_pick_tile), and each lane marches along i over
+// one i-chunk with register pipelines for every x-stencil and for the 4-point
+// density means, so each field plane is fetched from HBM once per march.  j/k neighbours come from L1/L2; the XCD-aware tile order
 // keeps neighbouring tiles (which share those lines) on one L2.
 //
 // Arithmetic follows the reference expression trees (built with
@@ -36,8 +35,8 @@ struct VelLaunch {
 // launch does dvelcx_H_opt + dvelc2_H.
 // The tile's first row (awp_pick_tile) is wave-uniform; a lane's row within
 // the tile rides in its byte offsets.
-template <int BJ, bool OOP, class ST, bool DM2 = false>
-__global__ __launch_bounds__(64 * BJ) void dvelcx_kernel(
+template <int MAXW, bool OOP, class ST, bool DM2 = false>
+__global__ __launch_bounds__(64 * MAXW) void dvelcx_kernel(
     typename ST::T* __restrict__ u1, typename ST::T* __restrict__ v1,
     typename ST::T* __restrict__ w1, const typename ST::T* __restrict__ u0,
     const typename ST::T* __restrict__ v0, const typename ST::T* __restrict__ w0,
@@ -168,30 +167,31 @@ __global__ __launch_bounds__(64 * BJ) void dvelcx_kernel(
 #undef RP
 }
 
-template <int BJ, class ST, bool DM2 = false>
+template <int MAXW, class ST, bool DM2 = false>
 void launch_vel(void* const* f9, void* const* v0, float* dcrjx, float* dcrjy, float* dcrjz,
                 float* d_1, hipStream_t St, VelLaunch L, const WaveScales& SC) {
   typedef typename ST::T T;
   const int nkj = L.nkt * L.njt;
   int nic, ichunk;
-  awp_split_march(L.ni, nkj, awp_tuning().vel_ichunk, awp_tuning().vel_target_wgs, &nic, &ichunk);
+  awp_split_march(L.ni, nkj, L.tile.waves, awp_tuning().vel_ichunk, awp_tuning().vel_target_wgs,
+                  &nic, &ichunk);
   L.ichunk = ichunk;
   L.nblocks = nkj * nic;
+  const dim3 grid(L.nblocks), block(64 * L.tile.waves);
+#define AWP_VEL_ARGS                                                                             \
+  (const T*)f9[3], (const T*)f9[4], (const T*)f9[5], (const T*)f9[6], (const T*)f9[7],           \
+      (const T*)f9[8], dcrjx, dcrjy, dcrjz, d_1, L, SC
   if (DM2)
-    hipLaunchKernelGGL((dvelcx_kernel<BJ, false, ST, true>), dim3(L.nblocks), dim3(64 * BJ), 0, St, (T*)f9[0], (T*)f9[1], (T*)f9[2], nullptr, nullptr, nullptr,
-                       (const T*)f9[3], (const T*)f9[4], (const T*)f9[5], (const T*)f9[6],
-                       (const T*)f9[7], (const T*)f9[8], dcrjx, dcrjy, dcrjz, d_1, L, SC);
+    hipLaunchKernelGGL((dvelcx_kernel<MAXW, false, ST, true>), grid, block, 0, St, (T*)f9[0],
+                       (T*)f9[1], (T*)f9[2], nullptr, nullptr, nullptr, AWP_VEL_ARGS);
   else if (v0)
-    hipLaunchKernelGGL((dvelcx_kernel<BJ, true, ST, false>), dim3(L.nblocks), dim3(64 * BJ), 0, St,
-                       (T*)f9[0], (T*)f9[1], (T*)f9[2], (const T*)v0[0], (const T*)v0[1],
-                       (const T*)v0[2], (const T*)f9[3], (const T*)f9[4], (const T*)f9[5],
-                       (const T*)f9[6], (const T*)f9[7], (const T*)f9[8], dcrjx, dcrjy, dcrjz,
-                       d_1, L, SC);
+    hipLaunchKernelGGL((dvelcx_kernel<MAXW, true, ST, false>), grid, block, 0, St, (T*)f9[0],
+                       (T*)f9[1], (T*)f9[2], (const T*)v0[0], (const T*)v0[1], (const T*)v0[2],
+                       AWP_VEL_ARGS);
   else
-    hipLaunchKernelGGL((dvelcx_kernel<BJ, false, ST, false>), dim3(L.nblocks), dim3(64 * BJ), 0, St,
-                       (T*)f9[0], (T*)f9[1], (T*)f9[2], nullptr, nullptr, nullptr,
-                       (const T*)f9[3], (const T*)f9[4], (const T*)f9[5], (const T*)f9[6],
-                       (const T*)f9[7], (const T*)f9[8], dcrjx, dcrjy, dcrjz, d_1, L, SC);
+    hipLaunchKernelGGL((dvelcx_kernel<MAXW, false, ST, false>), grid, block, 0, St, (T*)f9[0],
+                       (T*)f9[1], (T*)f9[2], nullptr, nullptr, nullptr, AWP_VEL_ARGS);
+#undef AWP_VEL_ARGS
 }
 
 // f9: u1 v1 w1 xx yy zz xy xz yz in the storage type of ST; v0: null (u1 v1
@@ -232,18 +232,15 @@ void dvelcx_common(const char* W, void* const* f9, void* const* v0, float* dcrjx
   L.jfast = awp_tuning().vel_jfast;
   L.kb = awp_tuning().kalign ? (L.k0 & ~31) : L.k0;
   const int bj = awp_tuning().vel_bj;
-  L.tile = awp_pick_tile(L.k1 - L.kb + 1, 64 * bj, g.yline, awp_tuning().kw);
+  L.tile = awp_pick_tile(L.k1 - L.kb + 1, bj, awp_tuning().kw);
   L.nkt = L.tile.nkt;
   L.njt = awp_cdiv(L.j1 - L.j0 + 1, L.tile.rows);
   if (L.k1 < L.k0) return;
 #define AWP_VEL_LAUNCH(B) launch_vel<B, ST, DM2>(f9, v0, dcrjx, dcrjy, dcrjz, d_1, St, L, SC)
-  switch (bj) {
-    case 1: AWP_VEL_LAUNCH(1); break;
-    case 2: AWP_VEL_LAUNCH(2); break;
-    case 8: AWP_VEL_LAUNCH(8); break;
-    case 16: AWP_VEL_LAUNCH(16); break;
-    default: AWP_VEL_LAUNCH(4); break;
-  }
+  if (L.tile.waves > 8)
+    AWP_VEL_LAUNCH(16);
+  else
+    AWP_VEL_LAUNCH(8);
 #undef AWP_VEL_LAUNCH
   awp_check_launch(W);
 }

@@ -38,9 +38,9 @@ const char* awp_last_error_string(void);
 void awp_clear_error(void);
 
 /* Launch-shape knobs (no reference counterpart), process-global; results do
- * not depend on them.  Keys: vel_bj, str_bj (rows per workgroup: 1, 2, 4, 8,
- * 16), vel_target_wgs, str_target_wgs, vel_ichunk, str_ichunk (i-march
- * chunking, 0 = automatic), xcd_remap, kalign (0/1), topo_vel_ichunk,
+ * not depend on them.  Keys: vel_bj, str_bj (waves per workgroup: 1, 2, 4, 8,
+ * 16; 0 = automatic), vel_target_wgs, str_target_wgs, vel_ichunk, str_ichunk
+ * (i-march chunking, 0 = automatic), xcd_remap, kalign (0/1), topo_vel_ichunk,
  * topo_str_ichunk, topo_q_ichunk (planes per march, 1..4096), step_ichunk
  * (0 = automatic), step_target_wgs (awp_step's i-march chunking).  Returns 0,
  * or -1 for an unknown key or a value out of range. */

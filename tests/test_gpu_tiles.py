@@ -1,0 +1,63 @@
+"""The (k, j) tiles of the marching Cartesian kernels (awp_pick_tile) at the
+column heights where the rule changes: one wave and less, 64 m levels, one row
+per workgroup of 2, 3 and 4 waves, and 64-level runs beyond 256.  Velocity,
+stress bit for bit against the oracle: the arithmetic
+is the same expression by expression, so the tolerance is zero."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from awp_amd.grid import Dims
+from tests._fields import WAVE, first_mismatch, random_state
+
+pytestmark = pytest.mark.gpu
+
+DH, DT = 50.0, 0.0025
+VEL = ("u1", "v1", "w1", "xx", "yy", "zz", "xy", "xz", "yz")
+STR = ("xx", "yy", "zz", "xy", "xz", "yz", "r1", "r2", "r3", "r4", "r5", "r6", "u1", "v1", "w1")
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from awp_amd import _lib
+    lib = _lib.load()
+    for key in ("vel_bj", "str_bj", "vel_ichunk", "str_ichunk", "kw"):
+        _lib.set_tuning(key, 0)
+    return torch, lib, _lib
+
+
+@pytest.mark.parametrize("nz", [36, 61, 64, 65, 101, 128, 130, 191, 193, 255, 256, 257, 300])
+def test_column_heights_bit_exact(gpu, oracle_lib, nz):
+    torch, lib, _lib = gpu
+    d = Dims(11, 9, nz)
+    st, med = random_state(d, seed=3 + nz)
+    F, I = C.c_float, C.c_int
+    z9 = (F * 9)()
+    lib.SetDeviceConstValue((F * 1)(DH), F(DT), (I * 1)(d.nxt), (I * 1)(d.nyt), (I * 1)(d.nzt),
+                            1, 0.0, 0.0, z9, z9)
+    dev = {k: torch.from_numpy(np.ascontiguousarray(v)).cuda() for k, v in {**st, **med}.items()}
+    host = {k: v.copy() for k, v in st.items()}
+    p = lambda n: dev[n].data_ptr()  # noqa: E731
+    q = lambda n: (host[n] if n in host else med[n]).ctypes.data  # noqa: E731
+    s = torch.cuda.current_stream().cuda_stream
+    (s_i, e_i), (s_j, e_j) = d.i_range, d.j_range
+    sp = ("dcrjx", "dcrjy", "dcrjz")
+    lib.dvelcx_H_opt(*map(p, VEL + sp), p("d1"), d.nyt, d.nzt, s, s_i, e_i, 0, 1)
+    lib.dstrqc_H(*map(p, STR), *map(p, ("lam", "mu", "qp", "coeff", "qs") + sp), d.nyt, d.nzt, s,
+                 *map(p, ("lam_mu", "vx1", "vx2", "ww", "wwo")), d.nxt, 0, 0, 0, s_i, e_i, s_j,
+                 e_j, 0)
+    _lib.check()
+    o = oracle_lib.load()
+    o.awp_oracle_dvelcx_f32(*map(q, VEL + sp), q("d1"), d.nxt, d.nyt, d.nzt, DH, DT, s_i, e_i, 0,
+                            1)
+    o.awp_oracle_dstrqc_f32(*map(q, STR), *map(q, ("lam", "mu", "qp", "coeff", "qs") + sp),
+                            *map(q, ("lam_mu", "vx1", "vx2", "ww", "wwo")), d.nxt, d.nyt, d.nzt,
+                            DH, DT, d.nxt, 0, 0, 0, s_i, e_i, s_j, e_j, 0)
+    torch.cuda.synchronize()
+    for n in WAVE:
+        mm = first_mismatch(dev[n].cpu().numpy(), host[n])
+        assert mm is None, f"nz={nz}: {n} differs: {mm}"
