@@ -217,6 +217,9 @@ int awp_set_tuning(const char* key, int value) {
   } else if (!strcmp(key, "topo_str_split")) {
     if (value < 0 || value > 2) return -1;
     t.topo_str_split = value;
+  } else if (!strcmp(key, "topo_rate_chunk")) {
+    if (value < 0 || value > 4096) return -1;
+    t.topo_rate_chunk = value;
   } else if (!strcmp(key, "topo_rj")) {
     if (value < 0 || value > 8) return -1;
     t.topo_rj = value;

@@ -20,6 +20,7 @@
 // (double where it writes double literals), so results match the CPU
 // oracle bit for bit.
 #include "awp_common.h"
+#include "awp_math.h"
 #include "awp_store.h"
 #include "awp_topo_coef.h"
 #include "awp_tuning.h"
@@ -551,50 +552,18 @@ enum {
   C_VN, C_VO, C_VM2, C_VM1, C_VP1,   // v1 at (i+1, j), (i, j), (i, j-2), (i, j-1), (i, j+1)
   C_WN, C_WO, C_WM1, C_WP1, C_WP2    // w1 at (i+1, j), (i, j), (i, j-1), (i, j+1), (i, j+2)
 };
-// Rate groups of the two-pass update: 0 all six rates (and the one-pass
-// update), 1 the normal rates vs1, vs2, vs3, 2 the shear sums xy, xz, yz,
-// 3 the xy sum, 4 the xz and yz sums.  A group stages only the columns its
-// z sums read, in LDS slots 0.. .
-constexpr unsigned ST_COLS_XY =
-    (1u << C_UO) | (1u << C_UM1) | (1u << C_UP1) | (1u << C_UP2) | (1u << C_VN);
-constexpr unsigned ST_COLS_XZYZ = (1u << C_UO) | (1u << C_VO) | (1u << C_WN) | (1u << C_WM1) |
-                                  (1u << C_WP1) | (1u << C_WP2);
-constexpr unsigned st_group_cols(int group) {
-  return group == 1   ? (1u << C_UN) | (1u << C_VO) | (1u << C_VM2) | (1u << C_VM1) |
-                            (1u << C_VP1) | (1u << C_WO)
-         : group == 2 ? ST_COLS_XY | ST_COLS_XZYZ
-         : group == 3 ? ST_COLS_XY
-         : group == 4 ? ST_COLS_XZYZ
-                      : (1u << ST_NC) - 1u;
-}
-constexpr int st_group_ncols(int group) { return __builtin_popcount(st_group_cols(group)); }
-// LDS slot of column c in a group (the number of staged columns before it)
-constexpr int st_slot(int group, int c) {
-  return __builtin_popcount(st_group_cols(group) & ((1u << c) - 1u));
-}
-constexpr bool st_staged(int group, int c) { return (st_group_cols(group) >> c) & 1u; }
-
 // RATES: store the six strain-rate terms of every output cell into R
 // (TOPO_NRATES arrays of the field's size, rstride floats apart) for
 // topo_str_q_kernel, instead of applying the material and memory-variable
 // update here.
-// GROUP (RATES only): the rate group this launch computes and stores
-// (st_group_cols); launches of groups 1 and 2, or 1, 3 and 4, store what one
-// of group 0 does, each with fewer live registers and LDS slots.
-template <class ST, bool RATES, int GROUP = 0>
+template <class ST, bool RATES>
 __global__ __launch_bounds__(64 * VT_MAXW) void topo_str_kernel(const TopoStrArgs<ST> A,
                                                               const TGeom G, const VelTiles V,
                                                               float* __restrict__ R,
                                                               long long rstride) {
-  static_assert(GROUP == 0 || RATES, "rate groups apply to the two-pass update");
-  // normal rates, the xy sum, the xz and yz sums
-  constexpr bool GN = GROUP <= 1, GXY = GROUP != 1 && GROUP != 4,
-                 GZ = GROUP != 1 && GROUP != 3;
-  constexpr int NC = st_group_ncols(GROUP);
-#define SC_(c) st_slot(GROUP, c)
-  // [parity][row][slot][level of the chunk]: 2 * rj * NC * ch floats; the
+  // [parity][row][column][level of the chunk]: 2 * rj * ST_NC * ch floats; the
   // column of array c at parity base L
-#define LCOL(c) (L + SC_(c) * V.ch)
+#define LCOL(c) (L + (c) * V.ch)
   extern __shared__ float st_lds[];
   const int lane = (int)threadIdx.x;
   const int w = (int)threadIdx.y;
@@ -664,21 +633,21 @@ __global__ __launch_bounds__(64 * VT_MAXW) void topo_str_kernel(const TopoStrArg
   // prologue: stage the columns the first plane's windows need
   for (int q = 0; q < 3; ++q) {
     const int iu = ib - 1 + q, iv = ib - 2 + q;
-    float* L = st_lds + ((q & 1) * V.rj + row) * NC * V.ch;
+    float* L = st_lds + ((q & 1) * V.rj + row) * ST_NC * V.ch;
     ux[q + 1] = A.u1[colj + sl * iu];
     vx[q + 1] = A.v1[colj + sl * iv];
     wx[q + 1] = A.w1[colj + sl * iv];
-    if constexpr (GN) LCOL(C_UN)[kl] = ux[q + 1];
-    if constexpr (GXY) LCOL(C_VN)[kl] = vx[q + 1];
-    if constexpr (GZ) LCOL(C_WN)[kl] = wx[q + 1];
+    LCOL(C_UN)[kl] = ux[q + 1];
+    LCOL(C_VN)[kl] = vx[q + 1];
+    LCOL(C_WN)[kl] = wx[q + 1];
     // one-wave chunks read only their own LDS rows (see topo_vel_kernel)
     if (V.wsync && V.nseg == 1)
       wave_lds_sync();
     else
       __syncthreads();
-    if constexpr (GN) Zu[q + 1] = zu_x(LCOL(C_UN));
-    if constexpr (GXY) Zv[q + 1] = zv_x(LCOL(C_VN));
-    if constexpr (GZ) Zw[q + 1] = zw(LCOL(C_WN));
+    Zu[q + 1] = zu_x(LCOL(C_UN));
+    Zv[q + 1] = zv_x(LCOL(C_VN));
+    Zw[q + 1] = zw(LCOL(C_WN));
   }
 
   const float g_ck = M.g_c[K], g_k = M.g[K], g3c_k = M.g3_c[K], g3_k = M.g3[K];
@@ -688,7 +657,7 @@ __global__ __launch_bounds__(64 * VT_MAXW) void topo_str_kernel(const TopoStrArg
 
   for (int i = ib; i < ie; ++i) {
     const int par = (i + 1) & 1;  // the prologue used parities 0, 1, 0
-    float* L = st_lds + (par * V.rj + row) * NC * V.ch;
+    float* L = st_lds + (par * V.rj + row) * ST_NC * V.ch;
     const int pos = colj + sl * i;
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
@@ -702,28 +671,11 @@ __global__ __launch_bounds__(64 * VT_MAXW) void topo_str_kernel(const TopoStrArg
     ux[3] = A.u1[pos + 2 * sl];
     vx[3] = A.v1[pos + sl];
     wx[3] = A.w1[pos + sl];
-    float um1 = 0.f, up1 = 0.f, up2 = 0.f, vm2 = 0.f, vm1 = 0.f, vp1 = 0.f, wm1 = 0.f,
-          wp1 = 0.f, wp2 = 0.f;
-    if constexpr (GXY) {
-      um1 = A.u1[pos - yl];
-      up1 = A.u1[pos + yl];
-      up2 = A.u1[pos + 2 * yl];
-    }
-    if constexpr (GZ) {
-      wm1 = A.w1[pos - yl];
-      wp1 = A.w1[pos + yl];
-      wp2 = A.w1[pos + 2 * yl];
-    }
-    if constexpr (GN) {
-      vm2 = A.v1[pos - 2 * yl];
-      vm1 = A.v1[pos - yl];
-      vp1 = A.v1[pos + yl];
-    }
+    const float um1 = A.u1[pos - yl], up1 = A.u1[pos + yl], up2 = A.u1[pos + 2 * yl];
+    const float wm1 = A.w1[pos - yl], wp1 = A.w1[pos + yl], wp2 = A.w1[pos + 2 * yl];
+    const float vm2 = A.v1[pos - 2 * yl], vm1 = A.v1[pos - yl], vp1 = A.v1[pos + yl];
     const float uo = ux[1], vo = vx[2], wo = wx[2];
-    auto stage = [&](int c, float x) {
-      // c is a literal column at every call, so the test folds away
-      if (st_staged(GROUP, c)) L[st_slot(GROUP, c) * V.ch + kl] = x;
-    };
+    auto stage = [&](int c, float x) { LCOL(c)[kl] = x; };
     stage(C_UN, ux[3]);
     stage(C_UO, uo);
     stage(C_UM1, um1);
@@ -743,14 +695,14 @@ __global__ __launch_bounds__(64 * VT_MAXW) void topo_str_kernel(const TopoStrArg
       wave_lds_sync();
     else
       __syncthreads();
-    if constexpr (GN) Zu[3] = zu_x(LCOL(C_UN));
-    if constexpr (GXY) Zv[3] = zv_x(LCOL(C_VN));
-    if constexpr (GZ) Zw[3] = zw(LCOL(C_WN));
+    Zu[3] = zu_x(LCOL(C_UN));
+    Zv[3] = zv_x(LCOL(C_VN));
+    Zw[3] = zw(LCOL(C_WN));
     if (out) {
       const int q = j + AWP_ALIGN + i * fr;
       const float f_dcrj = A.dcrjx[i] * dcy * dcz;
       float vs1 = 0.f, vs2 = 0.f, vs3 = 0.f, xyv = 0.f, xzv = 0.f, yzv = 0.f;
-      if constexpr (GN) {
+      {
         float acc;
         // xx, yy, zz
         float Jii = M.f_c[q] * g3c_k;
@@ -788,7 +740,7 @@ __global__ __launch_bounds__(64 * VT_MAXW) void topo_str_kernel(const TopoStrArg
           vs3 = Jii * zs;
         }
       }
-      if constexpr (GXY) {
+      {
         float acc;
         // xy
         float J12i = M.f[q] * g3c_k6;
@@ -813,7 +765,7 @@ __global__ __launch_bounds__(64 * VT_MAXW) void topo_str_kernel(const TopoStrArg
         // xzv1 + xzv2 and yzv1 + yzv2 (stress_attenuation.cu:306-327)
         xyv = xyv1 + xyv2;
       }
-      if constexpr (GZ) {
+      {
         float acc;
         // xz
         float J13i = M.f_1[q] * g3_k;
@@ -862,24 +814,318 @@ __global__ __launch_bounds__(64 * VT_MAXW) void topo_str_kernel(const TopoStrArg
         yzv = yzv1 + yzv2;
       }
       if (RATES) {
-        if constexpr (GN) {
-          R[pos] = vs1;
-          R[rstride + pos] = vs2;
-          R[2 * rstride + pos] = vs3;
-        }
-        if constexpr (GXY) R[3 * rstride + pos] = xyv;
-        if constexpr (GZ) {
-          R[4 * rstride + pos] = xzv;
-          R[5 * rstride + pos] = yzv;
-        }
+        R[pos] = vs1;
+        R[rstride + pos] = vs2;
+        R[2 * rstride + pos] = vs3;
+        R[3 * rstride + pos] = xyv;
+        R[4 * rstride + pos] = xzv;
+        R[5 * rstride + pos] = yzv;
       } else {
         topo_str_update<ST>(A, pos, sl, yl, f_dcrj, vs1, vs2, vs3, xyv, xzv, yzv, A.vx1[pos],
                             A.vx2[pos], A.wwo[pos], A.ww[pos]);
       }
     }
   }
-#undef SC_
 #undef LCOL
+}
+
+// The strain-rate pass of the two-pass update, in two launches by march
+// direction.  Every shear rate is the sum of an x-group term (a 4-point
+// combination along i of one velocity column's z sums) and a y-group term
+// (along j); each normal rate has one of the two.  Marching along the group's
+// own direction, a column's z sum is formed once, when the column enters the
+// window, and carried through it.
+//   AX = 0, march along i: vs1, vs3, the x part of xy, both parts of xz
+//   AX = 1, march along j: vs2, the y part of xy (added to the stored x
+//                          part), both parts of yz
+// The z differences of the centre column (vs3, xz, yz) are formed from the
+// same staged column and ride one or two planes behind it.  A cell takes 6
+// seven-point and 3 four-point z sums, 6 velocity loads and 6 staged LDS
+// columns in the two launches together; the one-direction form (marching
+// along i for all six rates, in three launches) took 14, 3, 23 and 17, as the
+// y-group terms need the sums of four j neighbours at every plane.
+//
+// Waves that hold one-sided rows take every sum with per-lane coefficients
+// from LDS (c_rate_top), so their lanes do not diverge.
+#define RT_ASC 0   // first term of each sum: phdz4 ascending,
+#define RT_MID 9   // phdz4 from the middle,
+#define RT_W 18    // pdhz4 from the middle,
+#define RT_DZ 27   // dz4,
+#define RT_DHZ 34  // dhz4
+#define RT_N 42
+// [term][class]: class 0..5 is the one-sided row of level nz-1-class in the
+// order of zrow (the level furthest from the top first), class 6 the interior
+// row in its own order, then zeros for the terms a one-sided row has more
+// (they weigh the lane's own level, which an interior row weighs too).
+struct RateTop {
+  float v[RT_N][8];
+};
+constexpr int rt_mid(int t) { return t == 0 ? 3 : t <= 3 ? t - 1 : t; }
+constexpr RateTop rate_top() {
+  RateTop T{};
+  constexpr int dzo[4] = {1, 0, 2, 3}, dho[4] = {2, 0, 1, 3};
+  for (int t = 0; t < 9; ++t)
+    for (int c = 0; c < 6; ++c) {
+      T.v[RT_ASC + t][c] = T.v[RT_MID + t][c] = (float)TS_PHDZ4R[c][8 - t];
+      T.v[RT_W + t][c] = (float)TS_PDHZ4R[c][8 - t];
+      if (t < 7) T.v[RT_DZ + t][c] = (float)TS_DZ4R[c][6 - t];
+      if (t < 8) T.v[RT_DHZ + t][c] = (float)TS_DHZ4R[c][7 - t];
+    }
+  for (int t = 0; t < 7; ++t) {
+    T.v[RT_ASC + t][6] = (float)TS_PHDZ4[t];
+    T.v[RT_MID + t][6] = (float)TS_PHDZ4[rt_mid(t)];
+    T.v[RT_W + t][6] = (float)TS_PDHZ4[rt_mid(t)];
+  }
+  for (int t = 0; t < 4; ++t) {
+    T.v[RT_DZ + t][6] = (float)TOPO_D4[dzo[t]];
+    T.v[RT_DHZ + t][6] = (float)TOPO_D4[dho[t]];
+  }
+  return T;
+}
+__constant__ RateTop c_rate_top = rate_top();
+
+// A float read at a wave-uniform index of an array that no kernel in flight
+// writes: through the constant address space it is a scalar load.
+typedef const __attribute__((address_space(4))) float* uniform_ptr;
+__device__ __forceinline__ float uld(const float* a, int i) { return ((uniform_ptr)a)[i]; }
+
+#define RC_PAD 4  // LDS floats before and after a staged column: the halo lanes of
+                  // a chunk read up to 3 levels outside it and discard the sums
+
+template <class ST, int AX>
+__global__ __launch_bounds__(64 * VT_MAXW) void topo_rates_kernel(const TopoStrArgs<ST> A,
+                                                                  const TGeom G,
+                                                                  const VelTiles V,
+                                                                  float* __restrict__ R,
+                                                                  long long rstride) {
+  extern __shared__ float rt_lds[];  // [parity][row][u, v, w][RC_PAD + ch + RC_PAD]
+  __shared__ float s_top[RT_N * 8];
+  const int lane = (int)threadIdx.x;
+  const int w = (int)threadIdx.y;
+  const int seg = w % V.nseg, row = w / V.nseg;
+  const int t = (int)blockIdx.x;
+  const bool top = t == V.nint;
+  if (top) {  // uniform over the workgroup
+    for (int e = w * 64 + lane; e < RT_N * 8; e += V.nseg * V.rj * 64)
+      s_top[e] = (&c_rate_top.v[0][0])[e];
+    __syncthreads();
+  }
+  const int k0 = top ? V.ktop0 : V.step * t;
+  const int kl = seg * 64 + lane;  // level within the chunk
+  const int k = k0 + kl;
+  const int nz = G.nz;
+  const int w0 = top ? V.wtop0 : V.step * t + 3;
+  const int w1 = top ? nz : (V.step * t + V.ch - 3 < V.wtop0 ? V.step * t + V.ch - 3 : V.wtop0);
+  const bool bnd = k >= nz - 6;
+  // whether this wave holds one-sided rows
+  const bool topw = top && __builtin_amdgcn_readfirstlane(k0 + seg * 64 + 63) >= nz - 6;
+  // fixed line f (j or i), march m (i or j)
+  const int f0 = AX == 0 ? G.bj : G.bi, f1 = AX == 0 ? G.ej : G.ei;
+  const int m1 = AX == 0 ? G.ei : G.ej;
+  const int fw = f0 + (int)blockIdx.y * V.rj + row;
+  const bool fok = fw < f1;
+  const int f = __builtin_amdgcn_readfirstlane(fok ? fw : f1 - 1);
+  const int mb = (AX == 0 ? G.bi : G.bj) + (int)blockIdx.z * V.ichunk;
+  const int me = mb + V.ichunk < m1 ? mb + V.ichunk : m1;
+  if (mb >= me) return;  // uniform over the workgroup
+  const bool out = k >= w0 && k < w1 && fok;
+  const int sm = AX == 0 ? G.sl : G.yl;     // field stride along the march
+  const int fm = AX == 0 ? G.frow : 1;      // metric stride along the march
+  const int K = (k < 0 ? 0 : k) + AWP_ALIGN;  // array level (see topo_vel_kernel)
+  const int base = K + (AX == 0 ? G.yl : G.sl) * f;
+  const int qbase = AWP_ALIGN + (AX == 0 ? 1 : G.frow) * f;
+  const TMetrics& M = A.M;
+  const int cp = V.ch + 2 * RC_PAD;
+  const int own = RC_PAD + kl;  // this lane's level in a staged column
+  const int lb = RC_PAD + nz - 1 - k0;  // level nz-1 (top chunk)
+  const int cls = bnd ? nz - 1 - k : 6;
+
+  constexpr float phdz4[7] = {(float)TS_PHDZ4[0], (float)TS_PHDZ4[1], (float)TS_PHDZ4[2],
+                              (float)TS_PHDZ4[3], (float)TS_PHDZ4[4], (float)TS_PHDZ4[5],
+                              (float)TS_PHDZ4[6]};
+  constexpr float pdhz4[7] = {(float)TS_PDHZ4[0], (float)TS_PDHZ4[1], (float)TS_PDHZ4[2],
+                              (float)TS_PDHZ4[3], (float)TS_PDHZ4[4], (float)TS_PDHZ4[5],
+                              (float)TS_PDHZ4[6]};
+  auto asc = [&](const float* c) {
+    float acc = phdz4[0] * c[own - 3];
+#pragma unroll
+    for (int m = 1; m < 7; ++m) acc = acc + phdz4[m] * c[own + m - 3];
+    return acc;
+  };
+  auto mid = [&](const float(&cf)[7], const float* c) {
+    float acc = cf[3] * c[own];
+#pragma unroll
+    for (int m = 1; m < 7; ++m) acc = acc + cf[rt_mid(m)] * c[own + rt_mid(m) - 3];
+    return acc;
+  };
+  // the n-term sum of table rows r0 .. r0+n-1; off(t): the interior term's level
+  auto tops = [&](int r0, int n, auto off, const float* c) {
+    float acc = 0.f;
+#pragma unroll
+    for (int m = 0; m < n; ++m) {
+      const float x = s_top[(r0 + m) * 8 + cls] * c[bnd ? lb - (n - 1) + m : own + off(m)];
+      acc = m == 0 ? x : acc + x;
+    }
+    return acc;
+  };
+  auto off_asc = [](int m) { return m < 7 ? m - 3 : 0; };
+  auto off_mid = [](int m) { return m < 7 ? rt_mid(m) - 3 : 0; };
+  auto off_dz = [](int m) { return m == 1 ? -1 : m == 2 ? 1 : m == 3 ? 2 : 0; };
+  auto off_dhz = [](int m) { return m == 1 ? -2 : m == 2 ? -1 : m == 3 ? 1 : 0; };
+  struct Sums {
+    float zu, zv, zw, d, dw;  // d: dz of u (AX = 0) or v (AX = 1); dw: dhz of w (AX = 0)
+  };
+  int par = 0;
+  // stage the three columns entering the windows and form their z sums
+  auto enter = [&](float u, float v, float x) {
+    float* cu = rt_lds + (par * V.rj + row) * 3 * cp;
+    float *cv = cu + cp, *cw = cv + cp;
+    par ^= 1;
+    cu[own] = u;
+    cv[own] = v;
+    cw[own] = x;
+    // one-wave chunks read only their own LDS (see topo_vel_kernel)
+    if (V.wsync && V.nseg == 1)
+      wave_lds_sync();
+    else
+      __syncthreads();
+    Sums s;
+    const float* cd = AX == 0 ? cu : cv;
+    s.dw = 0.f;
+    if (!topw) {
+      s.zu = AX == 0 ? asc(cu) : mid(phdz4, cu);
+      s.zv = AX == 0 ? mid(phdz4, cv) : asc(cv);
+      s.zw = mid(pdhz4, cw);
+      s.d = D4F(1) * cd[own] + D4F(0) * cd[own - 1] + D4F(2) * cd[own + 1] + D4F(3) * cd[own + 2];
+      if (AX == 0)
+        s.dw = D4F(2) * cw[own] + D4F(0) * cw[own - 2] + D4F(1) * cw[own - 1] +
+               D4F(3) * cw[own + 1];
+    } else {
+      s.zu = AX == 0 ? tops(RT_ASC, 9, off_asc, cu) : tops(RT_MID, 9, off_mid, cu);
+      s.zv = AX == 0 ? tops(RT_MID, 9, off_mid, cv) : tops(RT_ASC, 9, off_asc, cv);
+      s.zw = tops(RT_W, 9, off_mid, cw);
+      s.d = tops(RT_DZ, 7, off_dz, cd);
+      if (AX == 0) s.dw = tops(RT_DHZ, 8, off_dhz, cw);
+    }
+    return s;
+  };
+
+  // windows: u covers m-1 .. m+2, v m-2 .. m+1, w m-2 .. m+1 (AX = 0) or
+  // m-1 .. m+2 (AX = 1)
+  constexpr int UL = -1, VL = -2, WL = AX == 0 ? -2 : -1;
+  float U[4], Vv[4], W[4], ZU[4], ZV[4], ZW[4], D[3], dwc = 0.f;
+  auto at = [&](int m) { return base + sm * m; };
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    U[q + 1] = A.u1[at(mb + UL + q)];
+    Vv[q + 1] = A.v1[at(mb + VL + q)];
+    W[q + 1] = A.w1[at(mb + WL + q)];
+  }
+  float un = A.u1[at(mb + UL + 3)], vn = A.v1[at(mb + VL + 3)], wn = A.w1[at(mb + WL + 3)];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const Sums s = enter(U[q + 1], Vv[q + 1], W[q + 1]);
+    ZU[q + 1] = s.zu;
+    ZV[q + 1] = s.zv;
+    ZW[q + 1] = s.zw;
+    D[q] = s.d;
+    dwc = s.dw;
+  }
+  const float g_ck = M.g_c[K], g_k = M.g[K], g3c_k = M.g3_c[K], g3_k = M.g3[K];
+  const float g3c_k6 = M.g3_c[bnd ? K : K + 6];  // dtopo_str_111 reads six levels up
+
+  for (int m = mb; m < me; ++m) {
+    const int pos = at(m);
+    const int q = qbase + fm * m;
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      U[x] = U[x + 1];
+      Vv[x] = Vv[x + 1];
+      W[x] = W[x + 1];
+      ZU[x] = ZU[x + 1];
+      ZV[x] = ZV[x + 1];
+      ZW[x] = ZW[x + 1];
+    }
+    U[3] = un;
+    Vv[3] = vn;
+    W[3] = wn;
+    // the next plane's columns; one plane past the bounds stays in the
+    // padded array
+    un = A.u1[at(m + 1 + UL + 3)];
+    vn = A.v1[at(m + 1 + VL + 3)];
+    wn = A.w1[at(m + 1 + WL + 3)];
+    float xpart = 0.f;
+    if (AX == 1 && out) xpart = R[3 * rstride + pos];
+    const Sums s = enter(U[3], Vv[3], W[3]);
+    ZU[3] = s.zu;
+    ZV[3] = s.zv;
+    ZW[3] = s.zw;
+    // D[0..2] end at the newest column before this one: u's centre is two
+    // planes behind it, v's one; w's centre is one behind
+    const float dc = AX == 0 ? D[1] : D[2];
+    D[0] = D[1];
+    D[1] = D[2];
+    D[2] = s.d;
+    const float Jii = awp_pow2_div(1.0f, uld(M.f_c, q) * g3c_k);
+    const float J12i = awp_pow2_div(1.0f, uld(M.f, q) * g3c_k6);
+    float acc;
+    if (AX == 0) {
+      acc = P4F(0) * uld(M.f1_1, q - fm) * ZU[0];
+      acc = acc + P4F(1) * uld(M.f1_1, q) * ZU[1];
+      acc = acc + P4F(2) * uld(M.f1_1, q + fm) * ZU[2];
+      acc = acc + P4F(3) * uld(M.f1_1, q + 2 * fm) * ZU[3];
+      const float vs1 =
+          D4F(1) * U[1] + D4F(0) * U[0] + D4F(2) * U[2] + D4F(3) * U[3] - Jii * g_ck * acc;
+      const float vs3 = Jii * dwc;
+      dwc = s.dw;
+      acc = P4F(2) * uld(M.f1_2, q) * ZV[2];
+      acc = acc + P4F(0) * uld(M.f1_2, q - 2 * fm) * ZV[0];
+      acc = acc + P4F(1) * uld(M.f1_2, q - fm) * ZV[1];
+      acc = acc + P4F(3) * uld(M.f1_2, q + fm) * ZV[3];
+      const float xyv2 =
+          D4F(2) * Vv[2] + D4F(0) * Vv[0] + D4F(1) * Vv[1] + D4F(3) * Vv[3] - J12i * g_ck * acc;
+      const float J13i = awp_pow2_div(1.0f, uld(M.f_1, q) * g3_k);
+      const float xzv1 = J13i * dc;
+      acc = P4F(2) * uld(M.f1_c, q) * ZW[2];
+      acc = acc + P4F(0) * uld(M.f1_c, q - 2 * fm) * ZW[0];
+      acc = acc + P4F(1) * uld(M.f1_c, q - fm) * ZW[1];
+      acc = acc + P4F(3) * uld(M.f1_c, q + fm) * ZW[3];
+      const float xzv2 =
+          D4F(2) * W[2] + D4F(0) * W[0] + D4F(1) * W[1] + D4F(3) * W[3] - J13i * g_k * acc;
+      if (out) {
+        R[pos] = vs1;
+        R[2 * rstride + pos] = vs3;
+        R[3 * rstride + pos] = xyv2;
+        R[4 * rstride + pos] = xzv1 + xzv2;
+      }
+    } else {
+      acc = P4F(2) * uld(M.f2_2, q) * ZV[2];
+      acc = acc + P4F(0) * uld(M.f2_2, q - 2) * ZV[0];
+      acc = acc + P4F(1) * uld(M.f2_2, q - 1) * ZV[1];
+      acc = acc + P4F(3) * uld(M.f2_2, q + 1) * ZV[3];
+      const float vs2 =
+          D4F(2) * Vv[2] + D4F(0) * Vv[0] + D4F(1) * Vv[1] + D4F(3) * Vv[3] - Jii * g_ck * acc;
+      acc = P4F(1) * uld(M.f2_1, q) * ZU[1];
+      acc = acc + P4F(0) * uld(M.f2_1, q - 1) * ZU[0];
+      acc = acc + P4F(2) * uld(M.f2_1, q + 1) * ZU[2];
+      acc = acc + P4F(3) * uld(M.f2_1, q + 2) * ZU[3];
+      const float xyv1 =
+          D4F(1) * U[1] + D4F(0) * U[0] + D4F(2) * U[2] + D4F(3) * U[3] - J12i * g_ck * acc;
+      const float J23i = awp_pow2_div(1.0f, uld(M.f_2, q) * g3_k);
+      const float yzv1 = J23i * dc;
+      acc = P4F(1) * uld(M.f2_c, q) * ZW[1];
+      acc = acc + P4F(0) * uld(M.f2_c, q - 1) * ZW[0];
+      acc = acc + P4F(2) * uld(M.f2_c, q + 1) * ZW[2];
+      acc = acc + P4F(3) * uld(M.f2_c, q + 2) * ZW[3];
+      const float yzv2 =
+          D4F(1) * W[1] + D4F(0) * W[0] + D4F(2) * W[2] + D4F(3) * W[3] - J23i * g_k * acc;
+      if (out) {
+        R[rstride + pos] = vs2;
+        R[3 * rstride + pos] = xyv1 + xpart;
+        R[5 * rstride + pos] = yzv1 + yzv2;
+      }
+    }
+  }
 }
 
 // The relaxation texture of the Q pass: the per-cell arrays (TOPO_TEX_ARRAYS),
@@ -1144,6 +1390,14 @@ void topo_tiles(int nz, VelTiles* V) {
   V->nint = V->wtop0 > 3 ? awp_cdiv(V->wtop0 - 3, V->step) : 0;
 }
 
+// Planes per march of a strain-rate launch: towards 16384 waves, 4 to 32
+// planes (a march re-reads and re-sums 3 columns at its start).
+int topo_chunk(int planes, int waves) {
+  if (awp_tuning().topo_rate_chunk > 0) return awp_tuning().topo_rate_chunk;
+  const long long c = (long long)planes * waves / 16384;
+  return c < 4 ? 4 : c > 32 ? 32 : (int)c;
+}
+
 template <class ST>
 void topo_velocity_launch(topo_t* T, const WaveScales& W, const char* where) {
   TGeom G;
@@ -1291,12 +1545,9 @@ void topo_stress_launch(topo_t* T, const WaveScales& W, const char* where, float
   V.wsync = awp_tuning().topo_wsync;
   dim3 block(64, V.nseg * V.rj, 1);
   dim3 grid(V.nint + 1, awp_cdiv(G.ej - G.bj, V.rj), awp_cdiv(G.ei - G.bi, V.ichunk));
-  // LDS of a launch of rate group g: 2 parities x rj rows x its columns
-  auto lds = [&](int g) {
-    return (size_t)2 * V.rj * st_group_ncols(g) * V.ch * sizeof(float);
-  };
+  const size_t lds = (size_t)2 * V.rj * ST_NC * V.ch * sizeof(float);
   if (!rates) {
-    hipLaunchKernelGGL((topo_str_kernel<ST, false>), grid, block, lds(0), st, A, G, V, nullptr,
+    hipLaunchKernelGGL((topo_str_kernel<ST, false>), grid, block, lds, st, A, G, V, nullptr,
                        0ll);
     awp_check_launch(where);
     return;
@@ -1304,20 +1555,18 @@ void topo_stress_launch(topo_t* T, const WaveScales& W, const char* where, float
   // two passes: strain rates into rates, then the material and memory-
   // variable update streaming them back
   const long long rstride = (long long)G.sl * (T->nx + 4 + AWP_NGSL2);
-  if (awp_tuning().topo_str_split == 2) {
-    hipLaunchKernelGGL((topo_str_kernel<ST, true, 1>), grid, block, lds(1), st, A, G, V, rates,
-                       rstride);
-    hipLaunchKernelGGL((topo_str_kernel<ST, true, 3>), grid, block, lds(3), st, A, G, V, rates,
-                       rstride);
-    hipLaunchKernelGGL((topo_str_kernel<ST, true, 4>), grid, block, lds(4), st, A, G, V, rates,
-                       rstride);
-  } else if (awp_tuning().topo_str_split) {
-    hipLaunchKernelGGL((topo_str_kernel<ST, true, 1>), grid, block, lds(1), st, A, G, V, rates,
-                       rstride);
-    hipLaunchKernelGGL((topo_str_kernel<ST, true, 2>), grid, block, lds(2), st, A, G, V, rates,
-                       rstride);
+  if (awp_tuning().topo_str_split) {
+    // one launch per march direction (topo_rates_kernel)
+    const int ni = G.ei - G.bi, nj = G.ej - G.bj;
+    const size_t rlds = (size_t)2 * V.rj * 3 * (V.ch + 2 * RC_PAD) * sizeof(float);
+    V.ichunk = topo_chunk(ni, (V.nint + 1) * nj * V.nseg);
+    const dim3 gi(V.nint + 1, awp_cdiv(nj, V.rj), awp_cdiv(ni, V.ichunk));
+    hipLaunchKernelGGL((topo_rates_kernel<ST, 0>), gi, block, rlds, st, A, G, V, rates, rstride);
+    V.ichunk = topo_chunk(nj, (V.nint + 1) * ni * V.nseg);
+    const dim3 gj(V.nint + 1, awp_cdiv(ni, V.rj), awp_cdiv(nj, V.ichunk));
+    hipLaunchKernelGGL((topo_rates_kernel<ST, 1>), gj, block, rlds, st, A, G, V, rates, rstride);
   } else {
-    hipLaunchKernelGGL((topo_str_kernel<ST, true, 0>), grid, block, lds(0), st, A, G, V, rates,
+    hipLaunchKernelGGL((topo_str_kernel<ST, true>), grid, block, lds, st, A, G, V, rates,
                        rstride);
   }
   const int qchunk = awp_tuning().topo_q_ichunk;

@@ -20,10 +20,11 @@ struct AwpTuning {
   int step_jfast;       // same, fused step
   int topo_vel_split;   // 1: the curvilinear velocity update as one launch per component
   int adj_jgroup;       // adjoint kernels' block order: 0 plane by plane, else j tiles per group
-  int topo_str_split;   // strain-rate pass: 0 one launch, 1 two (normal, shear), 2 three (normal, xy, xz+yz)
+  int topo_str_split;   // strain-rate pass: 0 one launch, else one per march direction
   int kw;               // k-run width of the Cartesian kernels: 0 by the idle-lane rules, 32, 64
   int topo_nseg;        // curvilinear stress kernel: waves per k chunk at most (1: one-wave segments)
   int topo_wsync;       // curvilinear kernels: 1 wave-scope LDS sync where a wave reads only its own
+  int topo_rate_chunk;  // > 0 forces the planes per march of the strain-rate launches
   int topo_rj;          // curvilinear stress kernel: > 0 forces the j rows per workgroup
 };
 
