@@ -11,13 +11,9 @@
 // Defaults from sweeps on MI355X: velocity and stress workgroups of 4 waves in
 // the chunks of awp_split_march (16-wave stress workgroups, of which a CU
 // holds one, took 951 against 832 us at 384x384x256 in bfloat16 storage); the
-// curvilinear velocity update as three launches (0.985 against 1.043 ms for
-// one launch at 384x384x192), its strain-rate pass as three (normal rates,
-// xy, xz and yz: 2.056 -> 2.006 -> 1.948 ms per stress update for one, two,
-// three launches), the velocity waves ordering their LDS at wave scope
-// (1.002 -> 0.971 ms); the adjoint kernels' blocks in groups of 8 j tiles over
+// curvilinear kernels in the chunks of topo_chunk; the adjoint kernels' blocks in groups of 8 j tiles over
 // all planes (adj_stress_local 551 -> 533 us at 256x256x128).
-static AwpTuning g_tuning = {0, 0, 10240, 10240, 0, 0, 1, 1, 8, 16, 1, 32, 2048, 0, 0, 0, 1, 8, 2, 0, 8, 1, 0};
+static AwpTuning g_tuning = {0, 0, 10240, 10240, 0, 0, 1, 1, 0, 16, 0, 32, 2048, 0, 0, 0, 8, 0, 8, 1, 0, 0};
 AwpTuning& awp_tuning() { return g_tuning; }
 
 namespace {
@@ -213,10 +209,10 @@ int awp_set_tuning(const char* key, int value) {
   } else if (!strcmp(key, "step_jfast")) {
     t.step_jfast = value ? 1 : 0;
   } else if (!strcmp(key, "topo_vel_split")) {
-    t.topo_vel_split = value ? 1 : 0;
+    // accepted: the curvilinear velocity update is one launch
   } else if (!strcmp(key, "topo_str_split")) {
+    // accepted: the strain-rate pass is one launch per march direction
     if (value < 0 || value > 2) return -1;
-    t.topo_str_split = value;
   } else if (!strcmp(key, "topo_rate_chunk")) {
     if (value < 0 || value > 4096) return -1;
     t.topo_rate_chunk = value;

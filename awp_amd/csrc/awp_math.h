@@ -54,3 +54,26 @@ __device__ __forceinline__ bool awp_q_low64(float q) {
 __device__ __forceinline__ bool awp_q_low32(float q) {
   return __builtin_bit_cast(uint32_t, q) >= 0x3b23d70au;
 }
+
+// Coarse-grained Q weights, y = awp_rcp(wwo).  Both branches are cheaper than
+// a divergent branch around either.
+// The production update's (kernel.cu:978-1045): binary64 test and quadratic.
+__device__ __forceinline__ float awp_qw_prod(float q, float ca, float cb, float wwo, float y) {
+  const double t = 2. * (double)q;
+  const float quad = (float)((double)ca * t * t + (double)cb * t);
+  return awp_div_by(awp_q_low64(q) ? quad : 2.0f * wwo * q, wwo, y);
+}
+
+// dstrqc_new's (kernel.cu:505-604) and the curvilinear update's: binary32
+// test; qpa keeps a binary64 quadratic (dbl), the others are binary32.
+__device__ __forceinline__ float awp_qw_new(float q, float ca, float cb, float wwo, float y,
+                                            bool dbl) {
+  float quad;
+  if (dbl) {
+    const double t = 2. * (double)q;
+    quad = (float)((double)ca * t * t + (double)cb * t);
+  } else {
+    quad = ca * (2.0f * q) * (2.0f * q) + cb * (2.0f * q);
+  }
+  return awp_div_by(awp_q_low32(q) ? quad : 2.0f * wwo * q, wwo, y);
+}

@@ -26,28 +26,6 @@ struct StrLaunch {
   float c1, c2, dth, dh1, DT;
 };
 
-// Production Q weight (kernel.cu:978-1045), y = awp_rcp(wwo).  Both branches
-// are cheaper than a divergent branch around either, so they are selected.
-__device__ __forceinline__ float qw_prod(float q, float ca, float cb, float wwo, float y) {
-  const double t = 2. * (double)q;
-  const float quad = (float)((double)ca * t * t + (double)cb * t);
-  return awp_div_by(awp_q_low64(q) ? quad : 2.0f * wwo * q, wwo, y);
-}
-
-// dstrqc_new's Q weights (kernel.cu:505-604): float test; qpa keeps a double
-// quadratic, the others are float.
-__device__ __forceinline__ float qw_new(float q, float ca, float cb, float wwo, float y,
-                                        bool dbl) {
-  float quad;
-  if (dbl) {
-    const double t = 2. * (double)q;
-    quad = (float)((double)ca * t * t + (double)cb * t);
-  } else {
-    quad = ca * (2.0f * q) * (2.0f * q) + cb * (2.0f * q);
-  }
-  return awp_div_by(awp_q_low32(q) ? quad : 2.0f * wwo * q, wwo, y);
-}
-
 // OOP: the stresses before the step are read from s0 (xx yy zz xy xz yz) and
 // the updated ones written to xx..yz (distinct arrays); otherwise xx..yz are
 // updated in place and s0 is unused.  The memory variables are always
@@ -197,26 +175,26 @@ __global__ __launch_bounds__(64 * MAXW) void dstrqc_kernel(
     float qpa, h, h1, h2, h3, qpaw, hw, h1w, h2w, h3w;
     if (!NEWLIT) {
       qpa = 0.0625f * sp8;
-      qpaw = qw_prod(qpa, ca, cb, f_wwo, r_wwo);
+      qpaw = awp_qw_prod(qpa, ca, cb, f_wwo, r_wwo);
       h = 0.0625f * ss8;
-      hw = qw_prod(h, ca, cb, f_wwo, r_wwo);
+      hw = awp_qw_prod(h, ca, cb, f_wwo, r_wwo);
       h1 = 0.250f * (sc + skm);
-      h1w = qw_prod(h1, ca, cb, f_wwo, r_wwo);
+      h1w = awp_qw_prod(h1, ca, cb, f_wwo, r_wwo);
       h2 = 0.250f * (sc + sjm);
-      h2w = qw_prod(h2, ca, cb, f_wwo, r_wwo);
+      h2w = awp_qw_prod(h2, ca, cb, f_wwo, r_wwo);
       h3 = 0.250f * (sc + Sc);
-      h3w = qw_prod(h3, ca, cb, f_wwo, r_wwo);
+      h3w = awp_qw_prod(h3, ca, cb, f_wwo, r_wwo);
     } else {
       qpa = 0.0625f * sp8;
-      qpaw = qw_new(qpa, ca, cb, f_wwo, r_wwo, true);
+      qpaw = awp_qw_new(qpa, ca, cb, f_wwo, r_wwo, true);
       h = 0.0625f * ss8;
-      hw = qw_new(h, ca, cb, f_wwo, r_wwo, false);
+      hw = awp_qw_new(h, ca, cb, f_wwo, r_wwo, false);
       h1 = 0.250f * (sc + skm);
-      h1w = qw_new(h1, ca, cb, f_wwo, r_wwo, false);
+      h1w = awp_qw_new(h1, ca, cb, f_wwo, r_wwo, false);
       h2 = 0.250f * (sc + sjm);
-      h2w = qw_new(h2, ca, cb, f_wwo, r_wwo, false);
+      h2w = awp_qw_new(h2, ca, cb, f_wwo, r_wwo, false);
       h3 = 0.250f * (sc + Sc);
-      h3w = qw_new(h3, ca, cb, f_wwo, r_wwo, false);
+      h3w = awp_qw_new(h3, ca, cb, f_wwo, r_wwo, false);
     }
     h = -xm * hw * dh1;
     h1 = -xmu1 * h1w * dh1;

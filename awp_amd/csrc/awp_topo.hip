@@ -41,10 +41,6 @@ constexpr FTab<R, C> ftab(const double (&a)[R][C]) {
   return t;
 }
 
-__constant__ FTab<6, 9> c_vel_dhpz4r = ftab(TV_DHPZ4R);
-__constant__ FTab<6, 8> c_vel_dhz4r = ftab(TV_DHZ4R);
-__constant__ FTab<6, 9> c_vel_dphz4r = ftab(TV_DPHZ4R);
-__constant__ FTab<6, 7> c_vel_dz4r = ftab(TV_DZ4R);
 __constant__ FTab<6, 9> c_str_phdz4r = ftab(TS_PHDZ4R);
 __constant__ FTab<6, 7> c_str_dz4r = ftab(TS_DZ4R);
 __constant__ FTab<6, 8> c_str_dhz4r = ftab(TS_DHZ4R);
@@ -102,27 +98,29 @@ __device__ __forceinline__ void wave_lds_sync() {
 // 3 <= k < nz-6 and dtopo_vel_112 (optimized_velocity.cu:1040-1627) on the top
 // six, in one kernel.
 //
-// A wave owns one (j, 64-level) column segment and marches along i.  At every
-// plane each lane forms, at its own level, the six horizontal 4-point
-// interpolants whose z derivatives the metric terms need, and publishes them
-// (with its own s13, s23, s33) in LDS; the 7-point (9-point on the top rows)
-// z sums then read the neighbouring levels from LDS instead of recomputing
-// 7 x 4 loads per term.  The x neighbours travel in register windows.  Lanes
-// 3..60 of a segment produce output, so segments start every 58 levels; the
-// last segment of a column ends at level nz-1 and also takes the one-sided top
-// rows (table row kk = nz-1-k), as a divergent branch of its wave.
-#define VT_BJ 4      // waves (j columns) per workgroup
-#define VT_NL 9      // LDS arrays per wave
-#define VT_MAXW 8    // waves per workgroup of the chunked stress kernel at most
+// A workgroup owns a chunk of 64 * nseg levels of one j row (several rows of
+// one-wave chunks) and marches along i.  At every plane each lane forms, at
+// its own level, the horizontal 4-point interpolants whose z derivatives the
+// metric terms need, and publishes them (with its own s13, s23, s33) in LDS;
+// the 7-point (9-point on the top rows) z sums then read the neighbouring
+// levels from LDS.  The x neighbours travel in register windows.  A chunk
+// writes all but its 3 outermost levels on either side, so chunks overlap by
+// six; the last one ends at level nz-1 and takes the one-sided top rows (table
+// row kk = nz-1-k) too: its waves that hold any form every z sum with
+// per-lane coefficients, so their lanes do not diverge.
+#define VT_MAXW 8    // waves per workgroup at most
+#define VT_NL 9      // staged LDS columns per row
+#define VT_PAD 4     // LDS floats before and after a staged column: the halo lanes of
+                     // a chunk read up to 3 levels outside it and discard the sums
 
-// The k tiling of a launch.  The velocity kernel takes one-wave segments
-// (the first four fields, 58 outputs each); the stress kernel takes chunks
-// of nseg waves that share one LDS column (all fields, topo_tiles).
+// The k tiling of a curvilinear launch (topo_tiles): chunks of nseg waves that
+// share one LDS column.
 struct VelTiles {
-  int nint;   // interior segments / chunks (58 or ch - 6 outputs each, from level 3)
-  int ktop0;  // first level of the top one (nz - 64 or nz - ch, may be negative)
-  int wtop0;  // first level the top one writes
+  int nint;   // interior chunks (ch - 6 outputs each, from level 3)
+  int ktop0;  // first level of the top chunk (nz - ch, may be negative)
+  int wtop0;  // first level the top chunk writes
   int ichunk; // planes per march
+  int njt;    // j tiles (velocity)
   int nseg;   // waves per chunk (64 levels each)
   int ch;     // levels per chunk, 64 * nseg
   int step;   // ch - 6
@@ -130,67 +128,175 @@ struct VelTiles {
   int wsync;  // 1: a wave that reads only its own LDS syncs at wave scope, not the workgroup's
 };
 
-// COMP: 0 updates u1, u2 and u3; 1, 2, 3 update only u1, u2 or u3 (the
-// other components' loads, LDS rows and arithmetic drop out), so three
-// launches with fewer live registers each give the same results.  The
-// one-component launches are asked for 8 waves per SIMD (64 VGPRs: 58-64
-// from 71-75, no spills in binary32).
-template <class ST, int COMP = 0>
-__global__ __launch_bounds__(64 * VT_BJ) __attribute__((amdgpu_waves_per_eu(COMP == 0 ? 1 : 8)))
-void topo_vel_kernel(const TopoVelArgs<ST> A,
-                                                              const TGeom G, const VelTiles V) {
-  constexpr bool DU = COMP == 0 || COMP == 1, DV = COMP == 0 || COMP == 2,
-                 DW = COMP == 0 || COMP == 3;
-  __shared__ float lds[2][VT_BJ][VT_NL][64];
+// A float read at a wave-uniform index of an array that no kernel in flight
+// writes: through the constant address space it is a scalar load.
+typedef const __attribute__((address_space(4))) float* uniform_ptr;
+__device__ __forceinline__ float uld(const float* a, int i) { return ((uniform_ptr)a)[i]; }
+
+// Order of an interior 7-point row: the middle, then from one end.
+__host__ __device__ constexpr int rt_mid(int t) { return t == 0 ? 3 : t <= 3 ? t - 1 : t; }
+
+// Per-lane coefficients [term][class] of the waves with one-sided rows: class
+// 0..5 is the row of level nz-1-class, the level furthest from the top
+// first; class 6 the interior row in its own order, then zeros for the terms
+// a one-sided row has more (they weigh the lane's own level).
+#define VT_ZC 0    // dhpz4 (times g_c)
+#define VT_ZN 9    // dphz4 (times g)
+#define VT_DHZ 18  // dhz4
+#define VT_DZ 26   // dz4
+#define VT_N 33
+struct VelTop {
+  float v[VT_N][8];
+};
+constexpr VelTop vel_top() {
+  VelTop T{};
+  constexpr int dho[4] = {2, 0, 1, 3}, dzo[4] = {1, 0, 2, 3};
+  for (int c = 0; c < 6; ++c) {
+    for (int t = 0; t < 9; ++t) {
+      T.v[VT_ZC + t][c] = (float)TV_DHPZ4R[c][8 - t];
+      T.v[VT_ZN + t][c] = (float)TV_DPHZ4R[c][8 - t];
+    }
+    for (int t = 0; t < 8; ++t) T.v[VT_DHZ + t][c] = (float)TV_DHZ4R[c][7 - t];
+    for (int t = 0; t < 7; ++t) T.v[VT_DZ + t][c] = (float)TV_DZ4R[c][6 - t];
+  }
+  for (int t = 0; t < 7; ++t) {
+    T.v[VT_ZC + t][6] = (float)TV_DHPZ4[rt_mid(t)];
+    T.v[VT_ZN + t][6] = (float)TV_DPHZ4[rt_mid(t)];
+  }
+  for (int t = 0; t < 4; ++t) {
+    T.v[VT_DHZ + t][6] = (float)TOPO_D4[dho[t]];
+    T.v[VT_DZ + t][6] = (float)TOPO_D4[dzo[t]];
+  }
+  return T;
+}
+__constant__ VelTop c_vel_top = vel_top();
+
+// All three components in one launch: it reads 10 arrays and writes 3 where a
+// launch per component reads 15 (384x384x192: 500 against 530 us; 256x256x192
+// 233 against 243).
+template <class ST>
+__global__ __launch_bounds__(64 * VT_MAXW) void topo_vel_kernel(const TopoVelArgs<ST> A,
+                                                               const TGeom G,
+                                                               const VelTiles V) {
+  constexpr int NL = VT_NL;
+  constexpr int CU = 0, CV = 3, CW = 6;  // columns: two interpolants and a stress each
+  extern __shared__ float vt_lds[];  // [parity][row][column][VT_PAD + ch + VT_PAD]
+  __shared__ float s_top[VT_N * 8];
   const int lane = (int)threadIdx.x;
   const int w = (int)threadIdx.y;
-  const int t = (int)blockIdx.x;
+  const int seg = w % V.nseg, row = w / V.nseg;
+  // k chunks fastest, then j tiles, then i chunks, a contiguous run of them
+  // per XCD: the rows that neighbouring j tiles share meet in one L2
+  const int b = awp_xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  const int t = b % (V.nint + 1), jt = b / (V.nint + 1) % V.njt;
+  const int ic = b / ((V.nint + 1) * V.njt);
   const bool top = t == V.nint;
-  const int k0 = top ? V.ktop0 : 58 * t;
-  const int k = k0 + lane;
+  if (top) {  // uniform over the workgroup
+    for (int e = w * 64 + lane; e < VT_N * 8; e += V.nseg * V.rj * 64)
+      s_top[e] = (&c_vel_top.v[0][0])[e];
+    __syncthreads();
+  }
+  const int k0 = top ? V.ktop0 : V.step * t;
+  const int kl = seg * 64 + lane;  // level within the chunk
+  const int k = k0 + kl;
   const int nz = G.nz;
   // levels this lane writes
-  const int w0 = top ? V.wtop0 : 58 * t + 3;
-  const int w1 = top ? nz : (58 * t + 61 < V.wtop0 ? 58 * t + 61 : V.wtop0);
-  bool out = k >= w0 && k < w1;
-  const bool bnd = k >= nz - 6;  // one-sided rows (top segment only)
-  const int kk = nz - 1 - k;
+  const int w0 = top ? V.wtop0 : V.step * t + 3;
+  const int w1 = top ? nz : (V.step * t + V.ch - 3 < V.wtop0 ? V.step * t + V.ch - 3 : V.wtop0);
+  const bool bnd = k >= nz - 6;  // one-sided rows (top chunk only)
+  const bool topw = top && __builtin_amdgcn_readfirstlane(k0 + seg * 64 + 63) >= nz - 6;
   // every wave of the workgroup runs the same planes (uniform barrier count);
   // a wave past the last column works on a copy of it and stores nothing
-  const int jw = G.bj + (int)(blockIdx.y * VT_BJ) + w;
+  const int jw = G.bj + jt * V.rj + row;
   const bool jok = jw < G.ej;
   const int j = __builtin_amdgcn_readfirstlane(jok ? jw : G.ej - 1);
-  const int ib = (int)blockIdx.z * V.ichunk;
+  const int ib = ic * V.ichunk;
   const int ie = ib + V.ichunk < G.ei ? ib + V.ichunk : G.ei;
   if (ib >= ie) return;  // uniform over the workgroup
-  out = out && jok;
+  const bool out = k >= w0 && k < w1 && jok;
   const int sl = G.sl, yl = G.yl, fr = G.frow;
-  // every lane reads at its own level; the top segment of a grid with
-  // nz < 64 starts below level 0, and those lanes (never outputs, never read
+  // every lane reads at its own level; the top chunk of a grid with
+  // nz < ch starts below level 0, and those lanes (never outputs, never read
   // by an output's stencil) read level 0 instead
   const int kr = k < 0 ? 0 : k;
   const int kg = kr + AWP_ALIGN;
   const int col0 = yl * (j + AWP_NGSL + 2) + AWP_ALIGN;   // level 0 of column (i = -10)
   const TMetrics& M = A.M;
+  const int cp = V.ch + 2 * VT_PAD;
+  const int own = VT_PAD + kl;          // this lane's level in a staged column
+  const int lb = VT_PAD + nz - 1 - k0;  // level nz-1 (top chunk)
+  const int cls = bnd ? nz - 1 - k : 6;
 
-  constexpr float dhpz4[7] = {(float)TV_DHPZ4[0], (float)TV_DHPZ4[1], (float)TV_DHPZ4[2],
-                              (float)TV_DHPZ4[3], (float)TV_DHPZ4[4], (float)TV_DHPZ4[5],
-                              (float)TV_DHPZ4[6]};
-  constexpr float dphz4[7] = {(float)TV_DPHZ4[0], (float)TV_DPHZ4[1], (float)TV_DPHZ4[2],
-                              (float)TV_DPHZ4[3], (float)TV_DPHZ4[4], (float)TV_DPHZ4[5],
-                              (float)TV_DPHZ4[6]};
-  // per-level weights of the z sums (interior rows); the top rows form theirs
-  // from the tables inside their branch
-  float cz[7], czp[7];
+  // per-level weights of the z sums, term by term in the order they are added
+  // (7 terms; 9 in the waves with one-sided rows)
+  float cz[9], czp[9];
+  if (!topw) {
 #pragma unroll
-  for (int m = 0; m < 7; ++m) {
-    const int kk2 = kg + m - 3;  // >= align - 3
-    cz[m] = dhpz4[m] * M.g_c[kk2];
-    czp[m] = dphz4[m] * M.g[kk2];
+    for (int m = 0; m < 7; ++m) {
+      const int kk2 = kg + rt_mid(m) - 3;  // >= align - 3
+      cz[m] = (float)TV_DHPZ4[rt_mid(m)] * M.g_c[kk2];
+      czp[m] = (float)TV_DPHZ4[rt_mid(m)] * M.g[kk2];
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < 9; ++m) {
+      const int kk2 = AWP_ALIGN + (bnd ? nz - 9 + m : kr + (m < 7 ? rt_mid(m) - 3 : 0));
+      cz[m] = s_top[(VT_ZC + m) * 8 + cls] * M.g_c[kk2];
+      czp[m] = s_top[(VT_ZN + m) * 8 + cls] * M.g[kk2];
+    }
   }
+  // z sum of a staged column with weights c
+  auto zsum = [&](const float(&c)[9], const float* L) {
+    float acc = 0.f;
+    if (!topw) {
+#pragma unroll
+      for (int m = 0; m < 7; ++m) {
+        const float x = c[m] * L[own + rt_mid(m) - 3];
+        acc = m == 0 ? x : acc + x;
+      }
+    } else {
+#pragma unroll
+      for (int m = 0; m < 9; ++m) {
+        const float x = c[m] * L[bnd ? lb - 8 + m : own + (m < 7 ? rt_mid(m) - 3 : 0)];
+        acc = m == 0 ? x : acc + x;
+      }
+    }
+    return acc;
+  };
+  // acc (if any) plus the terms of dhz4 / dz4 on a staged column
+  auto add_dhz = [&](bool first, float acc, const float* L) {
+    if (!topw) {
+      const float x = D4F(2) * L[own];
+      acc = first ? x : acc + x;
+      acc = acc + D4F(0) * L[own - 2];
+      acc = acc + D4F(1) * L[own - 1];
+      return acc + D4F(3) * L[own + 1];
+    }
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      const int o = m == 1 ? -2 : m == 2 ? -1 : m == 3 ? 1 : 0;
+      const float x = s_top[(VT_DHZ + m) * 8 + cls] * L[bnd ? lb - 7 + m : own + o];
+      acc = first && m == 0 ? x : acc + x;
+    }
+    return acc;
+  };
+  auto add_dz = [&](float acc, const float* L) {
+    if (!topw) {
+      acc = acc + D4F(1) * L[own];
+      acc = acc + D4F(0) * L[own - 1];
+      acc = acc + D4F(2) * L[own + 1];
+      return acc + D4F(3) * L[own + 2];
+    }
+#pragma unroll
+    for (int m = 0; m < 7; ++m) {
+      const int o = m == 1 ? -1 : m == 2 ? 1 : m == 3 ? 2 : 0;
+      acc = acc + s_top[(VT_DZ + m) * 8 + cls] * L[bnd ? lb - 6 + m : own + o];
+    }
+    return acc;
+  };
   const float g3c = M.g3_c[kg], g3v = M.g3[kg];
   const float dcz = A.dcrjz[kg];
-  const float dcy = A.dcrjy[j + AWP_NGSL + 2];
+  const float dcy = uld(A.dcrjy, j + AWP_NGSL + 2);
 
   // x windows at level k: s11(i-2..i+1), s12(i-1..i+2), s13(i-1..i+2)
   auto P = [&](int i) { return col0 + sl * (i + AWP_NGSL + 2) + kr; };
@@ -221,174 +327,96 @@ void topo_vel_kernel(const TopoVelArgs<ST> A,
                 s22p2 = A.s22[p + 2 * yl];
     const float s23m2 = A.s23[p - 2 * yl], s23m1 = A.s23[p - yl], s23o = A.s23[p],
                 s23p1 = A.s23[p + yl];
-    const float s33o = A.s33[p];
     const float s12o = s12x[1], s13o = s13x[1];
+    float* L = vt_lds + (par * V.rj + row) * NL * cp;
     // interpolants at this level, operands in the reference's order
-    const float I11 = P4F(2) * s11w[2] + P4F(0) * s11w[0] + P4F(1) * s11w[1] + P4F(3) * s11w[3];
-    const float I12 = P4F(2) * s12o + P4F(0) * s12m2 + P4F(1) * s12m1 + P4F(3) * s12p1;
-    const float I12x = P4F(1) * s12x[1] + P4F(0) * s12x[0] + P4F(2) * s12x[2] + P4F(3) * s12x[3];
-    const float I22 = P4F(1) * s22o + P4F(0) * s22m1 + P4F(2) * s22p1 + P4F(3) * s22p2;
-    const float I13 = P4F(1) * s13x[1] + P4F(0) * s13x[0] + P4F(2) * s13x[2] + P4F(3) * s13x[3];
-    const float I23 = P4F(2) * s23o + P4F(0) * s23m2 + P4F(1) * s23m1 + P4F(3) * s23p1;
-    float(*L)[64] = lds[par][w];
-    if (DU) {
-      L[0][lane] = I11;
-      L[1][lane] = I12;
-      L[6][lane] = s13o;
-    }
-    if (DV) {
-      L[2][lane] = I12x;
-      L[3][lane] = I22;
-      L[7][lane] = s23o;
-    }
-    if (DW) {
-      L[4][lane] = I13;
-      L[5][lane] = I23;
-      L[8][lane] = s33o;
-    }
-    // density at plane i
+    L[CU * cp + own] =
+        P4F(2) * s11w[2] + P4F(0) * s11w[0] + P4F(1) * s11w[1] + P4F(3) * s11w[3];
+    L[(CU + 1) * cp + own] =
+        P4F(2) * s12o + P4F(0) * s12m2 + P4F(1) * s12m1 + P4F(3) * s12p1;
+    L[(CU + 2) * cp + own] = s13o;
+    L[CV * cp + own] =
+        P4F(1) * s12x[1] + P4F(0) * s12x[0] + P4F(2) * s12x[2] + P4F(3) * s12x[3];
+    L[(CV + 1) * cp + own] =
+        P4F(1) * s22o + P4F(0) * s22m1 + P4F(2) * s22p1 + P4F(3) * s22p2;
+    L[(CV + 2) * cp + own] = s23o;
+    L[CW * cp + own] =
+        P4F(1) * s13x[1] + P4F(0) * s13x[0] + P4F(2) * s13x[2] + P4F(3) * s13x[3];
+    L[(CW + 1) * cp + own] =
+        P4F(2) * s23o + P4F(0) * s23m2 + P4F(1) * s23m1 + P4F(3) * s23p1;
+    L[(CW + 2) * cp + own] = A.s33[p];
+    // density at plane i, and the velocities before the step
     const float r_k1 = A.rho[p - 1], r_k = A.rho[p], r_j = A.rho[p - yl],
                 r_jk1 = A.rho[p - yl - 1];
-    // each wave reads only its own LDS rows: with wsync the waves of a
-    // workgroup do not wait for each other
-    if (V.wsync)
+    const float u = ST::ld(A.u1, p, A.su1), v = ST::ld(A.u2, p, A.su2),
+                x = ST::ld(A.u3, p, A.su3);
+    // one-wave chunks read only their own LDS rows: with wsync the waves of
+    // the workgroup do not wait for each other
+    if (V.wsync && V.nseg == 1)
       wave_lds_sync();
     else
       __syncthreads();
 
-    if (out) {
-      const int q = (j + AWP_ALIGN + AWP_NGSL + 2) + (i + AWP_NGSL + 2) * fr;
-      float rho1, rho2, rho3;
-      if (!bnd) {
-        const float c = 0.25f;
-        rho1 = c * (r_k1 + r_jk1) + c * (r_k + r_j);
-        rho2 = c * (r_k1 + rm_k1) + c * (r_k + rm_k);
-        rho3 = c * (r_k + rm_k) + c * (r_j + rm_j);
-      } else {
-        rho1 = (float)(0.25 * (double)(r_k1 + r_jk1) + 0.25 * (double)(r_k + r_j));
-        rho2 = (float)(0.25 * (double)(r_k1 + rm_k1) + 0.25 * (double)(r_k + rm_k));
-        rho3 = (float)(0.25 * (double)(r_k + rm_k) + 0.25 * (double)(r_j + rm_j));
-      }
-      float Ai1 = M.f_1[q] * g3c * rho1;
-      Ai1 = dbl_quot(A.nu, Ai1);
-      float Ai2 = M.f_2[q] * g3c * rho2;
-      Ai2 = dbl_quot(A.nu, Ai2);
-      float Ai3 = M.f_c[q] * g3v * rho3;
-      Ai3 = dbl_quot(A.nu, Ai3);
-      const float f_dcrj = A.dcrjx[i + AWP_NGSL + 2] * dcy * dcz;
-      float z11, z12, z12x, z22, z13, z23;
-      if (!bnd) {
-        // order 3, 0, 1, 2, 4, 5, 6
-#pragma unroll
-        for (int tt = 0; tt < 7; ++tt) {
-          const int m = tt == 0 ? 3 : (tt <= 3 ? tt - 1 : tt);
-          const int o = lane + m - 3;
-          const float t11 = cz[m] * L[0][o], t12 = cz[m] * L[1][o];
-          const float t12x = cz[m] * L[2][o], t22 = cz[m] * L[3][o];
-          const float t13 = czp[m] * L[4][o], t23 = czp[m] * L[5][o];
-          if (tt == 0) {
-            z11 = t11; z12 = t12; z12x = t12x; z22 = t22; z13 = t13; z23 = t23;
-          } else {
-            z11 = z11 + t11; z12 = z12 + t12; z12x = z12x + t12x; z22 = z22 + t22;
-            z13 = z13 + t13; z23 = z23 + t23;
-          }
-        }
-      } else {
-        // levels nz-9 .. nz-1 live in lanes 55 .. 63 of the top segment
-        const int lb = nz - 1 - k0;  // lane of level nz-1
-#pragma unroll
-        for (int m = 8; m >= 0; --m) {
-          const int o = lb - m;
-          const float cr = c_vel_dhpz4r.v[kk][m] * M.g_c[AWP_ALIGN + nz - 1 - m];
-          const float crp = c_vel_dphz4r.v[kk][m] * M.g[AWP_ALIGN + nz - 1 - m];
-          const float t11 = cr * L[0][o], t12 = cr * L[1][o];
-          const float t12x = cr * L[2][o], t22 = cr * L[3][o];
-          const float t13 = crp * L[4][o], t23 = crp * L[5][o];
-          if (m == 8) {
-            z11 = t11; z12 = t12; z12x = t12x; z22 = t22; z13 = t13; z23 = t23;
-          } else {
-            z11 = z11 + t11; z12 = z12 + t12; z12x = z12x + t12x; z22 = z22 + t22;
-            z13 = z13 + t13; z23 = z23 + t23;
-          }
-        }
-      }
-      float s;
-      // u1
-      if (DU) {
-      s = D4F(2) * M.f_c[q] * g3c * s11w[2];
-      s = s + D4F(0) * M.f_c[q - 2 * fr] * g3c * s11w[0];
-      s = s + D4F(1) * M.f_c[q - fr] * g3c * s11w[1];
-      s = s + D4F(3) * M.f_c[q + fr] * g3c * s11w[3];
-      s = s + D4F(2) * M.f[q] * g3c * s12o;
-      s = s + D4F(0) * M.f[q - 2] * g3c * s12m2;
-      s = s + D4F(1) * M.f[q - 1] * g3c * s12m1;
-      s = s + D4F(3) * M.f[q + 1] * g3c * s12p1;
-      if (!bnd) {
-        s = s + D4F(2) * L[6][lane];
-        s = s + D4F(0) * L[6][lane - 2];
-        s = s + D4F(1) * L[6][lane - 1];
-        s = s + D4F(3) * L[6][lane + 1];
-      } else {
-        const int lb = nz - 1 - k0;
-#pragma unroll
-        for (int m = 7; m >= 0; --m) s = s + c_vel_dhz4r.v[kk][m] * L[6][lb - m];
-      }
-      s = s - M.f1_1[q] * z11;
-      s = s - M.f2_1[q] * z12;
-      const float v1 = (A.a * ST::ld(A.u1, p, A.su1) + Ai1 * s) * f_dcrj;
-      ST::st(A.u1, p, v1, A.iu1);
-      }
-      // u2
-      if (DV) {
-      if (!bnd) {
-        s = D4F(2) * s23o;
-        s = s + D4F(0) * L[7][lane - 2];
-        s = s + D4F(1) * L[7][lane - 1];
-        s = s + D4F(3) * L[7][lane + 1];
-      } else {
-        const int lb = nz - 1 - k0;
-        s = c_vel_dhz4r.v[kk][7] * L[7][lb - 7];
-#pragma unroll
-        for (int m = 6; m >= 0; --m) s = s + c_vel_dhz4r.v[kk][m] * L[7][lb - m];
-      }
-      s = s + D4F(1) * M.f[q] * g3c * s12x[1];
-      s = s + D4F(0) * M.f[q - fr] * g3c * s12x[0];
-      s = s + D4F(2) * M.f[q + fr] * g3c * s12x[2];
-      s = s + D4F(3) * M.f[q + 2 * fr] * g3c * s12x[3];
-      s = s + D4F(1) * M.f_c[q] * g3c * s22o;
-      s = s + D4F(0) * M.f_c[q - 1] * g3c * s22m1;
-      s = s + D4F(2) * M.f_c[q + 1] * g3c * s22p1;
-      s = s + D4F(3) * M.f_c[q + 2] * g3c * s22p2;
-      s = s - M.f1_2[q] * z12x;
-      s = s - M.f2_2[q] * z22;
-      const float v2 = (A.a * ST::ld(A.u2, p, A.su2) + Ai2 * s) * f_dcrj;
-      ST::st(A.u2, p, v2, A.iu2);
-      }
-      // u3
-      if (DW) {
-      s = D4F(2) * M.f_2[q] * g3v * s23o;
-      s = s + D4F(0) * M.f_2[q - 2] * g3v * s23m2;
-      s = s + D4F(1) * M.f_2[q - 1] * g3v * s23m1;
-      s = s + D4F(3) * M.f_2[q + 1] * g3v * s23p1;
-      s = s + D4F(1) * M.f_1[q] * g3v * s13x[1];
-      s = s + D4F(0) * M.f_1[q - fr] * g3v * s13x[0];
-      s = s + D4F(2) * M.f_1[q + fr] * g3v * s13x[2];
-      s = s + D4F(3) * M.f_1[q + 2 * fr] * g3v * s13x[3];
-      if (!bnd) {
-        s = s + D4F(1) * s33o;
-        s = s + D4F(0) * L[8][lane - 1];
-        s = s + D4F(2) * L[8][lane + 1];
-        s = s + D4F(3) * L[8][lane + 2];
-      } else {
-        const int lb = nz - 1 - k0;
-#pragma unroll
-        for (int m = 6; m >= 0; --m) s = s + c_vel_dz4r.v[kk][m] * L[8][lb - m];
-      }
-      s = s - M.f1_c[q] * z13;
-      s = s - M.f2_c[q] * z23;
-      const float v3 = (A.a * ST::ld(A.u3, p, A.su3) + Ai3 * s) * f_dcrj;
-      ST::st(A.u3, p, v3, A.iu3);
-      }
+    const int q = (j + AWP_ALIGN + AWP_NGSL + 2) + (i + AWP_NGSL + 2) * fr;
+    // the top rows' means are binary64 sums rounded to binary32: the sum of
+    // two binary32 values rounds the same through binary64 (awp_quot's
+    // theorem), and a quarter of it is exact, so one form serves every row
+    const float c = 0.25f;
+    const float f_dcrj = uld(A.dcrjx, i + AWP_NGSL + 2) * dcy * dcz;
+    float s;
+    // u1
+    {
+      const float rho1 = c * (r_k1 + r_jk1) + c * (r_k + r_j);
+      const float Ai1 = awp_div(A.nu, uld(M.f_1, q) * g3c * rho1);
+      const float z11 = zsum(cz, L + CU * cp), z12 = zsum(cz, L + (CU + 1) * cp);
+      s = D4F(2) * uld(M.f_c, q) * g3c * s11w[2];
+      s = s + D4F(0) * uld(M.f_c, q - 2 * fr) * g3c * s11w[0];
+      s = s + D4F(1) * uld(M.f_c, q - fr) * g3c * s11w[1];
+      s = s + D4F(3) * uld(M.f_c, q + fr) * g3c * s11w[3];
+      s = s + D4F(2) * uld(M.f, q) * g3c * s12o;
+      s = s + D4F(0) * uld(M.f, q - 2) * g3c * s12m2;
+      s = s + D4F(1) * uld(M.f, q - 1) * g3c * s12m1;
+      s = s + D4F(3) * uld(M.f, q + 1) * g3c * s12p1;
+      s = add_dhz(false, s, L + (CU + 2) * cp);
+      s = s - uld(M.f1_1, q) * z11;
+      s = s - uld(M.f2_1, q) * z12;
+      if (out) ST::st(A.u1, p, (A.a * u + Ai1 * s) * f_dcrj, A.iu1);
+    }
+    // u2
+    {
+      const float rho2 = c * (r_k1 + rm_k1) + c * (r_k + rm_k);
+      const float Ai2 = awp_div(A.nu, uld(M.f_2, q) * g3c * rho2);
+      const float z12x = zsum(cz, L + CV * cp), z22 = zsum(cz, L + (CV + 1) * cp);
+      s = add_dhz(true, 0.f, L + (CV + 2) * cp);
+      s = s + D4F(1) * uld(M.f, q) * g3c * s12x[1];
+      s = s + D4F(0) * uld(M.f, q - fr) * g3c * s12x[0];
+      s = s + D4F(2) * uld(M.f, q + fr) * g3c * s12x[2];
+      s = s + D4F(3) * uld(M.f, q + 2 * fr) * g3c * s12x[3];
+      s = s + D4F(1) * uld(M.f_c, q) * g3c * s22o;
+      s = s + D4F(0) * uld(M.f_c, q - 1) * g3c * s22m1;
+      s = s + D4F(2) * uld(M.f_c, q + 1) * g3c * s22p1;
+      s = s + D4F(3) * uld(M.f_c, q + 2) * g3c * s22p2;
+      s = s - uld(M.f1_2, q) * z12x;
+      s = s - uld(M.f2_2, q) * z22;
+      if (out) ST::st(A.u2, p, (A.a * v + Ai2 * s) * f_dcrj, A.iu2);
+    }
+    // u3
+    {
+      const float rho3 = c * (r_k + rm_k) + c * (r_j + rm_j);
+      const float Ai3 = awp_div(A.nu, uld(M.f_c, q) * g3v * rho3);
+      const float z13 = zsum(czp, L + CW * cp), z23 = zsum(czp, L + (CW + 1) * cp);
+      s = D4F(2) * uld(M.f_2, q) * g3v * s23o;
+      s = s + D4F(0) * uld(M.f_2, q - 2) * g3v * s23m2;
+      s = s + D4F(1) * uld(M.f_2, q - 1) * g3v * s23m1;
+      s = s + D4F(3) * uld(M.f_2, q + 1) * g3v * s23p1;
+      s = s + D4F(1) * uld(M.f_1, q) * g3v * s13x[1];
+      s = s + D4F(0) * uld(M.f_1, q - fr) * g3v * s13x[0];
+      s = s + D4F(2) * uld(M.f_1, q + fr) * g3v * s13x[2];
+      s = s + D4F(3) * uld(M.f_1, q + 2 * fr) * g3v * s13x[3];
+      s = add_dz(s, L + (CW + 2) * cp);
+      s = s - uld(M.f1_c, q) * z13;
+      s = s - uld(M.f2_c, q) * z23;
+      if (out) ST::st(A.u3, p, (A.a * x + Ai3 * s) * f_dcrj, A.iu3);
     }
     rm_k1 = r_k1;
     rm_k = r_k;
@@ -409,58 +437,51 @@ struct TopoStrArgs {
   float DT, dth, dh1;
 };
 
-__device__ __forceinline__ float topo_qweight(float q, const float* coeff, int ww, float wwo,
-                                              bool dbl_poly) {
-  float w;
-  if (1.0f / (q * 2.0f) <= 200.0f) {
-    if (dbl_poly)
-      w = (float)((double)coeff[ww * 2 - 2] * (2. * (double)q) * (2. * (double)q) +
-                  (double)coeff[ww * 2 - 1] * (2. * (double)q));
-    else
-      w = coeff[ww * 2 - 2] * (2.0f * q) * (2.0f * q) + coeff[ww * 2 - 1] * (2.0f * q);
-  } else {
-    w = 2.0f * wwo * q;
-  }
-  return w / wwo;
+// The corners (j, k), (j-1, k), (j, k-1), (j-1, k-1) of one plane's 8-cell mean.
+struct Corner4 {
+  float c, jm, km, jk;
+};
+struct TopoMedium {
+  Corner4 lam, mu, qp, qs;
+};
+__device__ __forceinline__ Corner4 corner4(const float* a, int pos, int yl) {
+  return Corner4{a[pos], a[pos - yl], a[pos - 1], a[pos - yl - 1]};
+}
+template <class ST>
+__device__ __forceinline__ TopoMedium topo_medium(const TopoStrArgs<ST>& A, int pos, int yl) {
+  return TopoMedium{corner4(A.lam, pos, yl), corner4(A.mu, pos, yl), corner4(A.qp, pos, yl),
+                    corner4(A.qs, pos, yl)};
+}
+__device__ __forceinline__ float sum8(const Corner4& a, const Corner4& b) {
+  return a.c + b.c + a.jm + b.jm + a.km + b.km + a.jk + b.jk;
 }
 
 // The material averages, Q weights and the memory-variable recursion, shared
-// by the interior and the top kernel (stress_attenuation.cu:200-327, 462-467,
-// 534-540, 595-600, 651-656).
-// f_vx1, f_vx2, f_wwo, f_ww: the cell's relaxation texture.
+// by the one-pass kernel and the second pass (stress_attenuation.cu:200-327,
+// 462-467, 534-540, 595-600, 651-656).
+// m0, m1: the medium at planes i and i+1; f_vx1, f_vx2, f_wwo, ca, cb: the
+// cell's relaxation texture; r_wwo = awp_rcp(f_wwo).
 template <class ST>
-__device__ __forceinline__ void topo_str_update(const TopoStrArgs<ST>& A, int pos, int sl, int yl,
-                                                float f_dcrj, float nvs1, float nvs2,
-                                                float nvs3, float xyv, float xzv, float yzv,
-                                                float f_vx1, float f_vx2, float f_wwo,
-                                                int f_ww) {
-  const int pos_ip1 = pos + sl, pos_jm1 = pos - yl, pos_km1 = pos - 1;
-  const int pos_jk1 = pos - yl - 1, pos_ik1 = pos + sl - 1, pos_ijk = pos + sl - yl,
-            pos_ijk1 = pos + sl - yl - 1;
-  const float* lam = A.lam;
-  const float* mu = A.mu;
-  const float* qp = A.qp;
-  const float* qs = A.qs;
-  float xl = 8.0f / (lam[pos] + lam[pos_ip1] + lam[pos_jm1] + lam[pos_ijk] + lam[pos_km1] +
-                     lam[pos_ik1] + lam[pos_jk1] + lam[pos_ijk1]);
-  float xm = 16.0f / (mu[pos] + mu[pos_ip1] + mu[pos_jm1] + mu[pos_ijk] + mu[pos_km1] +
-                      mu[pos_ik1] + mu[pos_jk1] + mu[pos_ijk1]);
-  float xmu1 = 2.0f / (mu[pos] + mu[pos_km1]);
-  float xmu2 = awp_quot(2.0f, mu[pos] + mu[pos_jm1]);
-  float xmu3 = awp_quot(2.0f, mu[pos] + mu[pos_ip1]);
-  xl = xl + xm;
-  float qpa = 0.0625f * (qp[pos] + qp[pos_ip1] + qp[pos_jm1] + qp[pos_ijk] + qp[pos_km1] +
-                         qp[pos_ik1] + qp[pos_jk1] + qp[pos_ijk1]);
-  const float qpaw = topo_qweight(qpa, A.coeff, f_ww, f_wwo, true);
-  float h = 0.0625f * (qs[pos] + qs[pos_ip1] + qs[pos_jm1] + qs[pos_ijk] + qs[pos_km1] +
-                       qs[pos_ik1] + qs[pos_jk1] + qs[pos_ijk1]);
-  const float hw = topo_qweight(h, A.coeff, f_ww, f_wwo, false);
-  float h1 = 0.250f * (qs[pos] + qs[pos_km1]);
-  const float h1w = topo_qweight(h1, A.coeff, f_ww, f_wwo, false);
-  float h2 = 0.250f * (qs[pos] + qs[pos_jm1]);
-  const float h2w = topo_qweight(h2, A.coeff, f_ww, f_wwo, false);
-  float h3 = 0.250f * (qs[pos] + qs[pos_ip1]);
-  const float h3w = topo_qweight(h3, A.coeff, f_ww, f_wwo, false);
+__device__ __forceinline__ void topo_str_update(const TopoStrArgs<ST>& A, int pos, float f_dcrj,
+                                                const TopoMedium& m0, const TopoMedium& m1,
+                                                float nvs1, float nvs2, float nvs3, float xyv,
+                                                float xzv, float yzv, float f_vx1, float f_vx2,
+                                                float f_wwo, float r_wwo, float ca, float cb) {
+  float xm = awp_pow2_div(16.0f, sum8(m0.mu, m1.mu));
+  float xl = awp_pow2_div(8.0f, sum8(m0.lam, m1.lam)) + xm;
+  float xmu1 = awp_pow2_div(2.0f, m0.mu.c + m0.mu.km);
+  float xmu2 = awp_pow2_div(2.0f, m0.mu.c + m0.mu.jm);
+  float xmu3 = awp_pow2_div(2.0f, m0.mu.c + m1.mu.c);
+  float qpa = 0.0625f * sum8(m0.qp, m1.qp);
+  const float qpaw = awp_qw_new(qpa, ca, cb, f_wwo, r_wwo, true);
+  float h = 0.0625f * sum8(m0.qs, m1.qs);
+  const float hw = awp_qw_new(h, ca, cb, f_wwo, r_wwo, false);
+  float h1 = 0.250f * (m0.qs.c + m0.qs.km);
+  const float h1w = awp_qw_new(h1, ca, cb, f_wwo, r_wwo, false);
+  float h2 = 0.250f * (m0.qs.c + m0.qs.jm);
+  const float h2w = awp_qw_new(h2, ca, cb, f_wwo, r_wwo, false);
+  float h3 = 0.250f * (m0.qs.c + m1.qs.c);
+  const float h3w = awp_qw_new(h3, ca, cb, f_wwo, r_wwo, false);
   const float DT = A.DT, dth = A.dth, dh1 = A.dh1;
   h = -xm * hw * dh1;
   h1 = -xmu1 * h1w * dh1;
@@ -552,15 +573,9 @@ enum {
   C_VN, C_VO, C_VM2, C_VM1, C_VP1,   // v1 at (i+1, j), (i, j), (i, j-2), (i, j-1), (i, j+1)
   C_WN, C_WO, C_WM1, C_WP1, C_WP2    // w1 at (i+1, j), (i, j), (i, j-1), (i, j+1), (i, j+2)
 };
-// RATES: store the six strain-rate terms of every output cell into R
-// (TOPO_NRATES arrays of the field's size, rstride floats apart) for
-// topo_str_q_kernel, instead of applying the material and memory-variable
-// update here.
-template <class ST, bool RATES>
+template <class ST>
 __global__ __launch_bounds__(64 * VT_MAXW) void topo_str_kernel(const TopoStrArgs<ST> A,
-                                                              const TGeom G, const VelTiles V,
-                                                              float* __restrict__ R,
-                                                              long long rstride) {
+                                                              const TGeom G, const VelTiles V) {
   // [parity][row][column][level of the chunk]: 2 * rj * ST_NC * ch floats; the
   // column of array c at parity base L
 #define LCOL(c) (L + (c) * V.ch)
@@ -813,17 +828,12 @@ __global__ __launch_bounds__(64 * VT_MAXW) void topo_str_kernel(const TopoStrArg
         xzv = xzv1 + xzv2;
         yzv = yzv1 + yzv2;
       }
-      if (RATES) {
-        R[pos] = vs1;
-        R[rstride + pos] = vs2;
-        R[2 * rstride + pos] = vs3;
-        R[3 * rstride + pos] = xyv;
-        R[4 * rstride + pos] = xzv;
-        R[5 * rstride + pos] = yzv;
-      } else {
-        topo_str_update<ST>(A, pos, sl, yl, f_dcrj, vs1, vs2, vs3, xyv, xzv, yzv, A.vx1[pos],
-                            A.vx2[pos], A.wwo[pos], A.ww[pos]);
-      }
+      const float f_wwo = A.wwo[pos];
+      const int f_ww = A.ww[pos];
+      topo_str_update<ST>(A, pos, f_dcrj, topo_medium<ST>(A, pos, yl),
+                          topo_medium<ST>(A, pos + sl, yl), vs1, vs2, vs3, xyv, xzv, yzv,
+                          A.vx1[pos], A.vx2[pos], f_wwo, awp_rcp(f_wwo), A.coeff[f_ww * 2 - 2],
+                          A.coeff[f_ww * 2 - 1]);
     }
   }
 #undef LCOL
@@ -860,7 +870,6 @@ __global__ __launch_bounds__(64 * VT_MAXW) void topo_str_kernel(const TopoStrArg
 struct RateTop {
   float v[RT_N][8];
 };
-constexpr int rt_mid(int t) { return t == 0 ? 3 : t <= 3 ? t - 1 : t; }
 constexpr RateTop rate_top() {
   RateTop T{};
   constexpr int dzo[4] = {1, 0, 2, 3}, dho[4] = {2, 0, 1, 3};
@@ -884,21 +893,13 @@ constexpr RateTop rate_top() {
 }
 __constant__ RateTop c_rate_top = rate_top();
 
-// A float read at a wave-uniform index of an array that no kernel in flight
-// writes: through the constant address space it is a scalar load.
-typedef const __attribute__((address_space(4))) float* uniform_ptr;
-__device__ __forceinline__ float uld(const float* a, int i) { return ((uniform_ptr)a)[i]; }
-
-#define RC_PAD 4  // LDS floats before and after a staged column: the halo lanes of
-                  // a chunk read up to 3 levels outside it and discard the sums
-
 template <class ST, int AX>
 __global__ __launch_bounds__(64 * VT_MAXW) void topo_rates_kernel(const TopoStrArgs<ST> A,
                                                                   const TGeom G,
                                                                   const VelTiles V,
                                                                   float* __restrict__ R,
                                                                   long long rstride) {
-  extern __shared__ float rt_lds[];  // [parity][row][u, v, w][RC_PAD + ch + RC_PAD]
+  extern __shared__ float rt_lds[];  // [parity][row][u, v, w][VT_PAD + ch + VT_PAD]
   __shared__ float s_top[RT_N * 8];
   const int lane = (int)threadIdx.x;
   const int w = (int)threadIdx.y;
@@ -935,9 +936,9 @@ __global__ __launch_bounds__(64 * VT_MAXW) void topo_rates_kernel(const TopoStrA
   const int base = K + (AX == 0 ? G.yl : G.sl) * f;
   const int qbase = AWP_ALIGN + (AX == 0 ? 1 : G.frow) * f;
   const TMetrics& M = A.M;
-  const int cp = V.ch + 2 * RC_PAD;
-  const int own = RC_PAD + kl;  // this lane's level in a staged column
-  const int lb = RC_PAD + nz - 1 - k0;  // level nz-1 (top chunk)
+  const int cp = V.ch + 2 * VT_PAD;
+  const int own = VT_PAD + kl;  // this lane's level in a staged column
+  const int lb = VT_PAD + nz - 1 - k0;  // level nz-1 (top chunk)
   const int cls = bnd ? nz - 1 - k : 6;
 
   constexpr float phdz4[7] = {(float)TS_PHDZ4[0], (float)TS_PHDZ4[1], (float)TS_PHDZ4[2],
@@ -1140,38 +1141,55 @@ struct TopoTex {
 };
 
 // The material averages, Q weights and memory-variable recursion of the
-// stress update (topo_str_update) over the cells topo_str_kernel<ST, true>
-// wrote rates for: levels 3 <= k < nz of the stress bounds.  One lane per
-// level, 4 rows per workgroup, a march over a chunk of i; few registers, so
-// the per-cell loads of this streaming pass stay in flight.
+// stress update (topo_str_update) over the cells topo_rates_kernel wrote rates
+// for: levels 3 <= k < nz of the stress bounds.  It streams 136 B per cell
+// (6 rates and 4 medium arrays read, 6 stresses and 6 memory variables read
+// and written), so it runs as the Cartesian stress kernel does: tiles of
+// awp_pick_tile in XCD-aware order, an i-march that carries the medium's
+// plane i+1 in registers.  One plane per workgroup, in the launch's own order,
+// fetched the medium's neighbour planes and rows again in every XCD (1.75 GB
+// per 256x256x192 update for 1.11 algorithmic).
+struct TopoQLaunch {
+  AwpTile tile;
+  int nkt, njt, ichunk, nblocks;
+};
+
 template <class ST, int TEX>
-__global__ __launch_bounds__(256) void topo_str_q_kernel(const TopoStrArgs<ST> A, const TGeom G,
+__global__ __launch_bounds__(512) void topo_str_q_kernel(const TopoStrArgs<ST> A, const TGeom G,
                                                          const float* __restrict__ R,
-                                                         long long rstride, int ichunk,
+                                                         long long rstride, const TopoQLaunch L,
                                                          const TopoTex TT) {
-  __shared__ float s_tex[24];
-  if (TEX != TOPO_TEX_ARRAYS) {
-    const int tid = (int)(threadIdx.y * 64 + threadIdx.x);
-    if (tid < 24) s_tex[tid] = TT.t[tid];
-    __syncthreads();
-  }
-  const int k = 3 + (int)(blockIdx.x * 64 + threadIdx.x);  // topographic level
-  const int j = G.bj + (int)(blockIdx.y * 4 + threadIdx.y);
-  const int ib = G.bi + (int)blockIdx.z * ichunk;
-  const int ie = ib + ichunk < G.ei ? ib + ichunk : G.ei;
-  if (k >= G.nz || j >= G.ej) return;
+  __shared__ float s_tex[32];  // vx1[8], vx2[8], wwo[8], 1/wwo[8]
+  __shared__ float s_coeff[16];
+  const int tid = (int)threadIdx.x;
+  if (tid < 16) s_coeff[tid] = A.coeff[tid];
+  if (TEX != TOPO_TEX_ARRAYS && tid < 32)
+    s_tex[tid] = tid < 24 ? TT.t[tid] : awp_rcp(TT.t[tid - 8]);
+  __syncthreads();
+  const int b = awp_xcd_remap((int)blockIdx.x, L.nblocks);
+  int kt, jt, ic;
+  awp_tile3(b, L.nkt, L.njt, 0, kt, jt, ic);
+  const int lr = tid * L.tile.mul >> 20;  // row of this lane in the tile (awp_pick_tile)
+  const int K = AWP_ALIGN + kt * L.tile.width + (tid - lr * L.tile.width);  // array level
+  const int k = K - AWP_ALIGN;
+  const int j = G.bj + jt * L.tile.rows + lr;
+  if (lr >= L.tile.rows || k < 3 || k >= G.nz || j >= G.ej) return;
+  const int ib = G.bi + ic * L.ichunk;
+  const int ie = ib + L.ichunk < G.ei ? ib + L.ichunk : G.ei;
   const int sl = G.sl, yl = G.yl;
-  const int K = k + AWP_ALIGN;
   const float dcz = A.dcrjz[K];
   const float dcy = A.dcrjy[j];
-  for (int i = ib; i < ie; ++i) {
-    const int pos = yl * j + K + sl * i;
+  int pos = yl * j + K + sl * ib;
+  TopoMedium m0 = topo_medium<ST>(A, pos, yl);
+  for (int i = ib; i < ie; ++i, pos += sl) {
+    const TopoMedium m1 = topo_medium<ST>(A, pos + sl, yl);
     const float f_dcrj = A.dcrjx[i] * dcy * dcz;
-    float f_vx1, f_vx2, f_wwo;
+    float f_vx1, f_vx2, f_wwo, r_wwo;
     int f_ww;
     if (TEX == TOPO_TEX_ARRAYS) {
       f_vx1 = A.vx1[pos]; f_vx2 = A.vx2[pos]; f_wwo = A.wwo[pos];
       f_ww = A.ww[pos];
+      r_wwo = awp_rcp(f_wwo);
     } else {
       if (TEX == TOPO_TEX_TABLE) {
         f_ww = A.ww[pos];
@@ -1181,10 +1199,13 @@ __global__ __launch_bounds__(256) void topo_str_q_kernel(const TopoStrArgs<ST> A
       }
       const int t = (f_ww - 1) & 7;
       f_vx1 = s_tex[t]; f_vx2 = s_tex[8 + t]; f_wwo = s_tex[16 + t];
+      r_wwo = s_tex[24 + t];
     }
-    topo_str_update<ST>(A, pos, sl, yl, f_dcrj, R[pos], R[rstride + pos], R[2 * rstride + pos],
+    topo_str_update<ST>(A, pos, f_dcrj, m0, m1, R[pos], R[rstride + pos], R[2 * rstride + pos],
                         R[3 * rstride + pos], R[4 * rstride + pos], R[5 * rstride + pos],
-                        f_vx1, f_vx2, f_wwo, f_ww);
+                        f_vx1, f_vx2, f_wwo, r_wwo, s_coeff[(f_ww * 2 - 2) & 15],
+                        s_coeff[(f_ww * 2 - 1) & 15]);
+    m0 = m1;
   }
 }
 
@@ -1390,12 +1411,25 @@ void topo_tiles(int nz, VelTiles* V) {
   V->nint = V->wtop0 > 3 ? awp_cdiv(V->wtop0 - 3, V->step) : 0;
 }
 
-// Planes per march of a strain-rate launch: towards 16384 waves, 4 to 32
-// planes (a march re-reads and re-sums 3 columns at its start).
-int topo_chunk(int planes, int waves) {
-  if (awp_tuning().topo_rate_chunk > 0) return awp_tuning().topo_rate_chunk;
-  const long long c = (long long)planes * waves / 16384;
-  return c < 4 ? 4 : c > 32 ? 32 : (int)c;
+// Planes per march of a velocity or strain-rate launch whose planes take
+// `waves` waves each: 4 to `most`, the count that minimises rounds x (planes +
+// 3).  The card holds 4096 of these waves at a time (4 per SIMD: 108 to 127
+// VGPRs), a last round that is nearly empty takes as long as a full one, and a
+// march first loads and sums 3 planes for its windows.  At 131x97x85 the
+// velocity update takes 41 us with 6 planes (4268 waves), 31 with 8 (3298).
+int topo_chunk(int planes, int waves, int most, int forced) {
+  if (forced > 0) return forced;
+  int best = 4;
+  long long cost = 1ll << 62;
+  for (int c = 4; c <= most; ++c) {
+    const long long w = (long long)awp_cdiv(planes, c) * waves;
+    const long long x = (w + 4095) / 4096 * (c + 3);
+    if (x < cost) {
+      cost = x;
+      best = c;
+    }
+  }
+  return best;
 }
 
 template <class ST>
@@ -1441,23 +1475,15 @@ void topo_velocity_launch(topo_t* T, const WaveScales& W, const char* where) {
   G.bj = 0;
   G.ej = T->ny;
   hipStream_t st = T->stream_i;
-  // segments: interior ones every 58 levels from level 3, then the top one
-  // (levels nz-64 .. nz-1) writing from nz-61 (or 3) up
   VelTiles V;
-  V.ktop0 = T->nz - 64;
-  V.wtop0 = V.ktop0 + 3 > 3 ? V.ktop0 + 3 : 3;
-  V.nint = V.wtop0 > 3 ? awp_cdiv(V.wtop0 - 3, 58) : 0;
-  V.ichunk = awp_tuning().topo_vel_ichunk;
+  topo_tiles(T->nz, &V);
   V.wsync = awp_tuning().topo_wsync;
-  dim3 block(64, VT_BJ, 1);
-  dim3 grid(V.nint + 1, awp_cdiv(T->ny, VT_BJ), awp_cdiv(T->nx, V.ichunk));
-  if (awp_tuning().topo_vel_split) {
-    hipLaunchKernelGGL((topo_vel_kernel<ST, 1>), grid, block, 0, st, A, G, V);
-    hipLaunchKernelGGL((topo_vel_kernel<ST, 2>), grid, block, 0, st, A, G, V);
-    hipLaunchKernelGGL((topo_vel_kernel<ST, 3>), grid, block, 0, st, A, G, V);
-  } else {
-    hipLaunchKernelGGL((topo_vel_kernel<ST, 0>), grid, block, 0, st, A, G, V);
-  }
+  V.njt = awp_cdiv(T->ny, V.rj);
+  V.ichunk = topo_chunk(T->nx, (V.nint + 1) * T->ny * V.nseg, 8, awp_tuning().topo_vel_ichunk);
+  const dim3 block(64, V.nseg * V.rj, 1);
+  const dim3 grid((V.nint + 1) * V.njt * awp_cdiv(T->nx, V.ichunk));
+  const size_t lds = (size_t)2 * V.rj * VT_NL * (V.ch + 2 * VT_PAD) * sizeof(float);
+  hipLaunchKernelGGL((topo_vel_kernel<ST>), grid, block, lds, st, A, G, V);
   awp_check_launch(where);
 }
 
@@ -1547,30 +1573,30 @@ void topo_stress_launch(topo_t* T, const WaveScales& W, const char* where, float
   dim3 grid(V.nint + 1, awp_cdiv(G.ej - G.bj, V.rj), awp_cdiv(G.ei - G.bi, V.ichunk));
   const size_t lds = (size_t)2 * V.rj * ST_NC * V.ch * sizeof(float);
   if (!rates) {
-    hipLaunchKernelGGL((topo_str_kernel<ST, false>), grid, block, lds, st, A, G, V, nullptr,
-                       0ll);
+    hipLaunchKernelGGL((topo_str_kernel<ST>), grid, block, lds, st, A, G, V);
     awp_check_launch(where);
     return;
   }
   // two passes: strain rates into rates, then the material and memory-
   // variable update streaming them back
   const long long rstride = (long long)G.sl * (T->nx + 4 + AWP_NGSL2);
-  if (awp_tuning().topo_str_split) {
-    // one launch per march direction (topo_rates_kernel)
-    const int ni = G.ei - G.bi, nj = G.ej - G.bj;
-    const size_t rlds = (size_t)2 * V.rj * 3 * (V.ch + 2 * RC_PAD) * sizeof(float);
-    V.ichunk = topo_chunk(ni, (V.nint + 1) * nj * V.nseg);
-    const dim3 gi(V.nint + 1, awp_cdiv(nj, V.rj), awp_cdiv(ni, V.ichunk));
-    hipLaunchKernelGGL((topo_rates_kernel<ST, 0>), gi, block, rlds, st, A, G, V, rates, rstride);
-    V.ichunk = topo_chunk(nj, (V.nint + 1) * ni * V.nseg);
-    const dim3 gj(V.nint + 1, awp_cdiv(ni, V.rj), awp_cdiv(nj, V.ichunk));
-    hipLaunchKernelGGL((topo_rates_kernel<ST, 1>), gj, block, rlds, st, A, G, V, rates, rstride);
-  } else {
-    hipLaunchKernelGGL((topo_str_kernel<ST, true>), grid, block, lds, st, A, G, V, rates,
-                       rstride);
-  }
-  const int qchunk = awp_tuning().topo_q_ichunk;
-  dim3 gq(awp_cdiv(T->nz - 3, 64), awp_cdiv(G.ej - G.bj, 4), awp_cdiv(G.ei - G.bi, qchunk));
+  const int ni = G.ei - G.bi, nj = G.ej - G.bj;
+  const size_t rlds = (size_t)2 * V.rj * 3 * (V.ch + 2 * VT_PAD) * sizeof(float);
+  V.ichunk = topo_chunk(ni, (V.nint + 1) * nj * V.nseg, 24, awp_tuning().topo_rate_chunk);
+  const dim3 gi(V.nint + 1, awp_cdiv(nj, V.rj), awp_cdiv(ni, V.ichunk));
+  hipLaunchKernelGGL((topo_rates_kernel<ST, 0>), gi, block, rlds, st, A, G, V, rates, rstride);
+  V.ichunk = topo_chunk(nj, (V.nint + 1) * ni * V.nseg, 24, awp_tuning().topo_rate_chunk);
+  const dim3 gj(V.nint + 1, awp_cdiv(ni, V.rj), awp_cdiv(nj, V.ichunk));
+  hipLaunchKernelGGL((topo_rates_kernel<ST, 1>), gj, block, rlds, st, A, G, V, rates, rstride);
+  TopoQLaunch QL;
+  QL.tile = awp_pick_tile(T->nz, 0, awp_tuning().kw);
+  QL.nkt = QL.tile.nkt;
+  QL.njt = awp_cdiv(nj, QL.tile.rows);
+  int nic;
+  awp_split_march(ni, QL.nkt * QL.njt, QL.tile.waves, awp_tuning().topo_q_ichunk, 10240, &nic,
+                  &QL.ichunk);
+  QL.nblocks = QL.nkt * QL.njt * nic;
+  const dim3 gq(QL.nblocks), bq(64 * QL.tile.waves);
   TopoTex TT = {};
   if (texmode != TOPO_TEX_ARRAYS) {
     for (int m = 0; m < 24; ++m) TT.t[m] = tex[m];
@@ -1581,14 +1607,14 @@ void topo_stress_launch(topo_t* T, const WaveScales& W, const char* where, float
     TT.nzt = T->nz;
   }
   if (texmode == TOPO_TEX_RULE)
-    hipLaunchKernelGGL((topo_str_q_kernel<ST, TOPO_TEX_RULE>), gq, dim3(64, 4), 0, st, A, G,
-                       rates, rstride, qchunk, TT);
+    hipLaunchKernelGGL((topo_str_q_kernel<ST, TOPO_TEX_RULE>), gq, bq, 0, st, A, G,
+                       rates, rstride, QL, TT);
   else if (texmode == TOPO_TEX_TABLE)
-    hipLaunchKernelGGL((topo_str_q_kernel<ST, TOPO_TEX_TABLE>), gq, dim3(64, 4), 0, st, A, G,
-                       rates, rstride, qchunk, TT);
+    hipLaunchKernelGGL((topo_str_q_kernel<ST, TOPO_TEX_TABLE>), gq, bq, 0, st, A, G,
+                       rates, rstride, QL, TT);
   else
-    hipLaunchKernelGGL((topo_str_q_kernel<ST, TOPO_TEX_ARRAYS>), gq, dim3(64, 4), 0, st, A, G,
-                       rates, rstride, qchunk, TT);
+    hipLaunchKernelGGL((topo_str_q_kernel<ST, TOPO_TEX_ARRAYS>), gq, bq, 0, st, A, G,
+                       rates, rstride, QL, TT);
   awp_check_launch(where);
 }
 

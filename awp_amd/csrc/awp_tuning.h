@@ -10,17 +10,15 @@ struct AwpTuning {
   int str_ichunk;   // >0 forces the stress i-chunk length
   int xcd_remap;    // 1: XCD-aware tile order, 0: plain order
   int kalign;       // 1: start k tiles on a 32-float (128 B) line boundary
-  int topo_vel_ichunk;  // planes per march of the curvilinear velocity kernel
-  int topo_str_ichunk;  // same, curvilinear stress kernel
-  int topo_q_ichunk;    // planes per march of the two-pass stress update
+  int topo_vel_ichunk;  // planes per march of the curvilinear velocity kernel (0: topo_chunk)
+  int topo_str_ichunk;  // same, one-pass curvilinear stress kernel
+  int topo_q_ichunk;    // same, second pass of the two-pass update (0: awp_split_march)
   int step_ichunk;      // >0 forces the i-chunk length of the fused step (awp_step)
   int step_target_wgs;  // fused step: workgroups to aim for when splitting the i march
   int vel_jfast;        // 1: j tiles fastest in the block order (velocity)
   int str_jfast;        // same, stress
   int step_jfast;       // same, fused step
-  int topo_vel_split;   // 1: the curvilinear velocity update as one launch per component
   int adj_jgroup;       // adjoint kernels' block order: 0 plane by plane, else j tiles per group
-  int topo_str_split;   // strain-rate pass: 0 one launch, else one per march direction
   int kw;               // k-run width of the Cartesian kernels: 0 by the idle-lane rules, 32, 64
   int topo_nseg;        // curvilinear stress kernel: waves per k chunk at most (1: one-wave segments)
   int topo_wsync;       // curvilinear kernels: 1 wave-scope LDS sync where a wave reads only its own
