@@ -80,16 +80,31 @@ __global__ __launch_bounds__(256) void rescale_kernel(uint16_t* __restrict__ q, 
     q[i] = rescale1<ST>(q[i], shift);
 }
 
-// Largest |decoded value| (unit scale) into *out.  Both formats order
-// non-negative values as unsigned integers (NaN patterns above infinity), so
-// the pass takes the largest 15-bit magnitude pattern, decodes that one value,
-// and issues one vector atomic max per block on its binary32 bit pattern.
+// Largest |decoded value| (unit scale) of each of nf arrays of n values into
+// out[0 .. nf).  Both formats order non-negative values as unsigned integers
+// (NaN patterns above infinity), so the pass takes the largest 15-bit
+// magnitude pattern, decodes that one value, and issues one vector atomic max
+// per block on its binary32 bit pattern.  The atomics on one word follow each
+// other (about 10 ns each: 1024 blocks of four waves took 14.5 us on a
+// 3.9 M-value array that streams in 2), so a block is 16 waves and an array
+// gets at most 256 of them; the fields of a state share one launch
+// (blockIdx.y).
+constexpr int kAbsmaxThreads = 1024;
+struct AbsmaxFields {
+  const uint16_t* q[AWP_NSCALE];
+};
+
+__global__ __launch_bounds__(64) void absmax_clear_kernel(unsigned* __restrict__ out, int nf) {
+  if ((int)threadIdx.x < nf) out[threadIdx.x] = 0u;
+}
+
 template <class ST>
-__global__ __launch_bounds__(256) void absmax_kernel(const uint16_t* __restrict__ q,
-                                                     long long n, long long n8,
-                                                     unsigned* __restrict__ out) {
-  __shared__ unsigned red[4];
-  const long long stride = (long long)gridDim.x * 256;
+__global__ __launch_bounds__(kAbsmaxThreads) void absmax_kernel(const AbsmaxFields F, long long n,
+                                                                long long n8,
+                                                                unsigned* __restrict__ out) {
+  __shared__ unsigned red[kAbsmaxThreads / 64];
+  const uint16_t* __restrict__ q = F.q[blockIdx.y];
+  const long long stride = (long long)gridDim.x * kAbsmaxThreads;
   const uint4* q8 = reinterpret_cast<const uint4*>(q);
   unsigned m = 0u;
   auto fold = [&m](const uint4 v) {
@@ -102,7 +117,8 @@ __global__ __launch_bounds__(256) void absmax_kernel(const uint16_t* __restrict_
     }
   };
   // four independent 16-byte loads in flight per lane
-  long long i = blockIdx.x * 256ll + threadIdx.x;
+  const long long first = blockIdx.x * (long long)kAbsmaxThreads + threadIdx.x;
+  long long i = first;
   for (; i + 3 * stride < n8; i += 4 * stride) {
     const uint4 a = q8[i], b = q8[i + stride], c = q8[i + 2 * stride], d = q8[i + 3 * stride];
     fold(a);
@@ -111,7 +127,7 @@ __global__ __launch_bounds__(256) void absmax_kernel(const uint16_t* __restrict_
     fold(d);
   }
   for (; i < n8; i += stride) fold(q8[i]);
-  for (long long i = n8 * 8 + blockIdx.x * 256ll + threadIdx.x; i < n; i += stride) {
+  for (i = n8 * 8 + first; i < n; i += stride) {
     const unsigned b = q[i] & 0x7fffu;
     m = b > m ? b : m;
   }
@@ -124,16 +140,14 @@ __global__ __launch_bounds__(256) void absmax_kernel(const uint16_t* __restrict_
   __syncthreads();
   if (threadIdx.x == 0) {
     unsigned r = red[0];
-    for (int w = 1; w < 4; ++w) r = red[w] > r ? red[w] : r;
-    atomicMax(out, __float_as_uint(ST::dec((uint16_t)r, 1.0f)));
+    for (int w = 1; w < kAbsmaxThreads / 64; ++w) r = red[w] > r ? red[w] : r;
+    atomicMax(out + blockIdx.y, __float_as_uint(ST::dec((uint16_t)r, 1.0f)));
   }
 }
 
-// Blocks of the absmax pass: each block ends in one atomic on the same
-// word, so the grid stays at four blocks per CU (1024) and every lane loops.
 int absmax_grid(long long n) {
-  const long long b = (n / 8 + 255) / 256;
-  return (int)(b < 1024 ? (b < 1 ? 1 : b) : 1024);
+  const long long b = (n / 8 + 4 * kAbsmaxThreads - 1) / (4 * kAbsmaxThreads);
+  return (int)(b < 256 ? (b < 1 ? 1 : b) : 256);
 }
 
 long long vec8_count(const void* q, long long n) {
@@ -205,6 +219,39 @@ void awp_s16_rescale(uint16_t* q, long long n, int fmt, int shift, hipStream_t S
   awp_check_launch(W);
 }
 
+void awp_s16_absmax_fields(const uint16_t* const* q, int nf, long long n, int fmt, float* out,
+                           hipStream_t St) {
+  const char* W = "awp_s16_absmax_fields";
+  if (!fmt_ok(W, fmt)) return;
+  if (!q || !out || nf < 1 || nf > AWP_NSCALE) {
+    awp_set_error(AWP_ERR_ARG, "%s: q or out is NULL, or nf=%d outside [1, %d]", W, nf,
+                  (int)AWP_NSCALE);
+    return;
+  }
+  AbsmaxFields F = {};
+  bool vec = true;
+  for (int f = 0; f < nf; ++f) {
+    F.q[f] = q[f];
+    if (n > 0 && !q[f]) {
+      awp_set_error(AWP_ERR_ARG, "%s: array %d is NULL", W, f);
+      return;
+    }
+    vec = vec && ((uintptr_t)q[f] & 15u) == 0;
+  }
+  hipLaunchKernelGGL(absmax_clear_kernel, dim3(1), dim3(64), 0, St, (unsigned*)out, nf);
+  if (n > 0) {
+    const dim3 grid(absmax_grid(n), nf);
+    const long long n8 = vec ? n / 8 : 0;
+    if (fmt == AWP_FMT_BF16)
+      hipLaunchKernelGGL(absmax_kernel<StBF16>, grid, dim3(kAbsmaxThreads), 0, St, F, n, n8,
+                         (unsigned*)out);
+    else
+      hipLaunchKernelGGL(absmax_kernel<StF16>, grid, dim3(kAbsmaxThreads), 0, St, F, n, n8,
+                         (unsigned*)out);
+  }
+  awp_check_launch(W);
+}
+
 void awp_s16_absmax(const uint16_t* q, long long n, int fmt, float* out, hipStream_t St) {
   const char* W = "awp_s16_absmax";
   if (!fmt_ok(W, fmt)) return;
@@ -212,17 +259,10 @@ void awp_s16_absmax(const uint16_t* q, long long n, int fmt, float* out, hipStre
     awp_set_error(AWP_ERR_ARG, "%s: out is NULL", W);
     return;
   }
-  if (hipMemsetAsync(out, 0, sizeof(float), St) != hipSuccess) {
-    awp_set_error(AWP_ERR_HIP, "%s: hipMemsetAsync failed", W);
-    return;
-  }
-  if (n <= 0) return;
-  if (fmt == AWP_FMT_BF16)
-    hipLaunchKernelGGL(absmax_kernel<StBF16>, dim3(absmax_grid(n)), dim3(256), 0, St, q, n,
-                       vec8_count(q, n), (unsigned*)out);
+  if (n > 0)
+    awp_s16_absmax_fields(&q, 1, n, fmt, out, St);
   else
-    hipLaunchKernelGGL(absmax_kernel<StF16>, dim3(absmax_grid(n)), dim3(256), 0, St, q, n,
-                       vec8_count(q, n), (unsigned*)out);
+    hipLaunchKernelGGL(absmax_clear_kernel, dim3(1), dim3(64), 0, St, (unsigned*)out, 1);
   awp_check_launch(W);
 }
 

@@ -525,10 +525,9 @@ class Solver16(ScaledStorage, Solver):
 
     def _absmax_all(self) -> dict:
         L = self.levels[0]
-        n = L.dims.size
-        base = self._absbuf.data_ptr()
-        for idx, name in enumerate(FIELDS16):
-            self.lib.awp_s16_absmax(_ptr(L.f[name]), n, self.fmt, base + 4 * idx, self.stream)
+        q = (C.c_void_p * len(FIELDS16))(*[_ptr(L.f[name]) for name in FIELDS16])
+        self.lib.awp_s16_absmax_fields(q, len(FIELDS16), L.dims.size, self.fmt,
+                                       _ptr(self._absbuf), self.stream)
         _lib.check()
         vals = self._absbuf.cpu().numpy()
         return {name: float(vals[idx]) for idx, name in enumerate(FIELDS16)}

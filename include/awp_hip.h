@@ -287,6 +287,10 @@ void awp_s16_decode(const uint16_t* q, float* x, long long n, int fmt, float sca
                     hipStream_t St);
 void awp_s16_rescale(uint16_t* q, long long n, int fmt, int shift, hipStream_t St);
 void awp_s16_absmax(const uint16_t* q, long long n, int fmt, float* out, hipStream_t St);
+/* awp_s16_absmax of nf <= 15 arrays of n values each (q: a host array of
+ * device pointers) in one launch: out[f] for array f. */
+void awp_s16_absmax_fields(const uint16_t* const* q, int nf, long long n, int fmt, float* out,
+                           hipStream_t St);
 
 /* ---- Adjoint and material gradient (no reference counterpart) ----------
  * For callers that need dJ/d(lambda, mu, rho) of a receiver misfit through
