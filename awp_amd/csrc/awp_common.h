@@ -63,17 +63,6 @@ __device__ __forceinline__ int awp_xcd_remap(int b, int nblocks) {
 
 static inline int awp_cdiv(int a, int b) { return (a + b - 1) / b; }
 
-// k-run width of the plasticity kernels: a wave covers 64 consecutive k of
-// one j row, or 32 consecutive k of each of two j rows when that leaves at
-// least 16 fewer lanes idle per column of n levels (n = 96 fills 2 x 64
-// lanes to 75 % but 3 x 32 to 100 %).  forced: 32 or 64 from the tuning,
-// else 0 for this rule.
-static inline int awp_pick_kw(int n, int forced) {
-  if (forced == 32 || forced == 64) return forced;
-  const int idle64 = awp_cdiv(n, 64) * 64 - n, idle32 = awp_cdiv(n, 32) * 32 - n;
-  return idle64 - idle32 >= 16 ? 32 : 64;
-}
-
 // (k, j) tile of the marching Cartesian kernels: a workgroup of `waves` waves
 // covers `rows` j rows of `width` consecutive k each, lane t being row
 // t / width and level t % width, `nkt` tiles down a column of n levels.
@@ -97,6 +86,30 @@ static inline AwpTile awp_pick_tile(int n, int waves, int width) {
   t.waves = waves > 0 ? waves : row && width <= 0 ? awp_cdiv(n, 64) : 4;
   t.width = width > 0 ? width : row ? n : 64;
   if (t.width > 64 * t.waves) t.width = 64;
+  t.rows = 64 * t.waves / t.width;
+  t.nkt = awp_cdiv(n, t.width);
+  t.mul = ((1 << 20) + t.width - 1) / t.width;
+  return t;
+}
+
+// The tile of the plasticity kernels, which spend as many cycles on
+// arithmetic as on memory (binary64 sine, cosine and exponential): whole
+// columns (up to 256 levels, else equal parts) in the workgroup of 1 to 8
+// waves that leaves the fewest lanes idle, the smaller one among equals
+// (n = 48: 3 waves of 4 rows, all lanes; 64-level rows keep 75 %).
+static inline AwpTile awp_pick_full_tile(int n, int width) {
+  AwpTile t;
+  t.nkt = awp_cdiv(n, 256);
+  t.width = width > 0 ? width : awp_cdiv(n, t.nkt);
+  t.waves = 4;
+  float best = 0.0f;
+  for (int w = width > 0 ? 4 : 1; w <= (width > 0 ? 4 : 8); ++w) {
+    const float use = (float)(64 * w / t.width * t.width) / (float)(64 * w);
+    if (use > best + 0.001f) {
+      best = use;
+      t.waves = w;
+    }
+  }
   t.rows = 64 * t.waves / t.width;
   t.nkt = awp_cdiv(n, t.width);
   t.mul = ((1 << 20) + t.width - 1) / t.width;

@@ -4,7 +4,7 @@
 // stress rotated from the principal frame on the fly (rotate_principal,
 // :43-64).
 //
-// drprecpc_calc: wave64 along k, BJ waves along j, i-march with the plane
+// drprecpc_calc: lanes along k, i-march with the plane
 // (i+1) values of sigma2/xy/xz/mu and the rotated initial stress carried in
 // registers, so every per-cell array is fetched once and each plane's
 // initial stress is rotated once.  drprecpc_app only works where the
@@ -17,6 +17,7 @@
 #include <math.h>
 
 #include "awp_common.h"
+#include "awp_math.h"
 #include "awp_tuning.h"
 #include "../../include/awp_hip.h"
 
@@ -24,7 +25,7 @@ namespace {
 
 struct PlastLaunch {
   int k0, k1, j0, j1, i0, ni, ichunk, nkt, njt, nblocks, remap, srfpos, yline;
-  int kw;  // k-run width (awp_pick_kw)
+  AwpTile tile;
   long long slice;
   float DH, DT, Tv_fixed;
   float fmajor, fminor;
@@ -32,29 +33,20 @@ struct PlastLaunch {
 };
 
 // rotate_principal: ssp = RzT * diag((s2+pf)*fmajor, s2+pf, (s2+pf)*fminor) * Rz
-// - pf on the diagonal, with matmul3's accumulation order c = ((0+a0b0)+a1b1)+a2b2.
+// - pf on the diagonal, with matmul3's accumulation order c = (a0b0+a1b1)+a2b2.
+// The products with the diagonal matrix's zeros are left out: adding them
+// changes no value.
 __device__ __forceinline__ void rotate6(float sigma2, float pfluid, const PlastLaunch& L,
                                         float* o /* xx, yy, zz, xy, xz, yz */) {
-  float ss[9], tmp[9];
-#pragma unroll
-  for (int q = 0; q < 9; ++q) ss[q] = 0.0f;
-  ss[0] = (sigma2 + pfluid) * L.fmajor;
-  ss[4] = sigma2 + pfluid;
-  ss[8] = (sigma2 + pfluid) * L.fminor;
+  const float s = sigma2 + pfluid;
+  const float ss[3] = {s * L.fmajor, s, s * L.fminor};
+  float tmp[9];
 #pragma unroll
   for (int a = 0; a < 3; ++a)
 #pragma unroll
-    for (int b = 0; b < 3; ++b) {
-      float acc = 0.0f;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) acc += L.RzT[a * 3 + c] * ss[c * 3 + b];
-      tmp[a * 3 + b] = acc;
-    }
+    for (int c = 0; c < 3; ++c) tmp[a * 3 + c] = L.RzT[a * 3 + c] * ss[c];
   auto ent = [&](int a, int b) {
-    float acc = 0.0f;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) acc += tmp[a * 3 + c] * L.Rz[c * 3 + b];
-    return acc;
+    return tmp[a * 3] * L.Rz[b] + tmp[a * 3 + 1] * L.Rz[3 + b] + tmp[a * 3 + 2] * L.Rz[6 + b];
   };
   o[0] = ent(0, 0) - pfluid;
   o[1] = ent(1, 1) - pfluid;
@@ -70,8 +62,7 @@ __device__ __forceinline__ float pfluid_at(int srfpos, int k, float DH) {
   return (float)((double)DH / 2. * 9.81e3);
 }
 
-template <int BJ, int KW = 64>
-__global__ __launch_bounds__(64 * BJ) void drprecpc_calc_kernel(
+__global__ __launch_bounds__(512) void drprecpc_calc_kernel(
     const float* __restrict__ xx, const float* __restrict__ yy, const float* __restrict__ zz,
     const float* __restrict__ xy, const float* __restrict__ xz, const float* __restrict__ yz,
     const float* __restrict__ mu, const float* __restrict__ d1,
@@ -82,11 +73,11 @@ __global__ __launch_bounds__(64 * BJ) void drprecpc_calc_kernel(
   const int kt = b % L.nkt;
   const int jt = (b / L.nkt) % L.njt;
   const int ic = b / (L.nkt * L.njt);
-  // KW = 32: a wave covers 32 levels of each of two j rows
-  const int lane = (int)threadIdx.x;
-  const int k = L.k0 + kt * KW + (KW == 64 ? lane : lane % KW);
-  const int j = L.j0 + (jt * BJ + (int)threadIdx.y) * (64 / KW) + (KW == 64 ? 0 : lane / KW);
-  if (k > L.k1 || j > L.j1) return;
+  const int t = (int)threadIdx.x;
+  const int lr = t * L.tile.mul >> 20;  // row of this lane in the tile (awp_pick_full_tile)
+  const int k = L.k0 + kt * L.tile.width + (t - lr * L.tile.width);
+  const int j = L.j0 + jt * L.tile.rows + lr;
+  if (lr >= L.tile.rows || k > L.k1 || j > L.j1) return;
   const int ia = L.i0 + ic * L.ichunk;
   int nsteps = L.ni - ic * L.ichunk;
   if (nsteps > L.ichunk) nsteps = L.ichunk;
@@ -124,22 +115,23 @@ __global__ __launch_bounds__(64 * BJ) void drprecpc_calc_kernel(
     float Sxz = 0.25f * (xzc + xzn + xzkm + xznkm) + 0.5f * (ini[4] + inn[4]);
     float Syz = 0.25f * (yz[p] + yz[p - Y] + yz[p - 1] + yz[p - Y - 1]) + 0.5f * (ini[5] + inn[5]);
     float Sxy = 0.25f * (xyc + xyn + xyjm + xynjm) + 0.5f * (ini[3] + inn[3]);
-    float Tv = DH / sqrtf(1.0f / (muc * d1[p]));
-    if (L.Tv_fixed > 0.0f) Tv = L.Tv_fixed;
+    float Tv = L.Tv_fixed;
+    if (!(Tv > 0.0f)) Tv = DH / sqrtf(1.0f / (muc * d1[p]));  // uniform: d1 is not read otherwise
     const float Sxxp = Sxx, Syyp = Syy, Szzp = Szz, Sxyp = Sxy, Sxzp = Sxz, Syzp = Syz;
     const float rphi = phi[p] * 0.017453292519943295f;
-    const float sigma_m = (Sxx + Syy + Szz) / 3.0f;
+    const float sigma_m = awp_div_by(Sxx + Syy + Szz, 3.0f, (float)(1.0 / 3.0));
     const float SDxx = Sxx - sigma_m, SDyy = Syy - sigma_m, SDzz = Szz - sigma_m;
     const float secinv =
         0.5f * (SDxx * SDxx + SDyy * SDyy + SDzz * SDzz) + Sxz * Sxz + Sxy * Sxy + Syz * Syz;
     const float sqrtSecinv = sqrtf(secinv);
-    const float taulim2 = cohes[p] * (float)cos((double)rphi) -
-                          (sigma_m + pfluid) * (float)sin((double)rphi);
+    double sphi, cphi;
+    sincos((double)rphi, &sphi, &cphi);  // one argument reduction for both
+    const float taulim2 = cohes[p] * (float)cphi - (sigma_m + pfluid) * (float)sphi;
     const float taulim = taulim2 > 0.0f ? taulim2 : 0.0f;
     float iyldfac;
     if (sqrtSecinv > taulim) {
-      iyldfac = taulim / sqrtSecinv +
-                (1.0f - taulim / sqrtSecinv) * (float)exp((double)(-DT / Tv));
+      const float ratio = awp_div(taulim, sqrtSecinv);
+      iyldfac = ratio + (1.0f - ratio) * (float)exp((double)(-DT / Tv));
       Sxx = SDxx * iyldfac + sigma_m;
       Syy = SDyy * iyldfac + sigma_m;
       Szz = SDzz * iyldfac + sigma_m;
@@ -151,9 +143,12 @@ __global__ __launch_bounds__(64 * BJ) void drprecpc_calc_kernel(
     }
     if (iyldfac < 1.0f) {
       yldfac[p] = iyldfac;
-      const float xm = 2.0f / (muc + mun);
-      const float dxx = (Sxx - Sxxp) / xm, dyy = (Syy - Syyp) / xm, dzz = (Szz - Szzp) / xm;
-      const float dxy = (Sxy - Sxyp) / xm, dxz = (Sxz - Sxzp) / xm, dyz = (Syz - Syzp) / xm;
+      const float xm = awp_pow2_div(2.0f, muc + mun);
+      const float ym = awp_rcp(xm);
+      const float dxx = awp_div_by(Sxx - Sxxp, xm, ym), dyy = awp_div_by(Syy - Syyp, xm, ym),
+                  dzz = awp_div_by(Szz - Szzp, xm, ym);
+      const float dxy = awp_div_by(Sxy - Sxyp, xm, ym), dxz = awp_div_by(Sxz - Sxzp, xm, ym),
+                  dyz = awp_div_by(Syz - Syzp, xm, ym);
       neta[p] = neta[p] + sqrtf(0.5f * (dxx * dxx + dyy * dyy + dzz * dzz) +
                                 2.0f * (dxy * dxy + dxz * dxz + dyz * dyz));
     } else {
@@ -169,8 +164,7 @@ __global__ __launch_bounds__(64 * BJ) void drprecpc_calc_kernel(
   }
 }
 
-template <int BJ, int KW = 64>
-__global__ __launch_bounds__(64 * BJ) void drprecpc_app_kernel(
+__global__ __launch_bounds__(512) void drprecpc_app_kernel(
     float* __restrict__ xx, float* __restrict__ yy, float* __restrict__ zz,
     float* __restrict__ xy, float* __restrict__ xz, float* __restrict__ yz,
     const float* __restrict__ sigma2, const float* __restrict__ yldfac, const PlastLaunch L) {
@@ -178,11 +172,11 @@ __global__ __launch_bounds__(64 * BJ) void drprecpc_app_kernel(
   const int kt = b % L.nkt;
   const int jt = (b / L.nkt) % L.njt;
   const int ic = b / (L.nkt * L.njt);
-  // KW = 32: a wave covers 32 levels of each of two j rows
-  const int lane = (int)threadIdx.x;
-  const int k = L.k0 + kt * KW + (KW == 64 ? lane : lane % KW);
-  const int j = L.j0 + (jt * BJ + (int)threadIdx.y) * (64 / KW) + (KW == 64 ? 0 : lane / KW);
-  if (k > L.k1 || j > L.j1) return;
+  const int t = (int)threadIdx.x;
+  const int lr = t * L.tile.mul >> 20;  // row of this lane in the tile (awp_pick_full_tile)
+  const int k = L.k0 + kt * L.tile.width + (t - lr * L.tile.width);
+  const int j = L.j0 + jt * L.tile.rows + lr;
+  if (lr >= L.tile.rows || k > L.k1 || j > L.j1) return;
   const int ia = L.i0 + ic * L.ichunk;
   int nsteps = L.ni - ic * L.ichunk;
   if (nsteps > L.ichunk) nsteps = L.ichunk;
@@ -247,7 +241,7 @@ __global__ __launch_bounds__(64 * BJ) void drprecpc_app_kernel(
 }
 
 bool plast_setup(const char* W, int nzt, int xls, int xre, int yls, int yre, int d_i,
-                 float Tv_fixed, bool app, PlastLaunch& L) {
+                 float Tv_fixed, PlastLaunch& L) {
   if (!awp_grid_ok(d_i, W)) return false;
   const AwpGrid& g = awp_state().grid[d_i];
   if (nzt != g.nzt) {
@@ -282,11 +276,11 @@ bool plast_setup(const char* W, int nzt, int xls, int xre, int yls, int yre, int
     L.RzT[q] = pc.RzT[q];
   }
   L.remap = awp_tuning().xcd_remap;
-  L.kw = awp_pick_kw(L.k1 - L.k0 + 1, awp_tuning().kw);
-  L.nkt = awp_cdiv(L.k1 - L.k0 + 1, L.kw);
-  L.njt = awp_cdiv(L.j1 - L.j0 + 1, 4 * (64 / L.kw));
+  L.tile = awp_pick_full_tile(L.k1 - L.k0 + 1, awp_tuning().kw);
+  L.nkt = L.tile.nkt;
+  L.njt = awp_cdiv(L.j1 - L.j0 + 1, L.tile.rows);
   int nic, ichunk;
-  awp_split_i(L.ni, L.nkt * L.njt, 0, app ? 4096 : 2048, &nic, &ichunk);
+  awp_split_march(L.ni, L.nkt * L.njt, L.tile.waves, 0, 10240, &nic, &ichunk);
   L.ichunk = ichunk;
   L.nblocks = L.nkt * L.njt * nic;
   return true;
@@ -297,13 +291,9 @@ void calc_common(const char* W, float* xx, float* yy, float* zz, float* xy, floa
                  float* phi, float* neta, int nzt, int xls, int xre, int yls, int yre,
                  hipStream_t St, int d_i, float Tv) {
   PlastLaunch L;
-  if (!plast_setup(W, nzt, xls, xre, yls, yre, d_i, Tv, false, L)) return;
-  if (L.kw == 32)
-    hipLaunchKernelGGL((drprecpc_calc_kernel<4, 32>), dim3(L.nblocks), dim3(64, 4), 0, St, xx, yy,
-                       zz, xy, xz, yz, mu, d1, sigma2, yldfac, cohes, phi, neta, L);
-  else
-    hipLaunchKernelGGL((drprecpc_calc_kernel<4, 64>), dim3(L.nblocks), dim3(64, 4), 0, St, xx, yy,
-                       zz, xy, xz, yz, mu, d1, sigma2, yldfac, cohes, phi, neta, L);
+  if (!plast_setup(W, nzt, xls, xre, yls, yre, d_i, Tv, L)) return;
+  hipLaunchKernelGGL(drprecpc_calc_kernel, dim3(L.nblocks), dim3(64 * L.tile.waves), 0, St, xx, yy,
+                     zz, xy, xz, yz, mu, d1, sigma2, yldfac, cohes, phi, neta, L);
   awp_check_launch(W);
 }
 
@@ -337,13 +327,9 @@ void drprecpc_app_H(float* xx, float* yy, float* zz, float* xy, float* xz, float
   (void)mu;  // read by the reference only for a value it never uses (kernel.cu:1744-1772)
   const char* W = "drprecpc_app_H";
   PlastLaunch L;
-  if (!plast_setup(W, nzt, xls, xre, yls, yre, d_i, 0.0f, true, L)) return;
-  if (L.kw == 32)
-    hipLaunchKernelGGL((drprecpc_app_kernel<4, 32>), dim3(L.nblocks), dim3(64, 4), 0, St, xx, yy,
-                       zz, xy, xz, yz, sigma2, yldfac, L);
-  else
-    hipLaunchKernelGGL((drprecpc_app_kernel<4, 64>), dim3(L.nblocks), dim3(64, 4), 0, St, xx, yy,
-                       zz, xy, xz, yz, sigma2, yldfac, L);
+  if (!plast_setup(W, nzt, xls, xre, yls, yre, d_i, 0.0f, L)) return;
+  hipLaunchKernelGGL(drprecpc_app_kernel, dim3(L.nblocks), dim3(64 * L.tile.waves), 0, St, xx, yy,
+                     zz, xy, xz, yz, sigma2, yldfac, L);
   awp_check_launch(W);
 }
 
