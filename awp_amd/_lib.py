@@ -61,6 +61,8 @@ SIGNATURES: dict[str, list] = {
     "awp_adjoint_settle": [_fp, _fp, _s],
     "awp_adjoint_inject": [_fp] * 4 + [_i, _fp, _s],
     "awp_adjoint_flush": [_fp, _fp, C.c_longlong, _s],
+    "awp_adjoint_flush_grid": [_fp] * 4 + [_s],
+    "awp_move_fields": [_fp, _fp, _i, C.c_longlong, _s],
     "awp_misfit": [_fp, _fp, C.c_longlong, _fp, _fp, _fp, _s],
     "awp_misfit_noalloc": [_fp, _fp, C.c_longlong, _fp, _fp, _s],
     "awp_adjoint_map": [_fp] * 11 + [_s],

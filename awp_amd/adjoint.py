@@ -36,6 +36,15 @@ def _pp(ts):
     return (C.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
 
 
+def _move(lib, stream, dst, src=None) -> None:
+    """dst[n] = src[n] (0 without src) for contiguous tensors of one size, a
+    launch for every AWP_MOVE_FIELDS of them."""
+    for a in range(0, len(dst), 16):
+        d = dst[a:a + 16]
+        lib.awp_move_fields(_pp(d), _pp(src[a:a + 16]) if src else None, len(d),
+                            d[0].numel() * d[0].element_size(), stream)
+
+
 class AdjointProblem:
     """One grid, NVE = 1: forward with checkpoints, misfit, adjoint sweep."""
 
@@ -134,14 +143,14 @@ class AdjointProblem:
     # -- forward --
     def _reset(self) -> None:
         s = self.solver
-        for t in s.f.values():
-            t.zero_()
+        _move(self.lib, s.stream, list(s.f.values()))
         s.rec["out"].zero_()
         s.cur_step = 0
 
     def _save(self, n: int) -> None:
-        f = self.solver.f
-        self.checkpoints[n] = [f[x].clone() for x in FIELDS]
+        f = [self.solver.f[x] for x in FIELDS]
+        self.checkpoints[n] = [torch.empty_like(t) for t in f]
+        _move(self.lib, self.solver.stream, self.checkpoints[n], f)
 
     def forward(self) -> float:
         """Checkpointed forward run and the misfit (binary64)."""
@@ -161,8 +170,8 @@ class AdjointProblem:
             # from it
             if self.n_tail > 0:
                 s.step()
-            for x in VEL + STRESS:
-                self.slots[0][x].copy_(s.f[x])
+            _move(self.lib, s.stream, [self.slots[0][x] for x in VEL + STRESS],
+                  [s.f[x] for x in VEL + STRESS])
             rec = s.rec
             for n in range(self.n_tail + 1, self.nt + 1):
                 fout = self.slots[n - self.n_tail]
@@ -220,15 +229,15 @@ class AdjointProblem:
         s = self.solver
         lib = self.lib
         st = s.stream
-        for t in list(self.adj.values()) + self.scratch + self.g32 + self.g64:
-            t.zero_()
+        _move(lib, st, list(self.adj.values()) + self.scratch + self.g32)
+        _move(lib, st, self.g64)
         self.gl32.zero_()
         self.gl64.zero_()
         med = self._pointers()
         m = s.m
         adj = _pp([self.adj[n] for n in ADJ_ORDER])
         scratch = _pp(self.scratch)
-        g32 = _pp(self.g32)
+        g32, g64 = _pp(self.g32), _pp(self.g64)
         rec = s.rec
         npts = rec["n"]
         starts = sorted(set(self.checkpoints) |
@@ -241,8 +250,8 @@ class AdjointProblem:
             else:
                 # recompute the segment from its checkpoint into the ring
                 ring = self.ring
-                for x, t in zip(FIELDS, self.checkpoints[n0]):
-                    (ring[0][x] if x in ring[0] else s.f[x]).copy_(t)
+                _move(lib, st, [ring[0][x] if x in ring[0] else s.f[x] for x in FIELDS],
+                      self.checkpoints[n0])
                 s.cur_step = n0
                 for n in range(n0 + 1, n1 + 1):
                     self._recompute_step(ring[n - 1 - n0], ring[n - n0])
@@ -257,16 +266,15 @@ class AdjointProblem:
                                      m["dcrjx"].data_ptr(), m["dcrjy"].data_ptr(),
                                      m["dcrjz"].data_ptr(), scratch, g32,
                                      self.gl32.data_ptr(), self.col.data_ptr(), st)
-            for a, b in zip(self.g32, self.g64):
-                lib.awp_adjoint_flush(a.data_ptr(), b.data_ptr(), a.numel(), st)
-            lib.awp_adjoint_flush(self.gl32.data_ptr(), self.gl64.data_ptr(), self.gl32.numel(), st)
+            lib.awp_adjoint_flush_grid(g32, g64, self.gl32.data_ptr(), self.gl64.data_ptr(), st)
             _lib.check()
         # the adjoint state at step 0 complete (the last step's pending gather)
         lib.awp_adjoint_settle(adj, scratch, st)
         sh = self.dims.shape
         f64 = dict(dtype=torch.float64, device=self.dev)
-        glam, gmu, grho = (torch.zeros(sh, **f64) for _ in range(3))
-        lib.awp_adjoint_map(_pp(self.g64), self.gl64.data_ptr(), med, m["ww"].data_ptr(),
+        # every cell of the padded grid is written
+        glam, gmu, grho = (torch.empty(sh, **f64) for _ in range(3))
+        lib.awp_adjoint_map(g64, self.gl64.data_ptr(), med, m["ww"].data_ptr(),
                             m["coeff"].data_ptr(), m["dcrjx"].data_ptr(), m["dcrjy"].data_ptr(),
                             m["dcrjz"].data_ptr(), glam.data_ptr(), gmu.data_ptr(),
                             grho.data_ptr(), st)

@@ -18,6 +18,7 @@
 #include <mutex>
 
 #include "awp_common.h"
+#include "awp_math.h"
 #include "awp_tuning.h"
 #include "../../include/awp_hip.h"
 
@@ -41,10 +42,8 @@ struct AdjGrid {
 struct Blk3 {
   int x, y, z;
 };
-__device__ __forceinline__ Blk3 adj_block(const AdjGrid& G) {
-  const int nx = (int)gridDim.x, ny = (int)gridDim.y, nz = (int)gridDim.z;
-  const int nb = nx * ny * nz;
-  int b = awp_xcd_remap((int)(blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z)), nb);
+__device__ __forceinline__ Blk3 adj_block(const AdjGrid& G, int nx, int ny, int nz, int b) {
+  b = awp_xcd_remap(b, nx * ny * nz);
   if (G.jgroup <= 0 || G.jgroup >= ny) return Blk3{b % nx, (b / nx) % ny, b / (nx * ny)};
   const int x = b % nx;
   b /= nx;  // (j group, i, j tile in group), j tile fastest
@@ -61,6 +60,11 @@ __device__ __forceinline__ Blk3 adj_block(const AdjGrid& G) {
   }
   return Blk3{x, y0 + b % jg, b / jg};
 }
+__device__ __forceinline__ Blk3 adj_block(const AdjGrid& G) {
+  const int nx = (int)gridDim.x, ny = (int)gridDim.y;
+  return adj_block(G, nx, ny, (int)gridDim.z,
+                   (int)(blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z)));
+}
 
 __device__ __forceinline__ long long aidx(const AdjGrid& G, int i, int j, int k) {
   return (long long)i * G.slice + (long long)j * G.yline + k;
@@ -70,13 +74,12 @@ __device__ __forceinline__ long long aidx(const AdjGrid& G, int i, int j, int k)
 // interior columns: the band is a few levels deep, so the 256 lanes of a
 // block take nk = k1-k0+1 consecutive levels of 256/nk consecutive columns
 // (k fastest, then j) of one i plane, instead of one column per wave with
-// nk of its 64 lanes active.  Grid: (cdiv(nk * ny, 256), 1, nx).
+// nk of its 64 lanes active.  Blocks: (cdiv(nk * ny, 256), 1, nx).
 struct BandCell {
   int i, j, k;
   bool ok;
 };
-__device__ __forceinline__ BandCell band_cell(const AdjGrid& G, int k0, int k1) {
-  const Blk3 B = adj_block(G);
+__device__ __forceinline__ BandCell band_cell(const AdjGrid& G, int k0, int k1, const Blk3& B) {
   const int nk = k1 - k0 + 1;
   const int t = B.x * 256 + (int)(threadIdx.y * 64 + threadIdx.x);
   BandCell c;
@@ -87,19 +90,10 @@ __device__ __forceinline__ BandCell band_cell(const AdjGrid& G, int k0, int k1) 
   return c;
 }
 
-// Production Q weight (as the forward dstrqc).
-__device__ __forceinline__ float adj_qw(float q, float ca, float cb, float wwo) {
-  float w;
-  if (1. / ((double)q * 2.0) <= 200.0)
-    w = (float)((double)ca * (2. * (double)q) * (2. * (double)q) + (double)cb * (2. * (double)q));
-  else
-    w = 2.0f * wwo * q;
-  return w / wwo;
-}
-
 // fstr^T: the imaging copies move adjoint values from above the surface back
 // to the levels they were copied from; the zeroed and overwritten cells lose
-// their adjoint.
+// their adjoint.  A launch of its own only where the levels top-2 .. top are
+// not all in adj_stress_local_kernel's range, which does this otherwise.
 __global__ __launch_bounds__(256) void adj_fstr_kernel(float* __restrict__ zz,
                                                        float* __restrict__ xz,
                                                        float* __restrict__ yz, const AdjGrid G) {
@@ -166,10 +160,14 @@ __device__ __forceinline__ void vel_gather6(const CPtr6& Aw, long long q, const 
 // the normal strains, E4..E6 for the shear pairs) and the coefficient
 // gradients (strains of the forward velocity after the step).
 // Below the free-surface band (k <= top-3) the previous step's pending
-// velocity^T gather (weights Awp) is added to the stress adjoints first.
+// velocity^T gather (weights Awp) is added to the stress adjoints first; on
+// the three levels above it (fstr) fstr^T of the lane's cell: every level
+// above the surface is read by one lane, which clears it, so no lane waits for
+// another and the column's transpose costs no launch (6.4 us at 96x96x64).
+// Bound by memory: 216 B/cell and the neighbours from L2; 96x96x64 in 33.7 us.
 __global__ __launch_bounds__(256) void adj_stress_local_kernel(Adj15 A, Ptr6 Es, CPtr3 V,
                                                                Medium M, Grad8 Gr,
-                                                               const AdjGrid G, CPtr6 Awp) {
+                                                               const AdjGrid G, CPtr6 Awp, bool fstr) {
   // the Q coefficients by mechanism, from LDS (the lookup by ww would
   // otherwise be a second dependent round trip to memory)
   __shared__ float s_coeff[16];
@@ -237,12 +235,37 @@ __global__ __launch_bounds__(256) void adj_stress_local_kernel(Adj15 A, Ptr6 Es,
     aw_im = Aw_[p - S]; aw_i2m = Aw_[p - 2 * S]; aw_ip = Aw_[p + S];
     aw_jp = Aw_[p + Y]; aw_jm = Aw_[p - Y]; aw_j2 = Aw_[p + 2 * Y];
   }
+  // fstr^T: the values above the surface that this level receives.  zz: top
+  // from top+1, top-1 from top+2; xz, yz: top-1 from top+1, top-2 from top+2.
+  const int fd = fstr ? G.top - k : 3;  // levels below the surface
+  const long long fz = p + (fd == 0 ? 1 : 3), fs = p + (fd == 1 ? 2 : 4);
+  float up_zz = 0.f, up_xz = 0.f, up_yz = 0.f;
+  if (fd < 2) up_zz = A.f[2][fz];
+  if (fd == 1 || fd == 2) {
+    up_xz = A.f[4][fs];
+    up_yz = A.f[5][fs];
+  }
   float gold[5];
 #pragma unroll
   for (int c = 0; c < 5; ++c) gold[c] = Gr.f[3 + c][p];
   __builtin_amdgcn_sched_barrier(0);
 
   const float c1 = G.c1, c2 = G.c2;
+  if (fd < 3) {
+    if (fd < 2) {
+      sbl[2] -= up_zz;
+      A.f[2][fz] = 0.0f;
+    }
+    if (fd > 0) {
+      sbl[4] -= up_xz;
+      sbl[5] -= up_yz;
+      A.f[4][fs] = 0.0f;
+      A.f[5][fs] = 0.0f;
+    } else {
+      sbl[4] = 0.0f;
+      sbl[5] = 0.0f;
+    }
+  }
   if (has_pend) {
     // vel_gather6's sums, term for term
     pend[0] = c1 * (au0 - au_is) + c2 * (au_im - au_i2);
@@ -261,16 +284,17 @@ __global__ __launch_bounds__(256) void adj_stress_local_kernel(Adj15 A, Ptr6 Es,
   const float sm8 = m0 + m1 + m2 + m3 + m4 + m5 + m6 + m7;
   const float sp8 = p0 + p1 + p2 + p3 + p4 + p5 + p6 + p7;
   const float ss8 = q0 + q1 + q2 + q3 + q4 + q5 + q6 + q7;
-  const float xm = awp_quot(16.0f, sm8);
-  const float xl = awp_quot(8.0f, sl8) + xm;
-  const float xmu1 = awp_quot(2.0f, m0 + m4);
-  const float xmu2 = awp_quot(2.0f, m0 + m2);
-  const float xmu3 = awp_quot(2.0f, m0 + m1);
-  const float qpaw = adj_qw(0.0625f * sp8, ca, cb, f_wwo);
-  const float hw = adj_qw(0.0625f * ss8, ca, cb, f_wwo);
-  const float h1w = adj_qw(0.250f * (q0 + q4), ca, cb, f_wwo);
-  const float h2w = adj_qw(0.250f * (q0 + q2), ca, cb, f_wwo);
-  const float h3w = adj_qw(0.250f * (q0 + q1), ca, cb, f_wwo);
+  const float xm = awp_pow2_div(16.0f, sm8);
+  const float xl = awp_pow2_div(8.0f, sl8) + xm;
+  const float xmu1 = awp_pow2_div(2.0f, m0 + m4);
+  const float xmu2 = awp_pow2_div(2.0f, m0 + m2);
+  const float xmu3 = awp_pow2_div(2.0f, m0 + m1);
+  const float rw = awp_rcp(f_wwo);
+  const float qpaw = awp_qw_prod(0.0625f * sp8, ca, cb, f_wwo, rw);
+  const float hw = awp_qw_prod(0.0625f * ss8, ca, cb, f_wwo, rw);
+  const float h1w = awp_qw_prod(0.250f * (q0 + q4), ca, cb, f_wwo, rw);
+  const float h2w = awp_qw_prod(0.250f * (q0 + q2), ca, cb, f_wwo, rw);
+  const float h3w = awp_qw_prod(0.250f * (q0 + q1), ca, cb, f_wwo, rw);
   const float dth = G.dth, dh1 = G.dh1, DT = G.DT;
   // coefficients per unit of xl, xm, xmu_k (the step is linear in them)
   const float qf = -qpaw * dh1 * f_vx1;            // qpa = xl * qf
@@ -358,15 +382,11 @@ __device__ __forceinline__ Vec3 strain_gather(const CPtr6& E, long long c, long 
 
 // ghost^T, part 1 (column (i, j)): the adjoints of ug, vg and of the bracket
 // of the w ghost, and the lam_mu gradient, from the ghost-level adjoints
-// ubg, vbg, wbg (ub, vb, wb at top+1).
-__device__ __forceinline__ void ghost1_column(int i, int j, float ubg, float vbg, float wbg,
-                                              const CPtr3& V,
-                                              const float* __restrict__ lam_mu,
-                                              float* __restrict__ col,
-                                              float* __restrict__ glm, const AdjGrid& G) {
+// ubg, vbg, wbg (ub, vb, wb at top+1).  Bk, the bracket itself, needs only the
+// forward velocities, so that its loads need not wait for the adjoints.
+__device__ __forceinline__ float ghost1_bracket(int i, int j, const CPtr3& V, const AdjGrid& G) {
   const long long S = G.slice, Y = G.yline;
   const long long p = aidx(G, i, j, G.top);
-  const long long q2 = (long long)i * G.lam_mu_ld + j;
   const float* u = V.f[0];
   const float* v = V.f[1];
   const float* w = V.f[2];
@@ -375,168 +395,187 @@ __device__ __forceinline__ void ghost1_column(int i, int j, float ubg, float vbg
   const float vg = v[p] - (w[p + Y] - w[p]);
   const float vs1 = cx ? u[p + S] - (w[p + S] - w[p]) : 0.0f;
   const float vs2 = cy ? v[p - Y] - (w[p] - w[p - Y]) : 0.0f;
-  const float Bk = (vs1 - ug) + (u[p + S] - u[p]) + (vg - vs2) + (v[p] - v[p - Y]);
-  const float wgb = wbg;
-  const float s = -lam_mu[q2] * wgb;
-  glm[q2] += -wgb * Bk;
+  return (vs1 - ug) + (u[p + S] - u[p]) + (vg - vs2) + (v[p] - v[p - Y]);
+}
+__device__ __forceinline__ void ghost1_column(int i, int j, float ubg, float vbg, float wbg,
+                                              float Bk, float lm, float gl,
+                                              float* __restrict__ col,
+                                              float* __restrict__ glm, const AdjGrid& G) {
+  const long long q2 = (long long)i * G.lam_mu_ld + j;
+  const float s = -lm * wbg;
+  glm[q2] = gl + -wbg * Bk;
   const long long n2 = (long long)(G.nx + 4 + AWP_NGSL2) * G.lam_mu_ld;
   col[q2] = ubg - s;       // adjoint of ug
   col[n2 + q2] = vbg + s;  // adjoint of vg
   col[2 * n2 + q2] = s;    // adjoint of the bracket
 }
 
-// ghost^T, part 2 (column (i, j)): gather the ghost adjoints onto the cells
-// the ghosts were computed from, then clear the ghost adjoints.  The w
-// ghost's own term, wb[top-1] += wb[top+1], is left to the caller (the lane
-// of level top-1).
-__device__ __forceinline__ void ghost2_column(int i, int j, float* __restrict__ ub,
-                                              float* __restrict__ vb, float* __restrict__ wb,
-                                              const float* __restrict__ col,
-                                              const AdjGrid& G) {
-  const long long p = aidx(G, i, j, G.top);
+// ghost^T, part 2 (column (i, j)): the increments of the velocity adjoints at
+// level top, gathered from the columns whose ghosts were computed from it.
+// The w ghost's own term, wb[top-1] += wb[top+1], and the clearing of the
+// ghost level are left to the caller.
+__device__ __forceinline__ void ghost2_column(int i, int j, const float* __restrict__ col,
+                                              const AdjGrid& G, float& du, float& dv, float& dw) {
   const int L = G.lam_mu_ld;
   const long long n2 = (long long)(G.nx + 4 + AWP_NGSL2) * L;
   const int i0 = 2 + AWP_NGSL, i1 = G.nx + 1 + AWP_NGSL, j0 = 2 + AWP_NGSL, j1 = G.ny + 1 + AWP_NGSL;
-  auto AU = [&](int ii, int jj) { return col[(long long)ii * L + jj]; };
-  auto AV = [&](int ii, int jj) { return col[n2 + (long long)ii * L + jj]; };
-  auto SB = [&](int ii, int jj) { return col[2 * n2 + (long long)ii * L + jj]; };
+  const long long c = (long long)i * L + j;
+  const float *AU = col, *AV = col + n2, *SB = col + 2 * n2;
+  // all loads at once (the neighbours of an edge column are in the array, but
+  // hold nothing: their values are not used)
+  const float au = AU[c], av = AV[c], s = SB[c];
+  const float sl = SB[c - L], sf = SB[c + 1], aur = AU[c + L], avp = AV[c - 1];
   auto CX = [&](int ii) { return (ii - AWP_NGSL - 1) < G.nx; };
   auto CY = [&](int jj) { return (jj - AWP_NGSL - 1) > 1; };
-  const float s = SB(i, j);
-  float du = AU(i, j) - s;
-  float dv = AV(i, j) + s;
-  float dw = -AU(i, j) + AV(i, j) + (CX(i) ? s : 0.0f) + (CY(j) ? s : 0.0f);
+  du = au - s;
+  dv = av + s;
+  dw = -au + av + (CX(i) ? s : 0.0f) + (CY(j) ? s : 0.0f);
   if (i - 1 >= i0) {
-    const float sl = SB(i - 1, j);
     du += sl + (CX(i - 1) ? sl : 0.0f);   // u[top+x] of the left column
     dw += CX(i - 1) ? -sl : 0.0f;         // w[top+x] in its vs1
   }
   if (j + 1 <= j1) {
-    const float sf = SB(i, j + 1);
     dv += -sf + (CY(j + 1) ? -sf : 0.0f);  // v[top-y] of the next column
     dw += CY(j + 1) ? -sf : 0.0f;          // w[top-y] in its vs2
     dw += 0.0f;
   }
-  if (i + 1 <= i1) dw += AU(i + 1, j);     // w[top-x] of the right column's ug
-  if (j - 1 >= j0) dw += -AV(i, j - 1);    // w[top+y] of the previous column's vg
-  ub[p] += du;
-  vb[p] += dv;
-  wb[p] += dw;
-  ub[p + 1] = 0.0f;
-  vb[p + 1] = 0.0f;
-  wb[p + 1] = 0.0f;
+  if (i + 1 <= i1) dw += aur;     // w[top-x] of the right column's ug
+  if (j - 1 >= j0) dw += -avp;    // w[top+y] of the previous column's vg
 }
 
 // velocity^T, local part at cell (i, j, k): A = dcrj * f_d * adjoint (the
 // weights the stress adjoints gather), the velocity adjoint scaled by dcrj,
 // and the f_d gradients with the stress differences of the state before the
-// step.  GATHER: the strain -> velocity gather of the same cell first (levels
-// that the free-surface ghosts do not touch), so the velocity adjoints make
-// one trip through HBM instead of two.
-template <bool GATHER>
-__device__ __forceinline__ void vel_local_cell(int i, int j, int k, float* __restrict__ ub,
-                                               float* __restrict__ vb, float* __restrict__ wb,
-                                               const Ptr6& Aw, const CPtr6& Sg, const Medium& M,
-                                               const Grad8& Gr, const AdjGrid& G,
-                                               const CPtr6& E) {
+// step.  In two halves: what the cell's medium and forward state give, and the
+// rest, from the velocity adjoints a, b, c.
+struct VelLocal {
+  float dcrj, f1, f2, f3, Xu, Xv, Xw, g1, g2, g3;
+};
+__device__ __forceinline__ VelLocal vel_local_head(int i, int j, int k, const CPtr6& Sg,
+                                                   const Medium& M, const Grad8& Gr,
+                                                   const AdjGrid& G) {
   const long long S = G.slice, Y = G.yline;
   const long long p = aidx(G, i, j, k);
   const float* d1 = M.d1;
-  const float dcrj = M.dcrjx[i] * M.dcrjy[j] * M.dcrjz[k];
-  const float f1 = G.dth / (float)(0.25 * (double)(d1[p] + d1[p - Y] + d1[p - 1] + d1[p - Y - 1]));
-  const float f2 = G.dth / (float)(0.25 * (double)(d1[p] + d1[p + S] + d1[p - 1] + d1[p + S - 1]));
-  const float f3 = G.dth / (float)(0.25 * (double)(d1[p] + d1[p + S] + d1[p - Y] + d1[p + S - Y]));
+  VelLocal L;
+  L.dcrj = M.dcrjx[i] * M.dcrjy[j] * M.dcrjz[k];
+  // 0.25 * the float sum: the same float whether scaled in binary64 or 32
+  L.f1 = awp_div(G.dth, 0.25f * (d1[p] + d1[p - Y] + d1[p - 1] + d1[p - Y - 1]));
+  L.f2 = awp_div(G.dth, 0.25f * (d1[p] + d1[p + S] + d1[p - 1] + d1[p + S - 1]));
+  L.f3 = awp_div(G.dth, 0.25f * (d1[p] + d1[p + S] + d1[p - Y] + d1[p + S - Y]));
   const float c1 = G.c1, c2 = G.c2;
   const float *xx = Sg.f[0], *yy = Sg.f[1], *zz = Sg.f[2], *xy = Sg.f[3], *xz = Sg.f[4],
               *yz = Sg.f[5];
-  const float Xu = c1 * (xx[p] - xx[p - S]) + c2 * (xx[p + S] - xx[p - 2 * S]) +
-                   c1 * (xy[p] - xy[p - Y]) + c2 * (xy[p + Y] - xy[p - 2 * Y]) +
-                   c1 * (xz[p] - xz[p - 1]) + c2 * (xz[p + 1] - xz[p - 2]);
-  const float Xv = c1 * (xy[p + S] - xy[p]) + c2 * (xy[p + 2 * S] - xy[p - S]) +
-                   c1 * (yy[p + Y] - yy[p]) + c2 * (yy[p + 2 * Y] - yy[p - Y]) +
-                   c1 * (yz[p] - yz[p - 1]) + c2 * (yz[p + 1] - yz[p - 2]);
-  const float Xw = c1 * (xz[p + S] - xz[p]) + c2 * (xz[p + 2 * S] - xz[p - S]) +
-                   c1 * (yz[p] - yz[p - Y]) + c2 * (yz[p + Y] - yz[p - 2 * Y]) +
-                   c1 * (zz[p + 1] - zz[p]) + c2 * (zz[p + 2] - zz[p - 1]);
-  float a = ub[p], b = vb[p], c = wb[p];
-  if (GATHER) {
-    const Vec3 g = strain_gather(E, p, S, Y, c1, c2);
-    a += g.u;
-    b += g.v;
-    c += g.w;
-  }
-  Gr.f[0][p] += a * dcrj * Xu;
-  Gr.f[1][p] += b * dcrj * Xv;
-  Gr.f[2][p] += c * dcrj * Xw;
-  Aw.f[0][p] = dcrj * f1 * a;
-  Aw.f[1][p] = dcrj * f2 * b;
-  Aw.f[2][p] = dcrj * f3 * c;
+  L.Xu = c1 * (xx[p] - xx[p - S]) + c2 * (xx[p + S] - xx[p - 2 * S]) +
+         c1 * (xy[p] - xy[p - Y]) + c2 * (xy[p + Y] - xy[p - 2 * Y]) +
+         c1 * (xz[p] - xz[p - 1]) + c2 * (xz[p + 1] - xz[p - 2]);
+  L.Xv = c1 * (xy[p + S] - xy[p]) + c2 * (xy[p + 2 * S] - xy[p - S]) +
+         c1 * (yy[p + Y] - yy[p]) + c2 * (yy[p + 2 * Y] - yy[p - Y]) +
+         c1 * (yz[p] - yz[p - 1]) + c2 * (yz[p + 1] - yz[p - 2]);
+  L.Xw = c1 * (xz[p + S] - xz[p]) + c2 * (xz[p + 2 * S] - xz[p - S]) +
+         c1 * (yz[p] - yz[p - Y]) + c2 * (yz[p + Y] - yz[p - 2 * Y]) +
+         c1 * (zz[p + 1] - zz[p]) + c2 * (zz[p + 2] - zz[p - 1]);
+  L.g1 = Gr.f[0][p];
+  L.g2 = Gr.f[1][p];
+  L.g3 = Gr.f[2][p];
+  return L;
+}
+__device__ __forceinline__ void vel_local_tail(long long p, float a, float b, float c,
+                                               const VelLocal& L, float* __restrict__ ub,
+                                               float* __restrict__ vb, float* __restrict__ wb,
+                                               const Ptr6& Aw, const Grad8& Gr) {
+  const float dcrj = L.dcrj;
+  Gr.f[0][p] = L.g1 + a * dcrj * L.Xu;
+  Gr.f[1][p] = L.g2 + b * dcrj * L.Xv;
+  Gr.f[2][p] = L.g3 + c * dcrj * L.Xw;
+  Aw.f[0][p] = dcrj * L.f1 * a;
+  Aw.f[1][p] = dcrj * L.f2 * b;
+  Aw.f[2][p] = dcrj * L.f3 * c;
   ub[p] = dcrj * a;
   vb[p] = dcrj * b;
   wb[p] = dcrj * c;
 }
 
-// The strain gather and velocity^T below the free-surface band, levels
-// [k0, k1], one column's levels per wave; asked for 8 waves per SIMD (63
-// VGPRs from 72, no spills).
+// Two parts of one launch, on different blocks (the first nband ones are the
+// second part: a chain of round trips on few cells, hidden behind the first
+// part; 10.1 us as a launch of its own at 96x96x64).
+// 1: levels k0 .. k1 below the free-surface band, one column's levels per
+// wave: the strain -> velocity gather and velocity^T of the cell, so the
+// velocity adjoints make one trip through memory instead of two.
+// 2: levels top-1 .. top+1 (band_cell's lane map): the gather of each cell
+// and, on the ghost level top+1, ghost^T part 1 of the cell's column from the
+// values just gathered.  Part 1 reads only its own column's ghost level, so it
+// needs no barrier after the gathers of the other columns.
+// Asked for 8 waves per SIMD (64 VGPRs, no spills).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8)))
-void adj_vel_local_kernel(float* __restrict__ ub,
-                                                            float* __restrict__ vb,
-                                                            float* __restrict__ wb, Ptr6 Aw,
-                                                            CPtr6 Sg, Medium M, Grad8 Gr,
-                                                            const AdjGrid G, CPtr6 E, int k0,
-                                                            int k1) {
-  const Blk3 B = adj_block(G);
+void adj_vel_local_kernel(float* __restrict__ ub, float* __restrict__ vb,
+                          float* __restrict__ wb, Ptr6 Aw, CPtr6 Sg, Medium M, Grad8 Gr,
+                          const AdjGrid G, CPtr6 E, CPtr3 V, float* __restrict__ col,
+                          float* __restrict__ glm, int k0, int k1, int nkt, int njt, int nband) {
+  const long long S = G.slice, Y = G.yline;
+  const int bid = (int)blockIdx.x;
+  if (bid < nband) {
+    const BandCell b = band_cell(G, G.top - 1, G.top + 1,
+                                 adj_block(G, nband / G.nx, 1, G.nx, bid));
+    if (!b.ok) return;
+    const bool ghost = b.k == G.top + 1;
+    const long long c = aidx(G, b.i, b.j, b.k);
+    const long long q2 = (long long)b.i * G.lam_mu_ld + b.j;
+    float Bk = 0.0f, lm = 0.0f, gl = 0.0f;
+    if (ghost) {
+      Bk = ghost1_bracket(b.i, b.j, V, G);
+      lm = M.lam_mu[q2];
+      gl = glm[q2];
+    }
+    const float u0 = ub[c], v0 = vb[c], w0 = wb[c];
+    const Vec3 g = strain_gather(E, c, S, Y, G.c1, G.c2);
+    const float un = u0 + g.u, vn = v0 + g.v, wn = w0 + g.w;
+    ub[c] = un;
+    vb[c] = vn;
+    wb[c] = wn;
+    if (ghost) ghost1_column(b.i, b.j, un, vn, wn, Bk, lm, gl, col, glm, G);
+    return;
+  }
+  const Blk3 B = adj_block(G, nkt, njt, G.nx, bid - nband);
   const int k = k0 + (int)(B.x * 64 + threadIdx.x);
   const int j = 2 + AWP_NGSL + (int)(B.y * 4 + threadIdx.y);
   const int i = 2 + AWP_NGSL + B.z;
   if (k > k1 || j >= G.ny + 2 + AWP_NGSL) return;
-  vel_local_cell<true>(i, j, k, ub, vb, wb, Aw, Sg, M, Gr, G, E);
-}
-
-// The free-surface band, first part (levels top-1 .. top+1, band_cell's lane
-// map): the strain -> velocity gather of each cell, then, on the ghost level
-// top+1, ghost^T part 1 of the cell's column from the values just gathered.
-// Part 1 reads only its own column's ghost level, so it needs no barrier
-// after the gathers of the other columns.
-__global__ __launch_bounds__(256) void adj_band_gather_kernel(
-    float* __restrict__ ub, float* __restrict__ vb, float* __restrict__ wb, CPtr6 E, CPtr3 V,
-    const float* __restrict__ lam_mu, float* __restrict__ col, float* __restrict__ glm,
-    const AdjGrid G) {
-  const BandCell b = band_cell(G, G.top - 1, G.top + 1);
-  if (!b.ok) return;
-  const long long S = G.slice, Y = G.yline;
-  const long long c = aidx(G, b.i, b.j, b.k);
-  const Vec3 g = strain_gather(E, c, S, Y, G.c1, G.c2);
-  const float un = ub[c] + g.u, vn = vb[c] + g.v, wn = wb[c] + g.w;
-  ub[c] = un;
-  vb[c] = vn;
-  wb[c] = wn;
-  if (b.k == G.top + 1) ghost1_column(b.i, b.j, un, vn, wn, V, lam_mu, col, glm, G);
+  const long long p = aidx(G, i, j, k);
+  const VelLocal L = vel_local_head(i, j, k, Sg, M, Gr, G);
+  const float a = ub[p], b = vb[p], c = wb[p];
+  const Vec3 g = strain_gather(E, p, S, Y, G.c1, G.c2);
+  vel_local_tail(p, a + g.u, b + g.v, c + g.w, L, ub, vb, wb, Aw, Gr);
 }
 
 // The free-surface band, second part (levels top-1 and top, band_cell's lane
 // map: the two lanes of a column are neighbours in one wave).  The lane of
 // level top runs ghost^T part 2 of the column (its ghost adjoints gathered
-// from the neighbours' part 1) and hands the w ghost's adjoint wb[top+1],
-// read before part 2 clears it, to the lane of level top-1, which adds it to
+// from the neighbours' part 1), clears the ghost level and hands the w ghost's
+// adjoint wb[top+1], read before, to the lane of level top-1, which adds it to
 // its own cell; then each lane runs velocity^T on its cell, which reads only
-// that cell's adjoints.
+// that cell's adjoints.  A few waves per CU: one chain of round trips, so all
+// loads come first and the adjoints between the parts stay in registers.
 __global__ __launch_bounds__(256) void adj_band_ghost_kernel(
     float* __restrict__ ub, float* __restrict__ vb, float* __restrict__ wb,
     const float* __restrict__ col, Ptr6 Aw, CPtr6 Sg, Medium M, Grad8 Gr, const AdjGrid G) {
-  const BandCell b = band_cell(G, G.top - 1, G.top);
+  const BandCell b = band_cell(G, G.top - 1, G.top, adj_block(G));
   if (!b.ok) return;  // per column: both lanes of a column return or neither
   const bool at_top = b.k == G.top;
-  const long long p = aidx(G, b.i, b.j, G.top);
-  const float wg = at_top ? wb[p + 1] : 0.0f;
+  const long long p = aidx(G, b.i, b.j, b.k), pt = aidx(G, b.i, b.j, G.top);
+  const float wg = at_top ? wb[pt + 1] : 0.0f;
   const float wg_top = __shfl_down(wg, 1);  // the top lane's wb[top+1], on the top-1 lane
-  if (at_top)
-    ghost2_column(b.i, b.j, ub, vb, wb, col, G);
-  else
-    wb[p - 1] += wg_top;  // w[top-1] of the w ghost
-  const CPtr6 none = {};
-  vel_local_cell<false>(b.i, b.j, b.k, ub, vb, wb, Aw, Sg, M, Gr, G, none);
+  const float u0 = ub[p], v0 = vb[p], w0 = wb[p];
+  float du, dv, dw;
+  ghost2_column(b.i, b.j, col, G, du, dv, dw);
+  const VelLocal L = vel_local_head(b.i, b.j, b.k, Sg, M, Gr, G);
+  if (at_top) {
+    ub[pt + 1] = 0.0f;
+    vb[pt + 1] = 0.0f;
+    wb[pt + 1] = 0.0f;
+  }
+  vel_local_tail(p, at_top ? u0 + du : u0, at_top ? v0 + dv : v0, at_top ? w0 + dw : w0 + wg_top, L,
+                 ub, vb, wb, Aw, Gr);
 }
 
 // velocity^T, gather part: stress adjoints from the weighted velocity
@@ -548,7 +587,7 @@ __global__ __launch_bounds__(256) void adj_band_ghost_kernel(
 // band, which fstr^T touches, is gathered at once.
 __global__ __launch_bounds__(256) void adj_vel_gather_kernel(Adj15 Ab, CPtr6 Aw,
                                                              const AdjGrid G, int k0, int k1) {
-  const BandCell b = band_cell(G, k0, k1);
+  const BandCell b = band_cell(G, k0, k1, adj_block(G));
   if (!b.ok) return;
   const long long q = aidx(G, b.i, b.j, b.k);
   float g[6];
@@ -592,6 +631,59 @@ __global__ __launch_bounds__(256) void adj_flush_kernel(float* __restrict__ g32,
     g64[i] += (double)g32[i];
     g32[i] = 0.0f;
   }
+}
+
+// The same for the eight coefficient gradients of the grid and the surface's
+// lam_mu gradient, which are zero outside the interior columns and levels: one
+// launch over the interior cells (96x96x64, which fill a third of their padded
+// arrays: 27 us against nine flat launches of 73 us in all).
+struct Grad64 {
+  double* f[8];
+};
+__global__ __launch_bounds__(256) void adj_flush_grid_kernel(Grad8 g32, Grad64 g64,
+                                                             float* __restrict__ l32,
+                                                             double* __restrict__ l64,
+                                                             const AdjGrid G) {
+  const int k = AWP_ALIGN + (int)(blockIdx.x * 64 + threadIdx.x);
+  const int j = 2 + AWP_NGSL + (int)(blockIdx.y * 4 + threadIdx.y);
+  const int i = 2 + AWP_NGSL + (int)blockIdx.z;
+  if (k > G.top || j >= G.ny + 2 + AWP_NGSL) return;
+  const long long p = aidx(G, i, j, k);
+  float a[8];
+  double b[8];
+#pragma unroll
+  for (int f = 0; f < 8; ++f) {
+    a[f] = g32.f[f][p];
+    b[f] = g64.f[f][p];
+  }
+#pragma unroll
+  for (int f = 0; f < 8; ++f) {
+    g64.f[f][p] = b[f] + (double)a[f];
+    g32.f[f][p] = 0.0f;
+  }
+  if (k == G.top) {
+    const long long q = (long long)i * G.lam_mu_ld + j;
+    l64[q] += (double)l32[q];
+    l32[q] = 0.0f;
+  }
+}
+
+// dst[f] = src[f], or 0 without a source, over n bytes of each of nf arrays:
+// one launch for a state's fields (15 copies of 6.7 MB each took 4.9 us, and
+// as many clears 3.6 us, from their own launches).  Blocks stride over 16-byte
+// words (V = int4; V = char for the rest, or all if an array is not aligned).
+struct FieldPtrs {
+  char* dst[AWP_MOVE_FIELDS];
+  const char* src[AWP_MOVE_FIELDS];
+};
+template <class V>
+__global__ __launch_bounds__(256) void move_fields_kernel(FieldPtrs P, long long from,
+                                                          long long to) {
+  V* __restrict__ d = (V*)P.dst[blockIdx.y];
+  const V* __restrict__ s = (const V*)P.src[blockIdx.y];
+  const long long step = (long long)gridDim.x * 256;
+  for (long long q = from + blockIdx.x * 256ll + threadIdx.x; q < to; q += step)
+    d[q] = s ? s[q] : V{};
 }
 
 // residuals d - obs and the misfit 1/2 sum (d - obs)^2 in binary64: one
@@ -786,25 +878,25 @@ void awp_adjoint_step(float* const* adj, const float* const* fwd_v, const float*
   Grad8 Gr;
   for (int f = 0; f < 8; ++f) Gr.f[f] = grad[f];
   const Medium M = adj_medium(med, ww, coeff, dcrjx, dcrjy, dcrjz);
-  const dim3 b2(64, 4);
-  const dim3 g2(awp_cdiv(G.ny, 64), awp_cdiv(G.nx, 4));
-  hipLaunchKernelGGL(adj_fstr_kernel, g2, b2, 0, St, A.f[2], A.f[4], A.f[5], G);
   const int nks = G.top - (AWP_ALIGN + 3) + 1;
+  const bool fstr = nks >= 3;  // adj_stress_local_kernel covers fstr^T's levels
+  if (!fstr)
+    hipLaunchKernelGGL(adj_fstr_kernel, dim3(awp_cdiv(G.ny, 64), awp_cdiv(G.nx, 4)), dim3(64, 4),
+                       0, St, A.f[2], A.f[4], A.f[5], G);
   hipLaunchKernelGGL(adj_stress_local_kernel, dim3(awp_cdiv(nks, 64), awp_cdiv(G.ny, 4), G.nx),
-                     dim3(64, 4), 0, St, A, E, V, M, Gr, G, Awc);
+                     dim3(64, 4), 0, St, A, E, V, M, Gr, G, Awc, fstr);
   // levels align .. top-2: strain gather and velocity^T in one pass (the
-  // free-surface ghosts' transpose reads and writes only top-1 .. top+1)
-  const int kf1 = G.top - 2;
-  const int nkf = kf1 - AWP_ALIGN + 1;
-  hipLaunchKernelGGL(adj_vel_local_kernel, dim3(awp_cdiv(nkf, 64), awp_cdiv(G.ny, 4), G.nx),
-                     dim3(64, 4), 0, St, A.f[12], A.f[13], A.f[14], Aw, Sg, M, Gr, G, Ec,
-                     AWP_ALIGN, kf1);
+  // free-surface ghosts' transpose reads and writes only top-1 .. top+1);
   // levels top-1 .. top+1: gather and ghost^T part 1; then per column ghost^T
   // part 2 and velocity^T on top-1 .. top (band launches: (cdiv(nk * ny,
   // 256), 1, nx) blocks for nk levels)
   auto band = [&](int nk) { return dim3(awp_cdiv(nk * G.ny, 256), 1, G.nx); };
-  hipLaunchKernelGGL(adj_band_gather_kernel, band(3), dim3(64, 4), 0, St, A.f[12], A.f[13],
-                     A.f[14], Ec, V, M.lam_mu, col, grad_lam_mu, G);
+  const int kf1 = G.top - 2;
+  const int nkt = awp_cdiv(kf1 - AWP_ALIGN + 1, 64), njt = awp_cdiv(G.ny, 4);
+  const int nband = (int)band(3).x * G.nx;
+  hipLaunchKernelGGL(adj_vel_local_kernel, dim3(nband + nkt * njt * G.nx), dim3(64, 4), 0, St,
+                     A.f[12], A.f[13], A.f[14], Aw, Sg, M, Gr, G, Ec, V, col, grad_lam_mu,
+                     AWP_ALIGN, kf1, nkt, njt, nband);
   hipLaunchKernelGGL(adj_band_ghost_kernel, band(2), dim3(64, 4), 0, St, A.f[12], A.f[13],
                      A.f[14], col, Aw, Sg, M, Gr, G);
   // the free-surface band now; the levels below stay pending for the next
@@ -844,6 +936,52 @@ void awp_adjoint_flush(float* g32, double* g64, long long n, hipStream_t St) {
   long long b = (n + 255) / 256;
   hipLaunchKernelGGL(adj_flush_kernel, dim3((unsigned)(b < 4096 ? b : 4096)), dim3(256), 0, St,
                      g32, g64, n);
+  awp_check_launch(W);
+}
+
+void awp_adjoint_flush_grid(float* const* g32, double* const* g64, float* grad_lam_mu32,
+                            double* grad_lam_mu64, hipStream_t St) {
+  const char* W = "awp_adjoint_flush_grid";
+  if (!awp_grid_ok(0, W)) return;
+  const AdjGrid G = adj_grid(0);
+  Grad8 a;
+  Grad64 b;
+  for (int f = 0; f < 8; ++f) {
+    a.f[f] = g32[f];
+    b.f[f] = g64[f];
+  }
+  hipLaunchKernelGGL(adj_flush_grid_kernel, dim3(awp_cdiv(G.nz, 64), awp_cdiv(G.ny, 4), G.nx),
+                     dim3(64, 4), 0, St, a, b, grad_lam_mu32, grad_lam_mu64, G);
+  awp_check_launch(W);
+}
+
+void awp_move_fields(void* const* dst, const void* const* src, int nf, long long n,
+                     hipStream_t St) {
+  const char* W = "awp_move_fields";
+  if (nf < 0 || nf > AWP_MOVE_FIELDS || n < 0) {
+    awp_set_error(AWP_ERR_ARG, "%s: %d fields of %lld bytes (at most %d fields)", W, nf, n,
+                  AWP_MOVE_FIELDS);
+    return;
+  }
+  if (nf == 0 || n == 0) return;
+  FieldPtrs P = {};
+  bool wide = true;
+  for (int f = 0; f < nf; ++f) {
+    P.dst[f] = (char*)dst[f];
+    P.src[f] = src ? (const char*)src[f] : nullptr;
+    wide = wide && !(((uintptr_t)P.dst[f] | (uintptr_t)P.src[f]) & 15);
+  }
+  // at least 4 words a lane, and no more blocks than the chip holds at once
+  auto blocks = [&](long long w) {
+    const long long b = (w + 1023) / 1024, most = (2048 + nf - 1) / nf;
+    return dim3((unsigned)(b < most ? b : most), (unsigned)nf);
+  };
+  const long long w16 = wide ? n / 16 : 0;
+  if (w16)
+    hipLaunchKernelGGL(move_fields_kernel<int4>, blocks(w16), dim3(256), 0, St, P, 0ll, w16);
+  if (n > w16 * 16)
+    hipLaunchKernelGGL(move_fields_kernel<char>, blocks(n - w16 * 16), dim3(256), 0, St, P,
+                       w16 * 16, n);
   awp_check_launch(W);
 }
 

@@ -320,6 +320,15 @@ void awp_adjoint_inject(float* ub, float* vb, float* wb, const int* idx, int npt
                         const double* res, hipStream_t St);
 /* g64 += g32; g32 = 0 over n values */
 void awp_adjoint_flush(float* g32, double* g64, long long n, hipStream_t St);
+/* the same for the eight coefficient gradients of awp_adjoint_step (grad[8])
+ * and its grad_lam_mu, over the cells that it writes */
+void awp_adjoint_flush_grid(float* const* g32, double* const* g64, float* grad_lam_mu32,
+                            double* grad_lam_mu64, hipStream_t St);
+/* dst[f] = src[f] over n bytes of each of nf <= AWP_MOVE_FIELDS arrays, or 0
+ * where src[f] (or src itself) is null; no dst overlaps another array */
+#define AWP_MOVE_FIELDS 16
+void awp_move_fields(void* const* dst, const void* const* src, int nf, long long n,
+                     hipStream_t St);
 /* res = d - obs (binary64) and *J = 1/2 sum res^2 over n samples; work holds
  * AWP_MISFIT_PARTS doubles (one partial sum per block) */
 #define AWP_MISFIT_PARTS 256
