@@ -104,10 +104,13 @@ struct CodecBF16 {
 // (the same value as x * s, flushes included).  A multiply beside the
 // conversion would be fused into v_fma_mix*, which follows the binary32
 // denormal mode and so loses binary16 subnormals; ldexp has no mix form.
+// The scale is a normal number and the same for every lane, so its exponent
+// field is taken by scalar instructions (frexp has none: the 30 exponents of a
+// kernel would sit in vector registers).
 struct CodecF16 {
   static constexpr int fmt = AWP_FMT_F16;
   __device__ static __forceinline__ float scale(float x, float s) {
-    return __builtin_ldexpf(x, __builtin_amdgcn_frexp_expf(s) - 1);
+    return __builtin_ldexpf(x, (int)(__builtin_bit_cast(uint32_t, s) >> 23) - 127);
   }
   __device__ static __forceinline__ float to_f32(uint16_t q) { return awp_f16_to_f32(q); }
   __device__ static __forceinline__ uint16_t from_f32(float x) { return awp_f32_to_f16(x); }

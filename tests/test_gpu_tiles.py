@@ -1,7 +1,7 @@
 """The (k, j) tiles of the marching Cartesian kernels (awp_pick_tile) at the
 column heights where the rule changes: one wave and less, 64 m levels, one row
-per workgroup of 2, 3 and 4 waves, and 64-level runs beyond 256.  Velocity,
-stress bit for bit against the oracle: the arithmetic
+per workgroup of 2, 3 and 4 waves, and 64-level runs beyond 256; and the two routes of the
+free-surface velocity ghosts.  Bit for bit against the oracle: the arithmetic
 is the same expression by expression, so the tolerance is zero."""
 import ctypes as C
 
@@ -32,9 +32,19 @@ def gpu():
 
 @pytest.mark.parametrize("nz", [36, 61, 64, 65, 101, 128, 130, 191, 193, 255, 256, 257, 300])
 def test_column_heights_bit_exact(gpu, oracle_lib, nz):
+    _velocity_stress(gpu, oracle_lib, Dims(11, 9, nz))
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(256, 256, 4), (257, 256, 5), (512, 256, 4), (513, 256, 4)])
+def test_surface_ghosts_bit_exact(gpu, oracle_lib, nx, ny, nz):
+    """The velocity ghosts in the stress kernel (up to 2^17 columns) and in
+    their own launch (more)."""
+    _velocity_stress(gpu, oracle_lib, Dims(nx, ny, nz))
+
+
+def _velocity_stress(gpu, oracle_lib, d):
     torch, lib, _lib = gpu
-    d = Dims(11, 9, nz)
-    st, med = random_state(d, seed=3 + nz)
+    st, med = random_state(d, seed=3 + d.nzt)
     F, I = C.c_float, C.c_int
     z9 = (F * 9)()
     lib.SetDeviceConstValue((F * 1)(DH), F(DT), (I * 1)(d.nxt), (I * 1)(d.nyt), (I * 1)(d.nzt),
