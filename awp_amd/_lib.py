@@ -19,6 +19,17 @@ _f = C.c_float
 _s = C.c_void_p  # hipStream_t
 
 
+class RunArgs(C.Structure):
+    """awp_run_t of include/awp_hip.h."""
+    _fields_ = [("f", _fp * 15),
+                *[(n, _fp) for n in ("d1", "lam", "mu", "qp", "qs", "coeff", "lam_mu", "dcrjx",
+                                     "dcrjy", "dcrjz", "vx1", "vx2", "wwo", "ww", "tex", "psrc")],
+                ("src", _fp * 6),
+                *[(n, _fp) for n in ("rec_idx", "rec_out", "stream")],
+                *[(n, _i) for n in ("nxt", "nyt", "nzt", "NPC", "newlit", "s_i", "e_i", "s_j",
+                                    "e_j", "npsrc", "nst", "rec_n", "rec_rows")]]
+
+
 # name -> argtypes, in header order
 SIGNATURES: dict[str, list] = {
     "awp_last_error": [],
@@ -69,6 +80,7 @@ SIGNATURES: dict[str, list] = {
     "awp_dvelcx_oop": [_fp] * 16 + [_i, _i, _s, _i, _i, _i, _i],
     "awp_dstrqc_oop": [_fp] * 24 + [_i, _i, _s] + [_fp] * 5 + [_i] * 9,
     "awp_dstrqc_tex": [_fp] * 23 + [_i, _i, _s] + [_fp] * 3 + [_i] * 9,
+    "awp_run_steps": [C.POINTER(RunArgs), _i, _i],
     "awp_step": [_fp] * 11 + [_i, _i, _i, _s],
     "awp_stream_probe": [_fp, _i, _fp, _i, C.c_longlong, _i, _i, _i, _s],
     # topo_t* travels as a plain address (ctypes.byref of awp_amd.refstructs.Topo)

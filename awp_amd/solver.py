@@ -74,6 +74,8 @@ def check_dm_stack(media: Sequence[Medium]) -> None:
             raise ValueError("all grids share one time step")
 
 
+RUN_FIELDS = ("xx", "yy", "zz", "xy", "xz", "yz", "r1", "r2", "r3", "r4", "r5", "r6", "u1", "v1",
+              "w1")
 # the state awp_step reads from one set and writes to the other
 STEP_FIELDS = ("u1", "v1", "w1", "xx", "yy", "zz", "xy", "xz", "yz")
 
@@ -472,11 +474,55 @@ class Solver(PmclStepOrder):
     def run(self, nt: int, check_every: int = 0) -> None:
         if self.cur_step == 0:
             self.start()
+        if self._native():
+            # at most 256 steps a call, so that signals are seen
+            n, every = 0, abs(check_every)
+            while n < nt:
+                m = min(nt - n, 256, every - n % every if every else nt)
+                self.lib.awp_run_steps(C.byref(self._run_args()), self.cur_step, m)
+                self.cur_step += m
+                n += m
+                if every and n % every == 0:
+                    _lib.check()
+            _lib.check()
+            return
         for n in range(nt):
             self.step()
             if check_every and (n + 1) % check_every == 0:
                 _lib.check()
         _lib.check()
+
+    def _native(self) -> bool:
+        """Whether run's steps are exactly what awp_run_steps launches: one
+        Cartesian FP32 grid, NVE = 1, no part of the step replaced."""
+        return (self.lib is _lib.load() and self.ngrids == 1 and self.plastic is None and self.topo is None
+                and self.kinematic is None and self.pointio is None and not self.fused
+                and all(getattr(getattr(self, n), "__func__", None) is fn
+                        for n, fn in _STEP_METHODS.items()))
+
+    def _run_args(self) -> _lib.RunArgs:
+        L, r = self.levels[0], self.rec
+        d, f, m, s = L.dims, L.f, L.m, L.src
+        a = _lib.RunArgs()
+        a.f[:] = [_ptr(f[n]) for n in RUN_FIELDS]
+        for n in ("d1", "lam", "mu", "qp", "qs", "coeff", "lam_mu", "dcrjx", "dcrjy", "dcrjz",
+                  "vx1", "vx2", "wwo"):
+            setattr(a, n, _ptr(m[n]))
+        if L.texmode != "rule":
+            a.ww = _ptr(m["ww"])
+        if L.texmode != "arrays":
+            a.tex = C.addressof(L.tex)
+        a.newlit = int(self.variant != "dstrqc")
+        a.nxt, a.nyt, a.nzt, a.NPC = d.nxt, d.nyt, d.nzt, self.NPC
+        (a.s_i, a.e_i), (a.s_j, a.e_j) = d.i_range, d.j_range
+        if s is not None:
+            a.psrc, a.npsrc, a.nst = _ptr(s["psrc"]), s["npsrc"], s["nst"]
+            a.src[:] = [_ptr(t) for t in s["cols"]]
+        if r is not None:
+            a.rec_idx, a.rec_n = _ptr(r["idx"]), r["n"]
+            a.rec_out, a.rec_rows = _ptr(r["out"]), r["out"].shape[0]
+        a.stream = self.stream
+        return a
 
     def traces(self) -> np.ndarray:
         torch.cuda.synchronize(self.device)
@@ -485,6 +531,12 @@ class Solver(PmclStepOrder):
     def field(self, name: str, p: int = 0) -> np.ndarray:
         torch.cuda.synchronize(self.device)
         return self.levels[p].f[name].cpu().numpy()
+
+
+# the methods that make up a step of run
+_STEP_METHODS = {n: getattr(Solver, n) for n in
+                 ("step", "velocity", "velocity_dm", "_couple", "grid_dims", "stress_region",
+                  "stress", "_sources", "source_steps", "add_source", "free_surface", "record")}
 
 
 class Solver16(ScaledStorage, Solver):

@@ -388,6 +388,29 @@ void awp_dstrqc_tex(float* xx, float* yy, float* zz, float* xy, float* xz, float
                     hipStream_t St, float* lam_mu, const float* tex, int* ww, int NX, int NPC,
                     int rankx, int ranky, int s_i, int e_i, int s_j, int e_j, int d_i);
 
+/* nsteps steps of the pmcl3d loop on a single Cartesian grid, NVE = 1, one
+ * rank, after step cur_step (src/awp/pmcl3d.c:1628-2249; no launcher of the
+ * reference's): dvelcx_H_opt, the stress update, addsrc_H while the sources
+ * have a sample, fstr_H, awp_receivers_gather, as a caller of each would
+ * sequence them. */
+typedef struct {
+  float* f[15];                 /* xx yy zz xy xz yz r1..r6 u1 v1 w1 */
+  float *d1, *lam, *mu, *qp, *qs, *coeff, *lam_mu, *dcrjx, *dcrjy, *dcrjz;
+  float *vx1, *vx2, *wwo;
+  int* ww;
+  const float* tex;             /* awp_dstrqc_tex's table (with ww or NULL), or
+                                 * NULL: dstrqc_H, dstrqc_H_new if newlit */
+  int* psrc;
+  float* src[6];                /* axx ayy azz axz ayz axy */
+  const int* rec_idx;
+  float* rec_out;
+  void* stream;
+  int nxt, nyt, nzt, NPC, newlit, s_i, e_i, s_j, e_j;
+  int npsrc, nst;               /* nst = 0: no sources */
+  int rec_n, rec_rows;          /* rec_rows = 0: no receivers */
+} awp_run_t;
+void awp_run_steps(const awp_run_t* run, int cur_step, int nsteps);
+
 /* The extended entry point: one NVE = 1 step of a single Cartesian grid
  * (grid 0 of SetDeviceConstValue, ngrids = 1, one rank: NX = nxt, NPC = 0)
  * in one sweep, equal bit for bit to dvelcx_H_opt over the interior
