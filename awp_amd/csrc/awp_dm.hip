@@ -16,6 +16,7 @@
 // 125 fine values per output; it stages the 8 fine levels of a tile into LDS
 // once per field instead of re-reading them through the caches.
 #include "awp_common.h"
+#include "awp_math.h"
 #include "../../include/awp_hip.h"
 
 namespace {
@@ -59,16 +60,14 @@ __global__ __launch_bounds__(256) void dvelc2_kernel(
 
 // ---------------------------------------------------------------------------
 // dstrqc2.  Q weights with this kernel's literal types: the qpa test is single
-// precision and the else branches carry no factor 2 (kernel.cu:2638-2683).
-// ca, cb: coeff[ww*2-2], coeff[ww*2-1], loaded once per cell before the
-// branches.
-__device__ __forceinline__ float dm_qweight(float ca, float cb, float wwo, float q) {
-  float w;
-  if (1. / ((double)q * 2.0) <= 200.0)
-    w = (float)((double)ca * (2. * (double)q) * (2. * (double)q) + (double)cb * (2. * (double)q));
-  else
-    w = wwo * q;
-  return w / wwo;
+// precision (low: its outcome) and the else branches carry no factor 2
+// (kernel.cu:2638-2683).  ca, cb: coeff[ww*2-2], coeff[ww*2-1]; y =
+// awp_rcp(wwo).
+__device__ __forceinline__ float dm_qweight(float ca, float cb, float wwo, float y, float q,
+                                            bool low) {
+  const double t = 2. * (double)q;
+  const float quad = (float)((double)ca * t * t + (double)cb * t);
+  return awp_div_by(low ? quad : wwo * q, wwo, y);
 }
 
 // Relaxation texture of dstrqc2 (as in dstrqc_H's table forms): the
@@ -85,8 +84,13 @@ struct Dm2Tex {
   int xls, yls, nj, nzt;
 };
 
+// One lane per cell of the level, lanes along j.  Every array costs a line per
+// cell (columns are a yline apart), and a 288x288 level is little more than one
+// wave per SIMD: all loads go out together before any arithmetic (the
+// scheduling barrier keeps them there), and workgroups are single waves, which
+// spread evenly over the CUs: 70 -> 57 us.
 template <int TEX>
-__global__ __launch_bounds__(256) void dstrqc2_kernel(
+__global__ __launch_bounds__(64) void dstrqc2_kernel(
     float* __restrict__ xx, float* __restrict__ yy, float* __restrict__ zz,
     float* __restrict__ xy, float* __restrict__ xz, float* __restrict__ yz,
     float* __restrict__ r1, float* __restrict__ r2, float* __restrict__ r3,
@@ -100,62 +104,69 @@ __global__ __launch_bounds__(256) void dstrqc2_kernel(
     const float* __restrict__ wwop, const PlaneLaunch L, const Dm2Tex TT) {
   __shared__ float s_tex[24];
   if (TEX != DM2_TEX_ARRAYS) {
-    const int tid = (int)(threadIdx.y * 64 + threadIdx.x);
+    const int tid = (int)threadIdx.x;
     if (tid < 24) s_tex[tid] = TT.t[tid];
     __syncthreads();
   }
   const int j = L.j0 + (int)(blockIdx.x * 64 + threadIdx.x);
-  const int i = L.i0 + (int)(blockIdx.y * 4 + threadIdx.y);
-  if (j > L.j1 || i > L.i1) return;
+  const int i = L.i0 + (int)blockIdx.y;
+  if (j > L.j1) return;
   const int k = AWP_ALIGN + 2;
   const long long S = L.slice, Y = L.yline;
   const long long p = (long long)i * S + (long long)j * Y + k;
   const long long ip1 = p + S, jm1 = p - Y, ijk = p + S - Y, km1 = p - 1, ik1 = p + S - 1,
                   jk1 = p - Y - 1, ijk1 = p + S - Y - 1;
   const float DT = L.DT, dth = L.dth, dh1 = L.dh1;
-  const float f_dcrj = dcrjz[k] * dcrjx[i] * dcrjy[j];
-  float f_vx1, f_vx2, f_wwo;
-  int f_ww;
+  float f_vx1 = 0.0f, f_vx2 = 0.0f, f_wwo = 0.0f;
+  int f_ww = 1;
   if (TEX == DM2_TEX_ARRAYS) {
     f_vx1 = vx1p[p]; f_vx2 = vx2p[p]; f_wwo = wwop[p];
-    f_ww = wwp[p];
-  } else {
-    if (TEX == DM2_TEX_TABLE) {
-      f_ww = wwp[p];
-    } else {
+  }
+  if (TEX != DM2_TEX_RULE) f_ww = wwp[p];
+  const float l0 = lam[p], l1 = lam[ip1], l2 = lam[jm1], l3 = lam[ijk], l4 = lam[km1],
+              l5 = lam[ik1], l6 = lam[jk1], l7 = lam[ijk1];
+  const float m0 = mu[p], m1 = mu[ip1], m2 = mu[jm1], m3 = mu[ijk], m4 = mu[km1], m5 = mu[ik1],
+              m6 = mu[jk1], m7 = mu[ijk1];
+  const float p0 = qp[p], p1 = qp[ip1], p2 = qp[jm1], p3 = qp[ijk], p4 = qp[km1], p5 = qp[ik1],
+              p6 = qp[jk1], p7 = qp[ijk1];
+  const float q0 = qs[p], q1 = qs[ip1], q2 = qs[jm1], q3 = qs[ijk], q4 = qs[km1], q5 = qs[ik1],
+              q6 = qs[jk1], q7 = qs[ijk1];
+  const float u0 = u1[p], u_kp = u1[p + 1], u_ip = u1[p + S], u_jp = u1[p + Y];
+  const float v0 = v1[p], v_kp = v1[p + 1], v_im = v1[p - S], v_jm = v1[p - Y];
+  const float w0 = w1[p], w_im = w1[p - S], w_jp = w1[p + Y], w_km = w1[p - 1];
+  const float xx0 = xx[p], yy0 = yy[p], zz0 = zz[p], xy0 = xy[p], xz0 = xz[p], yz0 = yz[p];
+  const float r10 = r1[p], r20 = r2[p], r30 = r3[p], r40 = r4[p], r50 = r5[p], r60 = r6[p];
+  const float dcx = dcrjx[i], dcy = dcrjy[j], dcz = dcrjz[k];
+  __builtin_amdgcn_sched_barrier(0);
+
+  const float f_dcrj = dcz * dcx * dcy;
+  if (TEX != DM2_TEX_ARRAYS) {
+    if (TEX == DM2_TEX_RULE) {
       const int ni = i - TT.xls, col = ni * TT.nj + (j - TT.yls);
       f_ww = 1 + 4 * ((ni + 1) & 1) + 2 * ((col + 1) & 1) + ((TT.nzt + col * TT.nzt + 2) & 1);
     }
     const int t = (f_ww - 1) & 7;
     f_vx1 = s_tex[t]; f_vx2 = s_tex[8 + t]; f_wwo = s_tex[16 + t];
   }
-  float xl = awp_quot(8.0f, lam[p] + lam[ip1] + lam[jm1] + lam[ijk] + lam[km1] + lam[ik1] +
-                               lam[jk1] + lam[ijk1]);
-  float xm = awp_quot(16.0f, mu[p] + mu[ip1] + mu[jm1] + mu[ijk] + mu[km1] + mu[ik1] + mu[jk1] +
-                                 mu[ijk1]);
-  float xmu1 = awp_quot(2.0f, mu[p] + mu[km1]);
-  float xmu2 = awp_quot(2.0f, mu[p] + mu[jm1]);
-  float xmu3 = awp_quot(2.0f, mu[p] + mu[ip1]);
-  xl = xl + xm;
-  float qpa = (float)(0.0625 * (double)(qp[p] + qp[ip1] + qp[jm1] + qp[ijk] + qp[km1] +
-                                        qp[ik1] + qp[jk1] + qp[ijk1]));
   const float ca = coeff[f_ww * 2 - 2], cb = coeff[f_ww * 2 - 1];
-  float qpaw;
-  if (1.0f / (qpa * 2.0f) <= 200.0f)
-    qpaw = (float)((double)ca * (2. * (double)qpa) * (2. * (double)qpa) +
-                   (double)cb * (2. * (double)qpa));
-  else
-    qpaw = f_wwo * qpa;
-  qpaw = qpaw / f_wwo;
-  float h = 0.0625f * (qs[p] + qs[ip1] + qs[jm1] + qs[ijk] + qs[km1] + qs[ik1] + qs[jk1] +
-                       qs[ijk1]);
-  const float hw = dm_qweight(ca, cb, f_wwo, h);
-  float h1 = (float)(0.25 * (double)(qs[p] + qs[km1]));
-  const float h1w = dm_qweight(ca, cb, f_wwo, h1);
-  float h2 = (float)(0.250 * (double)(qs[p] + qs[jm1]));
-  const float h2w = dm_qweight(ca, cb, f_wwo, h2);
-  float h3 = (float)(0.250 * (double)(qs[p] + qs[ip1]));
-  const float h3w = dm_qweight(ca, cb, f_wwo, h3);
+  float xl = awp_pow2_div(8.0f, l0 + l1 + l2 + l3 + l4 + l5 + l6 + l7);
+  float xm = awp_pow2_div(16.0f, m0 + m1 + m2 + m3 + m4 + m5 + m6 + m7);
+  float xmu1 = awp_pow2_div(2.0f, m0 + m4);
+  float xmu2 = awp_pow2_div(2.0f, m0 + m2);
+  float xmu3 = awp_pow2_div(2.0f, m0 + m1);
+  xl = xl + xm;
+  // the means' power-of-two scales are exact, in binary64 as in binary32
+  const float rw = awp_rcp(f_wwo);
+  float qpa = 0.0625f * (p0 + p1 + p2 + p3 + p4 + p5 + p6 + p7);
+  const float qpaw = dm_qweight(ca, cb, f_wwo, rw, qpa, awp_q_low32(qpa));
+  float h = 0.0625f * (q0 + q1 + q2 + q3 + q4 + q5 + q6 + q7);
+  const float hw = dm_qweight(ca, cb, f_wwo, rw, h, awp_q_low64(h));
+  float h1 = 0.25f * (q0 + q4);
+  const float h1w = dm_qweight(ca, cb, f_wwo, rw, h1, awp_q_low64(h1));
+  float h2 = 0.25f * (q0 + q2);
+  const float h2w = dm_qweight(ca, cb, f_wwo, rw, h2, awp_q_low64(h2));
+  float h3 = 0.25f * (q0 + q1);
+  const float h3w = dm_qweight(ca, cb, f_wwo, rw, h3, awp_q_low64(h3));
   h = -xm * hw * dh1;
   h1 = -xmu1 * h1w * dh1;
   h2 = -xmu2 * h2w * dh1;
@@ -178,58 +189,58 @@ __global__ __launch_bounds__(256) void dstrqc2_kernel(
   const float vx1 = DT * (1 + f_vx2 * f_vx1);
   float f_r, f_rtmp, t, vs1, vs2, vs3;
 
-  vs1 = u1[p + 1] - u1[p];
-  vs2 = w1[p] - w1[p - S];
-  f_r = r5[p];
+  vs1 = u_kp - u0;
+  vs2 = w0 - w_im;
+  f_r = r50;
   f_rtmp = h2 * (vs1 + vs2);
-  t = xz[p] + xmu2 * (vs1 + vs2) + vx1 * f_r;
+  t = xz0 + xmu2 * (vs1 + vs2) + vx1 * f_r;
   r5[p] = f_vx2 * f_r + f_wwo * f_rtmp;
   f_rtmp = f_rtmp * (f_wwo - 1) + f_vx2 * f_r * (1 - f_vx1);
   xz[p] = (t + DT * f_rtmp) * f_dcrj;
 
-  vs1 = v1[p + 1] - v1[p];
-  vs2 = w1[p + Y] - w1[p];
-  f_r = r6[p];
+  vs1 = v_kp - v0;
+  vs2 = w_jp - w0;
+  f_r = r60;
   f_rtmp = h3 * (vs1 + vs2);
-  t = yz[p] + xmu3 * (vs1 + vs2) + vx1 * f_r;
+  t = yz0 + xmu3 * (vs1 + vs2) + vx1 * f_r;
   r6[p] = f_vx2 * f_r + f_wwo * f_rtmp;
   f_rtmp = f_rtmp * (f_wwo - 1) + f_vx2 * f_r * (1 - f_vx1);
   yz[p] = (t + DT * f_rtmp) * f_dcrj;
 
-  vs1 = u1[p + S] - u1[p];
-  vs2 = v1[p] - v1[p - Y];
-  vs3 = w1[p] - w1[p - 1];
+  vs1 = u_ip - u0;
+  vs2 = v0 - v_jm;
+  vs3 = w0 - w_km;
   float tmp = xl * (vs1 + vs2 + vs3);
   const float a1 = qpa * (vs1 + vs2 + vs3);
   tmp = tmp + DT * a1;
 
-  f_r = r1[p];
+  f_r = r10;
   f_rtmp = -h * (vs2 + vs3) + a1;
-  t = xx[p] + tmp - xm * (vs2 + vs3) + vx1 * f_r;
+  t = xx0 + tmp - xm * (vs2 + vs3) + vx1 * f_r;
   r1[p] = f_vx2 * f_r + f_wwo * f_rtmp;
   f_rtmp = f_rtmp * (f_wwo - 1) + f_vx2 * f_r * (1 - f_vx1);
   xx[p] = (t + DT * f_rtmp) * f_dcrj;
 
   // yy and zz take f_dcrj twice, as the reference (kernel.cu:2727-2740)
-  f_r = r2[p];
+  f_r = r20;
   f_rtmp = -h * (vs1 + vs3) + a1;
-  t = (yy[p] + tmp - xm * (vs1 + vs3) + vx1 * f_r) * f_dcrj;
+  t = (yy0 + tmp - xm * (vs1 + vs3) + vx1 * f_r) * f_dcrj;
   r2[p] = f_vx2 * f_r + f_wwo * f_rtmp;
   f_rtmp = f_rtmp * (f_wwo - 1) + f_vx2 * f_r * (1 - f_vx1);
   yy[p] = (t + DT * f_rtmp) * f_dcrj;
 
-  f_r = r3[p];
+  f_r = r30;
   f_rtmp = -h * (vs1 + vs2) + a1;
-  t = (zz[p] + tmp - xm * (vs1 + vs2) + vx1 * f_r) * f_dcrj;
+  t = (zz0 + tmp - xm * (vs1 + vs2) + vx1 * f_r) * f_dcrj;
   r3[p] = f_vx2 * f_r + f_wwo * f_rtmp;
   f_rtmp = f_rtmp * (f_wwo - 1) + f_vx2 * f_r * (1 - f_vx1);
   zz[p] = (t + DT * f_rtmp) * f_dcrj;
 
-  vs1 = u1[p + Y] - u1[p];
-  vs2 = v1[p] - v1[p - S];
-  f_r = r4[p];
+  vs1 = u_jp - u0;
+  vs2 = v0 - v_im;
+  f_r = r40;
   f_rtmp = h1 * (vs1 + vs2);
-  t = xy[p] + xmu1 * (vs1 + vs2) + vx1 * f_r;
+  t = xy0 + xmu1 * (vs1 + vs2) + vx1 * f_r;
   r4[p] = f_vx2 * f_r + f_wwo * f_rtmp;
   f_rtmp = f_rtmp * (f_wwo - 1) + f_vx2 * f_r * (1 - f_vx1);
   xy[p] = (t + DT * f_rtmp) * f_dcrj;
@@ -345,15 +356,10 @@ __global__ __launch_bounds__(64) void swap3_kernel(Fields9 L9, const Fields9 H9,
   const int fj0 = (j0 - 2 - AWP_NGSL) * 3 + AWP_NGSL;
 
   // weights ((1/ttl * (3-|ii|)) * (3-|jj|)) * (3-|kk|), n = (jj*5 + ii)*5 + kk;
-  // ttl = sum of the unnormalised products (kernel.cu:3053-3062), exact 729
+  // ttl = 9^3, the sum of the unnormalised products (kernel.cu:3053-3062)
   for (int n = lane; n < 125; n += 64) {
-    double ttl = 0.;
-    for (int jj = -SW_WWL; jj <= SW_WWL; ++jj)
-      for (int ii = -SW_WWL; ii <= SW_WWL; ++ii)
-        for (int kk = -SW_WWL; kk <= SW_WWL; ++kk)
-          ttl += (1. + SW_WWL - abs(jj)) * (1. + SW_WWL - abs(ii)) * (1. + SW_WWL - abs(kk));
     const int jj = n / 25 - SW_WWL, ii = (n / 5) % 5 - SW_WWL, kk = n % 5 - SW_WWL;
-    wt[n] = 1 / ttl * (1. + SW_WWL - abs(ii)) * (1. + SW_WWL - abs(jj)) *
+    wt[n] = 1 / 729. * (1. + SW_WWL - abs(ii)) * (1. + SW_WWL - abs(jj)) *
             (1. + SW_WWL - abs(kk));
   }
 
@@ -396,21 +402,29 @@ __global__ __launch_bounds__(64) void swap3_kernel(Fields9 L9, const Fields9 H9,
   __syncthreads();
   if (!active) return;
   const long long pc = (long long)i * C.slc + (long long)j * C.ylc + C.kc;
-  const int np = c_swap_np[f];
-  for (int q = 0; q < np; ++q) {
-    const SwapPass P = c_swap_pass[f][q];
-    const int a0 = 3 * ti + P.oi - SW_WWL, b0 = 3 * tj + P.oj - SW_WWL, l0 = P.kh - SW_WWL;
-    float sum = 0.0f;
-    int n = 0;
-    for (int jj = 0; jj < 5; ++jj)
-      for (int ii = 0; ii < 5; ++ii) {
-        const float* col = &slab[((a0 + ii) * SW_FJ + (b0 + jj)) * SW_CP + l0];
+  // Both passes of a field at once: their sums are chains of 125 rounded
+  // additions each, and the lane waits on one chain while the other moves
+  // (96x96 coarse columns 32.3 -> 30.6 us; the rest is the slab's lines).  A
+  // field of one pass runs it twice and stores it once.
+  const SwapPass P = c_swap_pass[f][0], Q = c_swap_pass[f][1];
+  const float* const cp = &slab[((3 * ti + P.oi - SW_WWL) * SW_FJ + (3 * tj + P.oj - SW_WWL)) *
+                                SW_CP + P.kh - SW_WWL];
+  const float* const cq = &slab[((3 * ti + Q.oi - SW_WWL) * SW_FJ + (3 * tj + Q.oj - SW_WWL)) *
+                                SW_CP + Q.kh - SW_WWL];
+  float sp = 0.0f, sq = 0.0f;
+  int n = 0;
+  for (int jj = 0; jj < 5; ++jj)
 #pragma unroll
-        for (int kk = 0; kk < 5; ++kk, ++n)
-          sum = (float)((double)sum + wt[n] * (double)col[kk]);
+    for (int ii = 0; ii < 5; ++ii) {
+      const int o = (ii * SW_FJ + jj) * SW_CP;
+#pragma unroll
+      for (int kk = 0; kk < 5; ++kk, ++n) {
+        sp = (float)((double)sp + wt[n] * (double)cp[o + kk]);
+        sq = (float)((double)sq + wt[n] * (double)cq[o + kk]);
       }
-    L9.f[f][pc + P.kc] = sum;
-  }
+    }
+  L9.f[f][pc + P.kc] = sp;
+  if (c_swap_np[f] == 2) L9.f[f][pc + Q.kc] = sq;
 }
 
 bool dm_grid_pair(int fine, const char* W, const AwpGrid** gf, const AwpGrid** gc) {
@@ -503,7 +517,7 @@ void dstrqc2_common(const char* W, float* xx, float* yy, float* zz, float* xy, f
   L.i0 = s_i; L.i1 = e_i; L.j0 = s_j; L.j1 = e_j;
   L.yline = g.yline; L.slice = g.slice;
   L.dth = g.dth; L.dh1 = g.dh1; L.DT = g.DT;
-  dim3 grid(awp_cdiv(e_j - s_j + 1, 64), awp_cdiv(e_i - s_i + 1, 4));
+  dim3 grid(awp_cdiv(e_j - s_j + 1, 64), e_i - s_i + 1);
   Dm2Tex TT = {};
   if (tex_mode != DM2_TEX_ARRAYS) {
     for (int m = 0; m < 24; ++m) TT.t[m] = tex[m];
@@ -514,15 +528,15 @@ void dstrqc2_common(const char* W, float* xx, float* yy, float* zz, float* xy, f
     TT.nzt = g.nzt;
   }
   if (tex_mode == DM2_TEX_RULE)
-    hipLaunchKernelGGL(dstrqc2_kernel<DM2_TEX_RULE>, grid, dim3(64, 4), 0, St, xx, yy, zz, xy,
+    hipLaunchKernelGGL(dstrqc2_kernel<DM2_TEX_RULE>, grid, dim3(64), 0, St, xx, yy, zz, xy,
                        xz, yz, r1, r2, r3, r4, r5, r6, u1, v1, w1, lam, mu, qp, qs, dcrjx, dcrjy,
                        dcrjz, coeff, nullptr, nullptr, nullptr, nullptr, L, TT);
   else if (tex_mode == DM2_TEX_TABLE)
-    hipLaunchKernelGGL(dstrqc2_kernel<DM2_TEX_TABLE>, grid, dim3(64, 4), 0, St, xx, yy, zz, xy,
+    hipLaunchKernelGGL(dstrqc2_kernel<DM2_TEX_TABLE>, grid, dim3(64), 0, St, xx, yy, zz, xy,
                        xz, yz, r1, r2, r3, r4, r5, r6, u1, v1, w1, lam, mu, qp, qs, dcrjx, dcrjy,
                        dcrjz, coeff, nullptr, nullptr, d_ww, nullptr, L, TT);
   else
-    hipLaunchKernelGGL(dstrqc2_kernel<DM2_TEX_ARRAYS>, grid, dim3(64, 4), 0, St, xx, yy, zz, xy,
+    hipLaunchKernelGGL(dstrqc2_kernel<DM2_TEX_ARRAYS>, grid, dim3(64), 0, St, xx, yy, zz, xy,
                        xz, yz, r1, r2, r3, r4, r5, r6, u1, v1, w1, lam, mu, qp, qs, dcrjx, dcrjy,
                        dcrjz, coeff, d_vx1, d_vx2, d_ww, d_wwo, L, TT);
   awp_check_launch(W);
