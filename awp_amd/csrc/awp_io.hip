@@ -11,8 +11,9 @@
 // Defaults from sweeps on MI355X: velocity and stress workgroups of 4 waves in
 // the chunks of awp_split_march (16-wave stress workgroups, of which a CU
 // holds one, took 951 against 832 us at 384x384x256 in bfloat16 storage); the
-// curvilinear kernels in the chunks of topo_chunk; the adjoint kernels' blocks in groups of 8 j tiles over
-// all planes (adj_stress_local 551 -> 533 us at 256x256x128).
+// curvilinear kernels in the chunks of topo_chunk; the adjoint kernels' blocks
+// in groups of 8 j tiles over all planes (adj_stress_local 551 -> 533 us at
+// 256x256x128).
 static AwpTuning g_tuning = {0, 0, 10240, 10240, 0, 0, 1, 1, 0, 16, 0, 32, 2048, 0, 0, 0, 8, 0, 8, 1, 0, 0};
 AwpTuning& awp_tuning() { return g_tuning; }
 

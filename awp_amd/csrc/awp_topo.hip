@@ -14,8 +14,10 @@
 //   awp_topo_geom_custom      geom_custom, geometry/geometry.c:188-210
 //
 // Lane map: one lane per level k (64 consecutive levels per wave, so every
-// field access of a wave is one contiguous 256-byte run), waves along j,
-// workgroups along i; the top six levels run in kernels of their own.
+// field access of a wave is one contiguous 256-byte run); the waves of a
+// workgroup share one column chunk in LDS and march along i (topo_rates_kernel
+// <ST, 1> along j).  The top six levels' one-sided rows are per-lane
+// coefficients of the wave at the surface, in the same launch.
 // Every expression keeps the reference's operand order and literal types
 // (double where it writes double literals), so results match the CPU
 // oracle bit for bit.
@@ -79,9 +81,6 @@ struct TopoVelArgs {
   float iu1, iu2, iu3, su1, su2, su3;  // velocity scales (decode / encode)
   float a, nu;
 };
-
-// the reference's nu * 1.0 / A with binary32 nu and A (x 1.0 is exact)
-__device__ __forceinline__ float dbl_quot(float num, float den) { return awp_quot(num, den); }
 
 // Orders one wave's LDS stores before its lanes read each other's values
 // (release, then acquire, at wavefront scope).  Enough where a wave reads

@@ -41,9 +41,11 @@ void awp_clear_error(void);
  * not depend on them.  Keys: vel_bj, str_bj (waves per workgroup: 1, 2, 4, 8,
  * 16; 0 = automatic), vel_target_wgs, str_target_wgs, vel_ichunk, str_ichunk
  * (i-march chunking, 0 = automatic), xcd_remap, kalign (0/1), topo_vel_ichunk,
- * topo_str_ichunk, topo_q_ichunk (planes per march, 1..4096), step_ichunk
- * (0 = automatic), step_target_wgs (awp_step's i-march chunking).  Returns 0,
- * or -1 for an unknown key or a value out of range. */
+ * topo_str_ichunk, topo_q_ichunk, topo_rate_chunk (planes per march, 1..4096),
+ * step_ichunk (0 = automatic), step_target_wgs (awp_step's i-march chunking).
+ * topo_vel_split and topo_str_split are accepted and change nothing: the
+ * curvilinear velocity is one launch and the strain rates two.  Returns 0, or
+ * -1 for an unknown key or a value out of range. */
 int awp_set_tuning(const char* key, int value);
 
 /* Replaces SetDeviceConstValue, include/awp/kernel_launch.h:24-26
