@@ -3,7 +3,7 @@
 // imaging and receivers, launched from native code.
 //
 // Bound by the host on a small grid: a step of 64x64x64 keeps the GPU busy for
-// 26 us, but assembling the arguments of its launches in Python took 47 us.
+// 22 us, but assembling the arguments of its launches in Python took 47 us.
 // The arguments change over a run only by the step's number, so a run passes
 // them once: ten steps of 64x64x64 468 -> 225 us.
 #include "awp_common.h"

@@ -89,9 +89,9 @@ __global__ __launch_bounds__(64 * MAXW) void dvelcx_kernel(
 
   for (int s = 0; s < nsteps; ++s) {
     // Keeps the waves of a workgroup on one plane: they share halo lines, and
-    // drift apart over the march without it (512x512x256 834 -> 815 us,
-    // 400x300x200 349 -> 335, 243x187x101 63.4 -> 61.0; the stress update gains
-    // nothing from it).  nsteps is the same for every wave of the workgroup; a
+    // drift apart over the march without it (back to back, 512x512x256 834 ->
+    // 815 us, 400x300x200 349 -> 335, 243x187x101 63.4 -> 61.0; the stress update
+    // gains nothing from it).  nsteps is the same for every wave of the workgroup; a
     // wave that ended above no longer counts.
     __builtin_amdgcn_s_barrier();
     // readfirstlane hides the plane recurrence from loop strength reduction,

@@ -35,16 +35,6 @@ def test_column_heights_bit_exact(gpu, oracle_lib, nz):
     _velocity_stress(gpu, oracle_lib, Dims(11, 9, nz))
 
 
-@pytest.mark.parametrize("nz", [36, 65, 130, 200, 257])
-def test_wide_velocity_tiles_bit_exact(gpu, oracle_lib, nz):
-    """16 rows a workgroup, which only large grids take by themselves."""
-    gpu[2].set_tuning("vel_bj", 16)
-    try:
-        _velocity_stress(gpu, oracle_lib, Dims(11, 37, nz))
-    finally:
-        gpu[2].set_tuning("vel_bj", 0)
-
-
 @pytest.mark.parametrize("nx,ny,nz", [(256, 256, 4), (257, 256, 5), (512, 256, 4), (513, 256, 4)])
 def test_surface_ghosts_bit_exact(gpu, oracle_lib, nx, ny, nz):
     """The velocity ghosts in the stress kernel (up to 2^17 columns) and in
