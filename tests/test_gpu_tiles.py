@@ -1,7 +1,7 @@
 """The (k, j) tiles of the marching Cartesian kernels (awp_pick_tile) at the
 column heights where the rule changes: one wave and less, 64 m levels, one row
-per workgroup of 2, 3 and 4 waves, and 64-level runs beyond 256; and the two routes of the
-free-surface velocity ghosts.  Bit for bit against the oracle: the arithmetic
+per workgroup of 2, 3 and 4 waves, 64-level runs beyond 256 and 32-level runs up to 32; and the
+two routes of the free-surface velocity ghosts.  Bit for bit against the oracle: the arithmetic
 is the same expression by expression, so the tolerance is zero."""
 import ctypes as C
 
@@ -30,7 +30,7 @@ def gpu():
     return torch, lib, _lib
 
 
-@pytest.mark.parametrize("nz", [36, 61, 64, 65, 101, 128, 130, 191, 193, 255, 256, 257, 300])
+@pytest.mark.parametrize("nz", [4, 5, 31, 32, 33, 36, 61, 64, 65, 101, 128, 130, 191, 193, 255, 256, 257, 300])
 def test_column_heights_bit_exact(gpu, oracle_lib, nz):
     _velocity_stress(gpu, oracle_lib, Dims(11, 9, nz))
 

@@ -1,0 +1,62 @@
+"""The tile and march rules of the Cartesian kernels, compiled for the host:
+every level and row of a column is some lane's, exactly one's, and the lanes
+that a tile leaves idle are those its rule allows."""
+import os
+import shutil
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+NMAX = 700
+PROGRAM = r"""
+#include <stdio.h>
+#include <stdlib.h>
+#include "awp_common.h"
+#include "awp_tuning.h"
+int main() {
+  for (int n = 1; n <= %d; ++n)
+    for (int rule = 0; rule < 2; ++rule) {
+      const AwpTile t = rule ? awp_pick_full_tile(n, 0) : awp_pick_tile(n, 0, 0);
+      int wrong = 0;
+      for (int l = 0; l < 64 * t.waves; ++l) wrong += (l * t.mul >> 20) != l / t.width;
+      printf("%%d %%d %%d %%d %%d %%d %%d\n", rule, n, t.width, t.rows, t.waves, t.nkt, wrong);
+    }
+}
+""" % NMAX
+
+
+def run_host(tmp_path, program):
+    """Compile a host program against the library's headers; its output."""
+    if not Path(HIPCC).exists() and shutil.which("hipcc") is None:
+        pytest.skip("no hipcc")
+    src, exe = tmp_path / "rules.hip", tmp_path / "rules"
+    src.write_text(program)
+    subprocess.run([HIPCC, "--offload-host-only", "-std=c++17", "-O1", "-I",
+                    str(ROOT / "awp_amd" / "csrc"), str(src), "-o", str(exe)], check=True,
+                   capture_output=True)
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+    return np.array([[int(x) for x in line.split()] for line in out.splitlines()])
+
+
+@pytest.fixture(scope="module")
+def tiles(tmp_path_factory):
+    return run_host(tmp_path_factory.mktemp("tiles"), PROGRAM)
+
+
+def test_tiles_cover_the_column(tiles):
+    rule, n, width, rows, waves, nkt, wrong = tiles.T
+    assert (wrong == 0).all()
+    assert (rows >= 1).all() and (waves >= 1).all() and (waves <= 8).all()
+    assert (rows * width <= 64 * waves).all()
+    assert (nkt * width >= n).all() and ((nkt - 1) * width < n).all()
+
+
+def test_short_columns_keep_their_lanes(tiles):
+    """n levels of a 32-level run busy at least n / 32 of the lanes."""
+    for rule, n, width, rows, waves, nkt, _ in tiles:
+        if rule == 0 and n <= 32:
+            assert rows * 32 >= 64 * waves, (n, width, rows, waves)
