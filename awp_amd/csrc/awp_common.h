@@ -61,6 +61,15 @@ __device__ __forceinline__ int awp_xcd_remap(int b, int nblocks) {
   return x * q + (x < r ? x : r) + s;
 }
 
+// The same within one i-chunk of a march: of the chunk's n workgroups (n a
+// multiple of the XCDs, the last few without a tile), each XCD takes one run
+// of neighbouring tiles, so the XCDs share halo lines only at the runs' ends
+// but stay in the same few planes.  (awp_xcd_remap over the whole launch gives
+// every XCD chunks of its own, eight streams of planes far apart.)
+__host__ __device__ __forceinline__ int awp_xcd_in_chunk(int r, int n) {
+  return r % AWP_NXCD * (n / AWP_NXCD) + r / AWP_NXCD;
+}
+
 static inline int awp_cdiv(int a, int b) { return (a + b - 1) / b; }
 
 // (k, j) tile of the marching Cartesian kernels: a workgroup of `waves` waves

@@ -280,7 +280,7 @@ bool plast_setup(const char* W, int nzt, int xls, int xre, int yls, int yre, int
   L.nkt = L.tile.nkt;
   L.njt = awp_cdiv(L.j1 - L.j0 + 1, L.tile.rows);
   int nic, ichunk;
-  awp_split_march(L.ni, L.nkt * L.njt, L.tile.waves, 0, 10240, &nic, &ichunk);
+  awp_split_march(L.ni, L.nkt * L.njt, L.tile.waves, 0, 10240, 16, &nic, &ichunk);
   L.ichunk = ichunk;
   L.nblocks = L.nkt * L.njt * nic;
   return true;

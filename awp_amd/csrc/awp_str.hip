@@ -442,7 +442,7 @@ void dstrqc_common(const char* W, void* const* f15, const CStress6& S0, float* l
   L.njt = awp_cdiv(L.j1 - L.j0 + 1, L.tile.rows);
   int nic, ichunk;
   awp_split_march(L.ni, L.nkt * L.njt, L.tile.waves, awp_tuning().str_ichunk,
-                  awp_tuning().str_target_wgs, &nic, &ichunk);
+                  awp_tuning().str_target_wgs, 16, &nic, &ichunk);
   L.ichunk = ichunk;
   L.nblocks = L.nkt * L.njt * nic;
 #define AWP_STR_ARGS                                                                          \

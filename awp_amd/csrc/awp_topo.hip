@@ -1592,7 +1592,7 @@ void topo_stress_launch(topo_t* T, const WaveScales& W, const char* where, float
   QL.nkt = QL.tile.nkt;
   QL.njt = awp_cdiv(nj, QL.tile.rows);
   int nic;
-  awp_split_march(ni, QL.nkt * QL.njt, QL.tile.waves, awp_tuning().topo_q_ichunk, 10240, &nic,
+  awp_split_march(ni, QL.nkt * QL.njt, QL.tile.waves, awp_tuning().topo_q_ichunk, 10240, 16, &nic,
                   &QL.ichunk);
   QL.nblocks = QL.nkt * QL.njt * nic;
   const dim3 gq(QL.nblocks), bq(64 * QL.tile.waves);

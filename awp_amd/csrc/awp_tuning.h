@@ -28,20 +28,21 @@ struct AwpTuning {
 
 AwpTuning& awp_tuning();
 
-// The same for the Cartesian velocity and stress kernels: chunks of 4 to 16
-// planes towards `target` workgroups of 4 waves (10240 = 40 per CU).  Longer
-// chunks re-read fewer planes at their ends but leave the last round of
-// workgroups nearly empty: at 243x187x101 chunks of 4 against 16 planes took
-// the stress update (per-cell texture) 194 against 216 us, at 400x300x200
-// 8 against 32 took 860 against 938 us; at 512x512x256 16 and longer are level
-// (1.99 ms).  A grid too small for one round of 1280 workgroups (5 per CU) at
-// 4 planes takes fewer.
-static inline void awp_split_march(int ni, int nkj, int waves, int forced, int target, int* nic,
-                                   int* ichunk) {
+// Chunks of a march over ni planes whose tiling gives nkj workgroups of `waves`
+// waves per chunk, for the Cartesian kernels and the second curvilinear stress
+// pass: 4 to `most` planes towards `target` workgroups of 4 waves (10240 = 40
+// per CU).  Longer chunks re-read fewer planes at their ends but leave the last
+// round of workgroups nearly empty.  most = 16 for the stress updates: at
+// 243x187x101 chunks of 4 against 16 planes took the stress update (per-cell
+// texture) 194 against 216 us, at 400x300x200 8 against 32 took 860 against 938
+// us; at 512x512x256 16 and longer are level (1.99 ms).  A grid too small for
+// one round of 1280 workgroups (5 per CU) at 4 planes takes fewer.
+static inline void awp_split_march(int ni, int nkj, int waves, int forced, int target, int most,
+                                   int* nic, int* ichunk) {
   const long long planes = (long long)ni * nkj * waves / 4;
   long long c = planes / target;
   if (c < 4) c = 4;
-  if (c > 16) c = 16;
+  if (c > most) c = most;
   if (c > planes / 1280) c = planes / 1280;
   if (forced > 0) c = forced;
   if (c < 1) c = 1;

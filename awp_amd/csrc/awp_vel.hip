@@ -20,6 +20,7 @@ namespace {
 struct VelLaunch {
   int kb, k0, k1, j0, j1, i0;  // kb: k of lane 0 in tile 0; [k0, k1] active
   int nkt, njt, ichunk, ni, nblocks, remap, jfast;
+  int nper;  // > 0: awp_xcd_in_chunk order, nper workgroups per i-chunk
   AwpTile tile;
   int yline;
   long long slice;
@@ -46,7 +47,14 @@ __global__ __launch_bounds__(64 * MAXW) void dvelcx_kernel(
     const typename ST::T* __restrict__ yz, const float* __restrict__ dcrjx,
     const float* __restrict__ dcrjy, const float* __restrict__ dcrjz,
     const float* __restrict__ d1, const VelLaunch L, const WaveScales SC) {
-  const int b = L.remap ? awp_xcd_remap(blockIdx.x, L.nblocks) : (int)blockIdx.x;
+  int b = (int)blockIdx.x;
+  if (L.nper > 0) {
+    const int tl = awp_xcd_in_chunk(b % L.nper, L.nper);
+    if (tl >= L.nkt * L.njt) return;
+    b = b / L.nper * (L.nkt * L.njt) + tl;
+  } else if (L.remap) {
+    b = awp_xcd_remap(b, L.nblocks);
+  }
   int kt, jt, ic;
   awp_tile3(b, L.nkt, L.njt, L.jfast, kt, jt, ic);
   const int t = (int)threadIdx.x;
@@ -89,8 +97,8 @@ __global__ __launch_bounds__(64 * MAXW) void dvelcx_kernel(
 
   for (int s = 0; s < nsteps; ++s) {
     // Keeps the waves of a workgroup on one plane: they share halo lines, and
-    // drift apart over the march without it (back to back, 512x512x256 834 ->
-    // 815 us, 400x300x200 349 -> 335, 243x187x101 63.4 -> 61.0; the stress update
+    // drift apart over the march without it (in step order 400x300x200 346 ->
+    // 328 us, 512x512x256 826 -> 809, 243x187x101 82.5 -> 79.3; the stress update
     // gains nothing from it).  nsteps is the same for every wave of the workgroup; a
     // wave that ended above no longer counts.
     __builtin_amdgcn_s_barrier();
@@ -179,10 +187,23 @@ void launch_vel(void* const* f9, void* const* v0, float* dcrjx, float* dcrjy, fl
   typedef typename ST::T T;
   const int nkj = L.nkt * L.njt;
   int nic, ichunk;
+  // Block order.  Where a chunk has 512 waves and more (64 per XCD), the XCDs
+  // stay side by side in one chunk (awp_xcd_in_chunk), with chunks of up to 4
+  // planes in binary32, whose ends the caches still hold, and 16 in 16 bits;
+  // else every XCD has chunks of its own (awp_xcd_remap), so that a small grid's
+  // planes are read through one L2.  In step order (after the stress update), us:
+  //                     512x512x256  256x256x256  768x768x96  320x320x192  128x128x96
+  //   chunks of its own     892          252          840         273         21.2
+  //   side by side          809          241          800         260         22.6
+  // (side by side with chunks of 16: 864, 240, 838, 275; of its own with any
+  // chunk of 4 to 256 planes at 512x512x256: 868 to 905).  300x40x100 19 / 21;
+  // in bfloat16 512x512x256 638 / 629, 243x187x101 58 / 60.
+  const bool side = L.remap && nkj * L.tile.waves >= 512;
   awp_split_march(L.ni, nkj, L.tile.waves, awp_tuning().vel_ichunk, awp_tuning().vel_target_wgs,
-                  &nic, &ichunk);
+                  side && ST::fmt == AWP_FMT_F32 ? 4 : 16, &nic, &ichunk);
   L.ichunk = ichunk;
-  L.nblocks = nkj * nic;
+  L.nper = side ? awp_cdiv(nkj, AWP_NXCD) * AWP_NXCD : 0;
+  L.nblocks = (side ? L.nper : nkj) * nic;
   const dim3 grid(L.nblocks), block(64 * L.tile.waves);
 #define AWP_VEL_ARGS                                                                             \
   (const T*)f9[3], (const T*)f9[4], (const T*)f9[5], (const T*)f9[6], (const T*)f9[7],           \

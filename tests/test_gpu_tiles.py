@@ -42,6 +42,14 @@ def test_surface_ghosts_bit_exact(gpu, oracle_lib, nx, ny, nz):
     _velocity_stress(gpu, oracle_lib, Dims(nx, ny, nz))
 
 
+# 510, 514, 768 and 516 waves per i-chunk; 257 and 129 tiles leave workgroups without one
+@pytest.mark.parametrize("nx,ny,nz", [(9, 255, 101), (9, 257, 101), (5, 256, 130), (7, 515, 64)])
+def test_velocity_block_orders_bit_exact(gpu, oracle_lib, nx, ny, nz):
+    """XCDs with i-chunks of their own (chunks below 512 waves) and side by
+    side in one chunk."""
+    _velocity_stress(gpu, oracle_lib, Dims(nx, ny, nz))
+
+
 def _velocity_stress(gpu, oracle_lib, d):
     torch, lib, _lib = gpu
     st, med = random_state(d, seed=3 + d.nzt)

@@ -60,3 +60,29 @@ def test_short_columns_keep_their_lanes(tiles):
     for rule, n, width, rows, waves, nkt, _ in tiles:
         if rule == 0 and n <= 32:
             assert rows * 32 >= 64 * waves, (n, width, rows, waves)
+
+
+ORDER = r"""
+#include <stdio.h>
+#include "awp_common.h"
+int main() {
+  for (int tiles = 1; tiles <= 300; ++tiles) {
+    const int n = awp_cdiv(tiles, AWP_NXCD) * AWP_NXCD;
+    for (int r = 0; r < n; ++r) printf("%d %d %d %d\n", tiles, n, r, awp_xcd_in_chunk(r, n));
+  }
+}
+"""
+
+
+def test_chunk_order_shares_every_chunk_among_the_xcds(tmp_path):
+    """Each tile of an i-chunk is one workgroup's, each XCD (workgroup mod 8)
+    takes one run of neighbouring tiles, and no XCD more than another plus one
+    short run: all of them work on the same planes."""
+    table = run_host(tmp_path, ORDER)
+    for tiles in range(1, 301):
+        _, n, r, t = table[table[:, 0] == tiles].T
+        assert len(r) == n[0] and n[0] - tiles < 8
+        assert sorted(t) == list(range(n[0]))
+        for x in range(8):
+            run = t[r % 8 == x]
+            assert len(run) == n[0] // 8 and (np.diff(run) == 1).all()
