@@ -78,6 +78,11 @@ static inline int awp_cdiv(int a, int b) { return (a + b - 1) / b; }
 //   n <= 32: rows of 32 levels, two per wave (4 waves).  A column of n levels
 //     would keep n of a wave's 64 lanes busy: 256x256x32 velocity 40.6 against
 //     34.4 us, stress 99.5 against 74.9; in bfloat16 33.0 / 26.3 and 78.4 / 55.6;
+//   64 < n <= 96 in 16-bit storage: likewise, three runs a row.  One row of 72 to
+//     96 levels idles 32 to 56 lanes of 128, and a seam costs less where a line
+//     holds 64 cells: bfloat16 150x130x90 velocity 24.8 / 22.9 us, stress 50.9 /
+//     47.8; 512x512x96 289 / 257 and 675 / 652 (binary32 288x288x96 119 / 138
+//     and 254 / 239, so rows there);
 //   n <= 64, n a multiple of 64, n > 256: rows of 64 levels, one per wave
 //     (4 waves), so a wave's accesses are whole 128-byte lines;
 //   else: one row of all n levels, ceil(n / 64) waves.  Cut into runs, such a
@@ -92,11 +97,12 @@ static inline int awp_cdiv(int a, int b) { return (a + b - 1) / b; }
 struct AwpTile {
   int width, rows, waves, nkt, mul;  // mul: t / width = t * mul >> 20 for t < 1024
 };
-static inline AwpTile awp_pick_tile(int n, int waves, int width) {
+static inline AwpTile awp_pick_tile(int n, bool bits16, int waves, int width) {
   AwpTile t;
-  const bool row = n > 64 && n <= 256 && n % 64 != 0;
+  const bool run32 = n <= 32 || (bits16 && n > 64 && n <= 96);
+  const bool row = !run32 && n > 64 && n <= 256 && n % 64 != 0;
   t.waves = waves > 0 ? waves : row && width <= 0 ? awp_cdiv(n, 64) : 4;
-  t.width = width > 0 ? width : row ? n : n <= 32 ? 32 : 64;
+  t.width = width > 0 ? width : row ? n : run32 ? 32 : 64;
   if (t.width > 64 * t.waves) t.width = 64;
   t.rows = 64 * t.waves / t.width;
   t.nkt = awp_cdiv(n, t.width);

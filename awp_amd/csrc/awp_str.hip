@@ -437,7 +437,7 @@ void dstrqc_common(const char* W, void* const* f15, const CStress6& S0, float* l
   }
   if (L.k1 < L.k0) return;
   const int bj = awp_tuning().str_bj;
-  L.tile = awp_pick_tile(L.k1 - L.kb + 1, bj, awp_tuning().kw);
+  L.tile = awp_pick_tile(L.k1 - L.kb + 1, ST::fmt != AWP_FMT_F32, bj, awp_tuning().kw);
   L.nkt = L.tile.nkt;
   L.njt = awp_cdiv(L.j1 - L.j0 + 1, L.tile.rows);
   int nic, ichunk;

@@ -1588,7 +1588,7 @@ void topo_stress_launch(topo_t* T, const WaveScales& W, const char* where, float
   const dim3 gj(V.nint + 1, awp_cdiv(ni, V.rj), awp_cdiv(nj, V.ichunk));
   hipLaunchKernelGGL((topo_rates_kernel<ST, 1>), gj, block, rlds, st, A, G, V, rates, rstride);
   TopoQLaunch QL;
-  QL.tile = awp_pick_tile(T->nz, 0, awp_tuning().kw);
+  QL.tile = awp_pick_tile(T->nz, false, 0, awp_tuning().kw);
   QL.nkt = QL.tile.nkt;
   QL.njt = awp_cdiv(nj, QL.tile.rows);
   int nic;

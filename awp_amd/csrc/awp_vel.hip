@@ -259,7 +259,7 @@ void dvelcx_common(const char* W, void* const* f9, void* const* v0, float* dcrjx
   L.jfast = awp_tuning().vel_jfast;
   L.kb = awp_tuning().kalign ? (L.k0 & ~31) : L.k0;
   const int bj = awp_tuning().vel_bj;
-  L.tile = awp_pick_tile(L.k1 - L.kb + 1, bj, awp_tuning().kw);
+  L.tile = awp_pick_tile(L.k1 - L.kb + 1, ST::fmt != AWP_FMT_F32, bj, awp_tuning().kw);
   L.nkt = L.tile.nkt;
   L.njt = awp_cdiv(L.j1 - L.j0 + 1, L.tile.rows);
   if (L.k1 < L.k0) return;

@@ -19,8 +19,8 @@ PROGRAM = r"""
 #include "awp_tuning.h"
 int main() {
   for (int n = 1; n <= %d; ++n)
-    for (int rule = 0; rule < 2; ++rule) {
-      const AwpTile t = rule ? awp_pick_full_tile(n, 0) : awp_pick_tile(n, 0, 0);
+    for (int rule = 0; rule < 3; ++rule) {
+      const AwpTile t = rule == 2 ? awp_pick_full_tile(n, 0) : awp_pick_tile(n, rule == 1, 0, 0);
       int wrong = 0;
       for (int l = 0; l < 64 * t.waves; ++l) wrong += (l * t.mul >> 20) != l / t.width;
       printf("%%d %%d %%d %%d %%d %%d %%d\n", rule, n, t.width, t.rows, t.waves, t.nkt, wrong);
@@ -56,10 +56,11 @@ def test_tiles_cover_the_column(tiles):
 
 
 def test_short_columns_keep_their_lanes(tiles):
-    """n levels of a 32-level run busy at least n / 32 of the lanes."""
+    """Columns of up to 32 levels, and of 65 to 96 in 16-bit storage, leave no
+    more lanes idle than runs of 32 levels."""
     for rule, n, width, rows, waves, nkt, _ in tiles:
-        if rule == 0 and n <= 32:
-            assert rows * 32 >= 64 * waves, (n, width, rows, waves)
+        if (rule < 2 and n <= 32) or (rule == 1 and 64 < n <= 96):
+            assert 64 * waves * nkt <= 32 * -(-n // 32) * rows, (n, width, rows, waves)
 
 
 ORDER = r"""
