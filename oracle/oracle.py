@@ -381,8 +381,9 @@ class OracleSolver16(OracleSolver):
     """The 16-bit storage mode (awp_amd.storage) on the oracle: the state is
     the stored 16-bit values; every launch decodes them to binary32, runs the
     FP32 oracle function and encodes the fields the launch writes.  The
-    free-surface ghosts are a pass of their own before the stress sweep, as
-    on the GPU, so the sweep reads the stored ghosts."""
+    free-surface ghosts are a pass of their own before the stress sweep, so
+    the sweep reads the stored ghosts (as on the GPU, whichever kernel forms
+    them)."""
 
     def __init__(self, medium, sources=None, receivers=None, nt_record: int = 0,
                  storage: str = "bf16", check_every: int | None = None, topography=None,
