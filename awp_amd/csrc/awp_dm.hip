@@ -26,6 +26,7 @@ struct PlaneLaunch {
   int yline;
   long long slice;
   float dth, dh1, DT;
+  int remap;  // dstrqc2: rows in XCD-contiguous order
 };
 
 // ---------------------------------------------------------------------------
@@ -88,7 +89,14 @@ struct Dm2Tex {
 // cell (columns are a yline apart), and a 288x288 level is little more than one
 // wave per SIMD: all loads go out together before any arithmetic (the
 // scheduling barrier keeps them there), and workgroups are single waves, which
-// spread evenly over the CUs: 70 -> 57 us.
+// spread evenly over the CUs (288x288 cells 70 -> 57 us within a step, 104 -> 89
+// from cold caches).  A row's medium lines serve the row before it too: on a
+// level of more than 2^18 cells, which runs in many rounds, the rows are in
+// XCD-contiguous order so that one L2 fetches them (768x768 489 -> 475 us within a
+// step; from cold caches 768x768 535 -> 510, 1152x1152 1161 -> 1119); on smaller
+// ones neighbouring rows run at the same time anyway, and plain order spreads
+// them better (from cold caches 288x288 89 against 91 us, 480x480 208 / 212,
+// 576x576 297 / 297).
 template <int TEX>
 __global__ __launch_bounds__(64) void dstrqc2_kernel(
     float* __restrict__ xx, float* __restrict__ yy, float* __restrict__ zz,
@@ -108,8 +116,10 @@ __global__ __launch_bounds__(64) void dstrqc2_kernel(
     if (tid < 24) s_tex[tid] = TT.t[tid];
     __syncthreads();
   }
-  const int j = L.j0 + (int)(blockIdx.x * 64 + threadIdx.x);
-  const int i = L.i0 + (int)blockIdx.y;
+  int b = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+  if (L.remap) b = awp_xcd_remap(b, (int)(gridDim.x * gridDim.y));
+  const int j = L.j0 + b % (int)gridDim.x * 64 + (int)threadIdx.x;
+  const int i = L.i0 + b / (int)gridDim.x;
   if (j > L.j1) return;
   const int k = AWP_ALIGN + 2;
   const long long S = L.slice, Y = L.yline;
@@ -517,6 +527,7 @@ void dstrqc2_common(const char* W, float* xx, float* yy, float* zz, float* xy, f
   L.i0 = s_i; L.i1 = e_i; L.j0 = s_j; L.j1 = e_j;
   L.yline = g.yline; L.slice = g.slice;
   L.dth = g.dth; L.dh1 = g.dh1; L.DT = g.DT;
+  L.remap = (long long)(e_i - s_i + 1) * (e_j - s_j + 1) > 1 << 18;
   dim3 grid(awp_cdiv(e_j - s_j + 1, 64), e_i - s_i + 1);
   Dm2Tex TT = {};
   if (tex_mode != DM2_TEX_ARRAYS) {

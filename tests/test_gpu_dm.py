@@ -79,7 +79,11 @@ def test_dvelc2_bit_exact(gpu, oracle_lib, pair):
     _compare(torch, dev, host, WAVE, "dvelc2")
 
 
-@pytest.mark.parametrize("pair", PAIRS, ids=lambda p: f"{p[1].nxt}x{p[1].nyt}x{p[1].nzt}")
+# and levels on either side of 2^18 cells, where the order of the rows changes
+LEVELS = PAIRS + [(Dims(170, 171, 4), Dims(510, 513, 5)), (Dims(171, 172, 4), Dims(513, 516, 5))]
+
+
+@pytest.mark.parametrize("pair", LEVELS, ids=lambda p: f"{p[1].nxt}x{p[1].nyt}x{p[1].nzt}")
 @pytest.mark.parametrize("sub", [None, (12, 30, 11, 13)])
 def test_dstrqc2_bit_exact(gpu, oracle_lib, pair, sub):
     torch, lib, _lib = gpu
