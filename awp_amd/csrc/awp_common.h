@@ -111,21 +111,32 @@ static inline AwpTile awp_pick_tile(int n, bool bits16, int waves, int width) {
 }
 
 // The tile of the plasticity kernels, which spend as many cycles on
-// arithmetic as on memory (binary64 sine, cosine and exponential): whole
-// columns (up to 256 levels, else equal parts) in the workgroup of 1 to 8
-// waves that leaves the fewest lanes idle, the smaller one among equals
-// (n = 48: 3 waves of 4 rows, all lanes; 64-level rows keep 75 %).
+// arithmetic as on memory (binary64 sine, cosine and exponential), so that idle
+// lanes cost more than seams inside a column.
+//   n <= 128: whole columns, in the workgroup of 1, 2, 3, 4 or 8 waves that
+//     leaves the fewest lanes idle, the smaller one among equals (n = 48: 3
+//     waves of 4 rows, all lanes; 64-level rows keep 75 %).  Not 5, 6 or 7:
+//     drprecpc_calc holds 100 VGPRs, four waves per SIMD, which such workgroups
+//     cannot fill evenly (256x256x96 calc 101 us with 3 waves, 158 with 5);
+//   else: runs of 64 levels, or of 32 where those leave fewer lanes idle, 4
+//     waves.  Whole columns (equal parts of them above 256) took 247 against 176
+//     us at 256x256x150, 265 / 225 at 256x256x200 and 462 / 312 at 256x256x300.
 static inline AwpTile awp_pick_full_tile(int n, int width) {
   AwpTile t;
-  t.nkt = awp_cdiv(n, 256);
-  t.width = width > 0 ? width : awp_cdiv(n, t.nkt);
   t.waves = 4;
-  float best = 0.0f;
-  for (int w = width > 0 ? 4 : 1; w <= (width > 0 ? 4 : 8); ++w) {
-    const float use = (float)(64 * w / t.width * t.width) / (float)(64 * w);
-    if (use > best + 0.001f) {
-      best = use;
-      t.waves = w;
+  if (width > 0) {
+    t.width = width;
+  } else if (n > 128) {
+    t.width = awp_cdiv(n, 32) * 32 < awp_cdiv(n, 64) * 64 ? 32 : 64;
+  } else {
+    t.width = n;
+    float best = 0.0f;
+    for (int w : {1, 2, 3, 4, 8}) {
+      const float use = (float)(64 * w / n * n) / (float)(64 * w);
+      if (use > best + 0.001f) {
+        best = use;
+        t.waves = w;
+      }
     }
   }
   t.rows = 64 * t.waves / t.width;

@@ -25,7 +25,7 @@ def gpu():
     return torch, _lib
 
 
-@pytest.mark.parametrize("nz", [36, 48, 65, 101, 256, 257])
+@pytest.mark.parametrize("nz", [36, 48, 65, 101, 128, 129, 150, 193, 256, 257])
 def test_plasticity_tiles(gpu, oracle_lib, nz):
     from awp_amd.plasticity import PlasticParams
     from tests.test_gpu_parity import _plastic_state

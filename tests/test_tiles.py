@@ -63,6 +63,15 @@ def test_short_columns_keep_their_lanes(tiles):
             assert 64 * waves * nkt <= 32 * -(-n // 32) * rows, (n, width, rows, waves)
 
 
+def test_plasticity_workgroups_fill_the_simds(tiles):
+    """drprecpc_calc runs four waves per SIMD: no workgroup of 5, 6 or 7 waves,
+    and no more lanes idle than in runs of 64 levels."""
+    for rule, n, width, rows, waves, nkt, _ in tiles:
+        if rule == 2:
+            assert waves in (1, 2, 3, 4, 8), (n, waves)
+            assert 64 * waves * nkt <= 64 * -(-n // 64) * rows, (n, width, rows, waves)
+
+
 ORDER = r"""
 #include <stdio.h>
 #include "awp_common.h"
