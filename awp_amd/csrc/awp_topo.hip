@@ -1381,17 +1381,19 @@ bool metrics_present(const TMetrics& M, const char* where) {
   return true;
 }
 
-// Chunks of the curvilinear stress kernel's k lane map for a column of nz
-// levels: nseg = min(topo_nseg, ceil(nz / 64)) waves of 64 levels per chunk,
-// so a column of up to 64 * topo_nseg levels is one chunk (nz = 192: three
-// waves, where one-wave segments of 58 outputs need four, one of them with
-// 12).  The velocity kernel
-// measured slower with chunks (1.06 against 0.99 ms at 384x384x192; its top
-// wave's one-sided rows hold the chunk's other waves at the plane barrier)
-// and keeps one-wave segments.
-void topo_tiles(int nz, VelTiles* V) {
+// Chunks of the curvilinear kernels' k lane map for a column of nz levels:
+// nseg = ceil(nz / 64) waves of 64 levels per chunk, at most `most` and
+// topo_nseg, so a column of up to 64 * nseg levels is one chunk (nz = 192: three
+// waves, where one-wave segments of 58 outputs need four, one of them with 12).
+// The velocity kernel takes chunks of 2 to 4 waves (one-wave segments at
+// 160x160x128 81 against 60 us, at 160x160x256 132 / 118) and one-wave segments
+// on columns of more than 256 levels: all waves of a chunk meet at every plane,
+// and with 5 to 8 of them 160x160x257 took 228 against 140 us, 256x256x320 610 /
+// 391 and 256x256x520 958 / 560.
+void topo_tiles(int nz, int most, VelTiles* V) {
   int nseg = awp_cdiv(nz, 64);
   const int cap = awp_tuning().topo_nseg;
+  if (nseg > most) nseg = most;
   if (nseg > cap) nseg = cap;
   if (nseg > VT_MAXW) nseg = VT_MAXW;
   if (nseg < 1) nseg = 1;
@@ -1475,7 +1477,7 @@ void topo_velocity_launch(topo_t* T, const WaveScales& W, const char* where) {
   G.ej = T->ny;
   hipStream_t st = T->stream_i;
   VelTiles V;
-  topo_tiles(T->nz, &V);
+  topo_tiles(T->nz, T->nz > 256 ? 1 : 4, &V);
   V.wsync = awp_tuning().topo_wsync;
   V.njt = awp_cdiv(T->ny, V.rj);
   V.ichunk = topo_chunk(T->nx, (V.nint + 1) * T->ny * V.nseg, 8, awp_tuning().topo_vel_ichunk);
@@ -1565,7 +1567,7 @@ void topo_stress_launch(topo_t* T, const WaveScales& W, const char* where, float
   if (G.ei <= G.bi || G.ej <= G.bj) return;
   hipStream_t st = T->stream_i;
   VelTiles V;
-  topo_tiles(T->nz, &V);
+  topo_tiles(T->nz, VT_MAXW, &V);
   V.ichunk = awp_tuning().topo_str_ichunk;
   V.wsync = awp_tuning().topo_wsync;
   dim3 block(64, V.nseg * V.rj, 1);

@@ -63,10 +63,11 @@ def test_plasticity_tiles(gpu, oracle_lib, nz):
         assert mm is None, f"nz={nz}: {n} differs: {mm}"
 
 
-# columns around one, two, three and eight waves; odd planes; few planes
+# columns around one, two, three, four and eight waves (the velocity takes one-wave
+# segments above four); odd planes; few planes
 @pytest.mark.parametrize("nx,ny,nz", [(20, 21, 18), (33, 18, 63), (18, 19, 64), (17, 34, 65),
                                       (21, 20, 127), (19, 18, 130), (18, 17, 193),
-                                      (17, 18, 520)])
+                                      (17, 18, 256), (18, 17, 257), (17, 18, 520)])
 def test_curvilinear_columns(gpu, oracle_lib, nx, ny, nz):
     torch, _lib = gpu
     from awp_amd.solver import FIELDS, Solver
