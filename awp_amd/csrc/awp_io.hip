@@ -196,10 +196,13 @@ int awp_set_tuning(const char* key, int value) {
   } else if (!strcmp(key, "kalign")) {
     t.kalign = value ? 1 : 0;
   } else if (!strcmp(key, "topo_vel_ichunk") || !strcmp(key, "topo_str_ichunk")) {
-    if (value < 1 || value > 4096) return -1;
-    (!strcmp(key, "topo_vel_ichunk") ? t.topo_vel_ichunk : t.topo_str_ichunk) = value;
+    // the velocity's march chooses its chunk (0); the one-pass stress update's
+    // is always set
+    const bool vel = !strcmp(key, "topo_vel_ichunk");
+    if (value < (vel ? 0 : 1) || value > 4096) return -1;
+    (vel ? t.topo_vel_ichunk : t.topo_str_ichunk) = value;
   } else if (!strcmp(key, "topo_q_ichunk")) {
-    if (value < 1 || value > 4096) return -1;
+    if (value < 0 || value > 4096) return -1;
     t.topo_q_ichunk = value;
   } else if (!strcmp(key, "step_ichunk")) {
     t.step_ichunk = value < 0 ? 0 : value;

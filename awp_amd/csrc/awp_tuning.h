@@ -20,10 +20,10 @@ struct AwpTuning {
   int step_jfast;       // same, fused step
   int adj_jgroup;       // adjoint kernels' block order: 0 plane by plane, else j tiles per group
   int kw;               // k-run width of the Cartesian kernels: 0 by the idle-lane rules, 32, 64
-  int topo_nseg;        // curvilinear stress kernel: waves per k chunk at most (1: one-wave segments)
+  int topo_nseg;        // curvilinear kernels: waves per k chunk at most (1: one-wave segments)
   int topo_wsync;       // curvilinear kernels: 1 wave-scope LDS sync where a wave reads only its own
   int topo_rate_chunk;  // > 0 forces the planes per march of the strain-rate launches
-  int topo_rj;          // curvilinear stress kernel: > 0 forces the j rows per workgroup
+  int topo_rj;          // curvilinear kernels: > 0 forces the j rows per workgroup
 };
 
 AwpTuning& awp_tuning();

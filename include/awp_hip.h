@@ -38,11 +38,18 @@ const char* awp_last_error_string(void);
 void awp_clear_error(void);
 
 /* Launch-shape knobs (no reference counterpart), process-global; results do
- * not depend on them.  Keys: vel_bj, str_bj (waves per workgroup: 1, 2, 4, 8,
- * 16; 0 = automatic), vel_target_wgs, str_target_wgs, vel_ichunk, str_ichunk
- * (i-march chunking, 0 = automatic), xcd_remap, kalign (0/1), topo_vel_ichunk,
- * topo_str_ichunk, topo_q_ichunk, topo_rate_chunk (planes per march, 1..4096),
- * step_ichunk (0 = automatic), step_target_wgs (awp_step's i-march chunking).
+ * not depend on them.  Keys (0 = automatic unless a range is given):
+ *   vel_bj, str_bj              waves per workgroup: 0, 1, 2, 4, 8, 16
+ *   vel_target_wgs, str_target_wgs, step_target_wgs   workgroups a march aims
+ *                               for, 1 and more
+ *   vel_ichunk, str_ichunk, step_ichunk               planes per march
+ *   topo_vel_ichunk, topo_q_ichunk, topo_rate_chunk   planes per march, up to 4096
+ *   topo_str_ichunk             the same, one-pass curvilinear stress, 1..4096
+ *   topo_nseg, topo_rj, topo_wsync   curvilinear chunks: waves at most (1..8), j
+ *                               rows per workgroup (up to 8), wave-scope sync (0/1)
+ *   kw                          k-run width of the Cartesian kernels: 0, 32, 64
+ *   xcd_remap, kalign, vel_jfast, str_jfast, step_jfast   block orders, 0/1
+ *   adj_jgroup                  adjoint block order: j tiles per group
  * topo_vel_split and topo_str_split are accepted and change nothing: the
  * curvilinear velocity is one launch and the strain rates two.  Returns 0, or
  * -1 for an unknown key or a value out of range. */

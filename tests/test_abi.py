@@ -150,3 +150,17 @@ def test_reference_struct_layouts():
         assert int(a) == want, (ref, name, a, want)
         seen += 1
     assert seen == sum(len(v) + 1 for v in members.values())
+
+
+def test_automatic_tuning_can_be_restored():
+    """Every key whose default chooses by itself takes that default, 0, back."""
+    from awp_amd import _lib
+    lib = _lib.load()
+    for key in ("vel_bj", "str_bj", "vel_ichunk", "str_ichunk", "step_ichunk", "topo_vel_ichunk",
+                "topo_q_ichunk", "topo_rate_chunk", "topo_rj", "kw"):
+        other = {"kw": 32}.get(key, 2)
+        assert lib.awp_set_tuning(key.encode(), other) == 0, key
+        assert lib.awp_set_tuning(key.encode(), 0) == 0, key
+    for key in ("topo_vel_ichunk", "topo_q_ichunk", "topo_str_ichunk"):
+        assert lib.awp_set_tuning(key.encode(), -1) == -1
+        assert lib.awp_set_tuning(key.encode(), 4097) == -1
