@@ -61,12 +61,11 @@ def _compare(torch, dev, host, names, tag):
 
 
 @pytest.mark.parametrize("dims", SIZES, ids=lambda d: f"{d.nxt}x{d.nyt}x{d.nzt}")
-@pytest.mark.parametrize("bj,ichunk,remap", [(4, 0, 1), (1, 3, 0), (8, 7, 1), (2, 1, 1), (16, 2, 1)])
-def test_dvelcx_bit_exact(gpu, oracle_lib, dims, bj, ichunk, remap):
+@pytest.mark.parametrize("bj,ichunk,remap", [(0, 0, 1), (4, 0, 1), (1, 3, 0), (8, 7, 1), (2, 1, 1),
+                                             (16, 2, 1)])
+def test_dvelcx_bit_exact(gpu, oracle_lib, tuning, dims, bj, ichunk, remap):
     torch, lib, _lib = gpu
-    _lib.set_tuning("vel_bj", bj)
-    _lib.set_tuning("vel_ichunk", ichunk)
-    _lib.set_tuning("xcd_remap", remap)
+    tuning(vel_bj=bj, vel_ichunk=ichunk, xcd_remap=remap)
     st, med = random_state(dims, seed=11 + dims.nzt)
     DH, DT = 50.0, 0.0025
     _set_grid(lib, dims, DH, DT)
@@ -82,9 +81,6 @@ def test_dvelcx_bit_exact(gpu, oracle_lib, dims, bj, ichunk, remap):
         *(_np(host[n]) for n in names), _np(med["dcrjx"]), _np(med["dcrjy"]),
         _np(med["dcrjz"]), _np(med["d1"]), dims.nxt, dims.nyt, dims.nzt, DH, DT, s_i, e_i, 0, 1)
     _compare(torch, dev, host, WAVE, "dvelcx")
-    _lib.set_tuning("vel_bj", 4)
-    _lib.set_tuning("vel_ichunk", 0)
-    _lib.set_tuning("xcd_remap", 1)
 
 
 def _run_dstrqc(torch, lib, _lib, oracle_lib, dims, variant, NPC=0, sub=None, d_i_grids=(0, 1)):
@@ -122,18 +118,12 @@ def test_dstrqc_bit_exact(gpu, oracle_lib, dims, variant):
     _run_dstrqc(torch, lib, _lib, oracle_lib, dims, variant)
 
 
-@pytest.mark.parametrize("bj,ichunk,remap", [(1, 5, 0), (8, 2, 1), (2, 0, 1), (4, 3, 1), (16, 1, 0)])
-def test_dstrqc_launch_shapes(gpu, oracle_lib, bj, ichunk, remap):
+@pytest.mark.parametrize("bj,ichunk,remap", [(0, 0, 1), (1, 5, 0), (8, 2, 1), (2, 0, 1), (4, 3, 1),
+                                             (16, 1, 0)])
+def test_dstrqc_launch_shapes(gpu, oracle_lib, tuning, bj, ichunk, remap):
     torch, lib, _lib = gpu
-    _lib.set_tuning("str_bj", bj)
-    _lib.set_tuning("str_ichunk", ichunk)
-    _lib.set_tuning("xcd_remap", remap)
-    try:
-        _run_dstrqc(torch, lib, _lib, oracle_lib, Dims(21, 19, 67), "dstrqc")
-    finally:
-        _lib.set_tuning("str_bj", 16)
-        _lib.set_tuning("str_ichunk", 0)
-        _lib.set_tuning("xcd_remap", 1)
+    tuning(str_bj=bj, str_ichunk=ichunk, xcd_remap=remap)
+    _run_dstrqc(torch, lib, _lib, oracle_lib, Dims(21, 19, 67), "dstrqc")
 
 
 def test_dstrqc_strips_and_periodic(gpu, oracle_lib):

@@ -24,10 +24,7 @@ def gpu():
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
     from awp_amd import _lib
-    lib = _lib.load()
-    for key in ("vel_bj", "str_bj", "vel_ichunk", "str_ichunk", "kw"):
-        _lib.set_tuning(key, 0)
-    return torch, lib, _lib
+    return torch, _lib.load(), _lib
 
 
 @pytest.mark.parametrize("nz", [4, 5, 31, 32, 33, 36, 61, 64, 65, 101, 128, 130, 191, 193, 255, 256, 257, 300])
