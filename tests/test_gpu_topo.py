@@ -99,26 +99,33 @@ def test_gpu_launcher_one_call_bit_exact(gpu, oracle_lib, which):
             (n, len(bad), tuple(bad[0]), a[tuple(bad[0])], b[tuple(bad[0])])
 
 
+# march chunks of one plane, of an odd number and beyond the grid; waves per
+# chunk and rows per workgroup; the workgroup barrier in place of the wave's
+SHAPES = [dict(topo_vel_ichunk=1, topo_rate_chunk=1, topo_q_ichunk=1),
+          dict(topo_vel_ichunk=7, topo_rate_chunk=5, topo_q_ichunk=3, topo_nseg=1, topo_rj=2),
+          dict(topo_vel_ichunk=4096, topo_rate_chunk=4096, topo_q_ichunk=4096, topo_rj=3),
+          dict(topo_nseg=1, topo_rj=1, topo_wsync=0)]
+
+
+def _shape_id(shape):
+    return "-".join(f"{k[5:]}={v}" for k, v in shape.items())
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("split", [1, 0])
-def test_gpu_topography_velocity_forms_bit_exact(gpu, oracle_lib, split):
-    """The curvilinear velocity update as one launch per component (the
-    default, awp_set_tuning("topo_vel_split", 1)) and as one launch for all
-    three: 40 steps bit-exact against the oracle."""
+@pytest.mark.parametrize("shape", SHAPES, ids=_shape_id)
+def test_gpu_topography_velocity_forms_bit_exact(gpu, oracle_lib, tuning, shape):
+    """The curvilinear velocity update in every launch shape: 40 steps
+    bit-exact against the oracle."""
     torch, _lib = gpu
     from awp_amd.solver import FIELDS, Solver
     from oracle.oracle import OracleSolver
-    lib = _lib.load()
     w = _workload()
     med = w.medium()
     topo = w.params["topography"]
-    assert lib.awp_set_tuning(b"topo_vel_split", split) == 0
-    try:
-        g = Solver(med, w.sources, w.receivers, nt_record=w.nt, topography=topo)
-        g.run(w.nt, check_every=10)
-        torch.cuda.synchronize()
-    finally:
-        assert lib.awp_set_tuning(b"topo_vel_split", 1) == 0
+    tuning(**{k: v for k, v in shape.items() if k not in ("topo_rate_chunk", "topo_q_ichunk")})
+    g = Solver(med, w.sources, w.receivers, nt_record=w.nt, topography=topo)
+    g.run(w.nt, check_every=10)
+    torch.cuda.synchronize()
     o = OracleSolver(med, w.sources, w.receivers, nt_record=w.nt, topography=topo)
     o.run(w.nt)
     assert np.abs(o.traces()).max() > 0
@@ -128,31 +135,24 @@ def test_gpu_topography_velocity_forms_bit_exact(gpu, oracle_lib, split):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("split", [1, 2, 0])
-def test_gpu_topography_rate_groups_bit_exact(gpu, oracle_lib, split):
-    """The strain-rate pass of the two-pass stress update as two launches
-    (normal rates, then shear sums: awp_set_tuning("topo_str_split", 1)), as
-    three (normal rates, the xy sum, the xz and yz sums: 2, the default) and
-    as one: 40 steps bit-exact against the oracle, FP32 and BF16 storage."""
+@pytest.mark.parametrize("shape", SHAPES, ids=_shape_id)
+def test_gpu_topography_rate_groups_bit_exact(gpu, oracle_lib, tuning, shape):
+    """The two-pass stress update (rates marched along i, then along j, then
+    the material pass) in every launch shape: 40 steps bit-exact against the
+    oracle, FP32 and BF16 storage."""
     torch, _lib = gpu
     from awp_amd.solver import FIELDS, Solver, Solver16
     from awp_amd.storage import FIELDS16
     from oracle.oracle import OracleSolver, OracleSolver16
-    lib = _lib.load()
     w = _workload()
     med = w.medium()
     topo = w.params["topography"]
-    default = 2
-    assert lib.awp_set_tuning(b"topo_str_split", split) == 0
-    try:
-        g = Solver(med, w.sources, w.receivers, nt_record=w.nt, topography=topo, texture="rule")
-        g.run(w.nt, check_every=10)
-        g16 = Solver16(med, w.sources, w.receivers, nt_record=w.nt, storage="bf16",
-                       topography=topo)
-        g16.run(w.nt, check_every=10)
-        torch.cuda.synchronize()
-    finally:
-        assert lib.awp_set_tuning(b"topo_str_split", default) == 0
+    tuning(**shape)
+    g = Solver(med, w.sources, w.receivers, nt_record=w.nt, topography=topo, texture="rule")
+    g.run(w.nt, check_every=10)
+    g16 = Solver16(med, w.sources, w.receivers, nt_record=w.nt, storage="bf16", topography=topo)
+    g16.run(w.nt, check_every=10)
+    torch.cuda.synchronize()
     o = OracleSolver(med, w.sources, w.receivers, nt_record=w.nt, topography=topo)
     o.run(w.nt)
     assert np.abs(o.traces()).max() > 0
@@ -285,12 +285,12 @@ def test_gpu_topography_workload_against_fp64(gpu, storage, tol):
 @pytest.mark.gpu
 @pytest.mark.parametrize("nseg", [8, 2, 1])
 def test_gpu_topography_stress_chunks_bit_exact(gpu, oracle_lib, nseg):
-    """The curvilinear stress kernel's k chunks on a 200-level column:
+    """The curvilinear kernels' k chunks on a 200-level column:
     awp_set_tuning("topo_nseg") 8 (the default: one chunk of four waves
     sharing an LDS column, 56 lanes below level 0), 2 (an interior chunk of
     two waves and the top chunk, overlapping by six levels) and 1 (one-wave
-    segments of 58 outputs).  24 steps with the two-pass (three rate groups)
-    and one-pass updates, bit-exact against the oracle."""
+    segments of 58 outputs).  24 steps with the two-pass and one-pass updates,
+    bit-exact against the oracle."""
     torch, _lib = gpu
     from awp_amd.solver import FIELDS, Solver
     from oracle.oracle import OracleSolver
@@ -321,9 +321,8 @@ def test_gpu_topography_stress_chunks_bit_exact(gpu, oracle_lib, nseg):
 def test_gpu_topography_wave_sync_bit_exact(gpu, oracle_lib, nseg, wsync):
     """The curvilinear kernels with wave-scope LDS ordering where a wave
     reads only its own LDS (awp_set_tuning("topo_wsync", 1), the default:
-    the velocity kernel, and the strain-rate kernels in one-wave segments;
-    chunks of several waves keep the workgroup barrier) and with the
-    workgroup barrier everywhere (0): 24 steps on a 200-level column,
+    one-wave segments; chunks of several waves keep the workgroup barrier)
+    and with the workgroup barrier everywhere (0): 24 steps on a 200-level column,
     bit-exact against the oracle."""
     torch, _lib = gpu
     from awp_amd.solver import FIELDS, Solver
