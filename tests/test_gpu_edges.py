@@ -120,6 +120,36 @@ def test_adjoint_band(gpu, nx, ny, nz):
         assert err < 2e-3, (n, err)
 
 
+@pytest.mark.parametrize("nx,ny,nz", [(9, 7, 4), (21, 18, 64), (12, 13, 70)])
+def test_adjoint_flush_of_the_grid(gpu, nx, ny, nz):
+    """awp_adjoint_flush_grid as awp_adjoint_flush of each array, which are zero
+    outside the cells that awp_adjoint_step writes."""
+    torch, _lib = gpu
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    d = Dims(nx, ny, nz)
+    F, I = C.c_float, C.c_int
+    lib.SetDeviceConstValue((F * 1)(50.0), F(0.0025), (I * 1)(nx), (I * 1)(ny), (I * 1)(nz), 1, 0.0,
+                            0.0, (F * 9)(), (F * 9)())
+    gen = torch.Generator(device="cuda").manual_seed(nz)
+    (xs, xe), (ys, ye) = d.i_range, d.j_range
+    g32 = [torch.zeros(d.shape, device="cuda") for _ in range(8)]
+    for t in g32:
+        box = t[xs:xe + 1, ys:ye + 1, 32:d.ktop + 1]
+        box.copy_(torch.randn(box.shape, generator=gen, device="cuda"))
+    l32 = torch.zeros(d.shape[:2], device="cuda")
+    l32[xs:xe + 1, ys:ye + 1] = torch.randn((nx, ny), generator=gen, device="cuda")
+    r64 = lambda sh: torch.randn(sh, generator=gen, device="cuda", dtype=torch.float64)  # noqa: E731
+    g64, l64 = [r64(d.shape) for _ in range(8)], r64(d.shape[:2])
+    a32, a64 = [t.clone() for t in g32 + [l32]], [t.clone() for t in g64 + [l64]]
+    for a, b in zip(a32, a64):
+        lib.awp_adjoint_flush(a.data_ptr(), b.data_ptr(), a.numel(), st)
+    pp = lambda ts: (C.c_void_p * 8)(*[t.data_ptr() for t in ts])  # noqa: E731
+    lib.awp_adjoint_flush_grid(pp(g32), pp(g64), l32.data_ptr(), l64.data_ptr(), st)
+    _lib.check()
+    for got, want in zip(g32 + [l32] + g64 + [l64], a32 + a64):
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("off,size", [(0, 1), (0, 16), (0, 4099), (1, 4099), (4, 65537)])
 def test_move_fields(gpu, off, size):
     """Copies and clears over unaligned starts and ragged ends, nothing beyond."""
