@@ -83,6 +83,7 @@ SIGNATURES: dict[str, list] = {
     "awp_run_steps": [C.POINTER(RunArgs), _i, _i],
     "awp_step": [_fp] * 11 + [_i, _i, _i, _s],
     "awp_stream_probe": [_fp, _i, _fp, _i, C.c_longlong, _i, _i, _i, _s],
+    "awp_math_probe": [_i, _fp, _fp, _fp, C.c_longlong, _s],
     # topo_t* travels as a plain address (ctypes.byref of awp_amd.refstructs.Topo)
     "topo_set_constants": [_fp],
     "topo_velocity_interior_H": [_fp],

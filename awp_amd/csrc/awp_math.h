@@ -6,8 +6,9 @@
 // and a binary64 one to about 14.  One cell of the stress update divides
 // fifteen times: 170 of its 530 VALU instructions.  Here:
 //   * the reciprocal is v_rcp_f32 (error below 1 ulp) and one Newton step in
-//     fused arithmetic, which gives the correctly rounded 1/b (checked over
-//     all 2^23 significands);
+//     fused arithmetic, which gives the correctly rounded 1/b (not by a general
+//     theorem: by what the instruction returns, which the tests check for all
+//     2^23 significands);
 //   * a quotient is a*y corrected once by its exact residual,
 //     q = fma(fma(-a*y, b, a), y, a*y), which with y = RN(1/b) is the
 //     correctly rounded a/b (P. W. Markstein, "Computation of elementary
@@ -17,7 +18,11 @@
 //     and NaN.
 // So the quotient's bits are those of a / b wherever a, b, 1/b and a/b are
 // normal numbers whose residual (2^-24 a) is one too: |a| > 2^-100 or a = 0,
-// 2^-125 < |b| < 2^125.
+// 2^-125 < |b| < 2^125.  For smaller a the residual is flushed and the quotient
+// is a*y, within 2 ulps of a / b.  Only the plasticity kernels divide fields:
+// stresses (Pa, 2^-100 is 8e-31) by 3, by the root of their second invariant
+// and by a modulus.  Values that small take part in the results through
+// squares, which flush to zero, or are added to terms 2^24 times larger.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

@@ -20,6 +20,7 @@
 #include <utility>
 
 #include "awp_common.h"
+#include "awp_math.h"
 #include "../../include/awp_hip.h"
 
 namespace {
@@ -95,7 +96,34 @@ BatchedFn batched_for(int nin) {
   return tab[nin - 1];
 }
 
+// The functions of awp_math.h, one element a lane.
+__global__ __launch_bounds__(256) void math_probe_kernel(int op, const float* __restrict__ a,
+                                                         const float* __restrict__ b,
+                                                         float* __restrict__ out, long long n) {
+  const long long e = blockIdx.x * 256ll + threadIdx.x;
+  if (e >= n) return;
+  const float x = a[e], y = b[e];
+  out[e] = op == 0   ? awp_rcp(x)
+           : op == 1 ? awp_div(x, y)
+           : op == 2 ? awp_pow2_div(x, y)
+           : op == 3 ? (float)awp_q_low64(x)
+                     : (float)awp_q_low32(x);
+}
+
 }  // namespace
+
+extern "C" void awp_math_probe(int op, const float* a, const float* b, float* out, long long n,
+                               hipStream_t St) {
+  const char* W = "awp_math_probe";
+  if (op < 0 || op > 4 || !a || !b || !out || n < 0 || n > 256ll * 0x7fffffff) {
+    awp_set_error(AWP_ERR_ARG, "%s: op=%d n=%lld out of range, or an array is NULL", W, op, n);
+    return;
+  }
+  if (n == 0) return;
+  hipLaunchKernelGGL(math_probe_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, St, op, a,
+                     b, out, n);
+  awp_check_launch(W);
+}
 
 extern "C" int awp_stream_probe(const float* const* in, int nin, float* const* out, int nout,
                                 long long n, int vec4, int blocks, int batched, hipStream_t St) {

@@ -449,6 +449,13 @@ void awp_step(const float* const* a9, float* const* b9, float* const* r6,
 int awp_stream_probe(const float* const* in, int nin, float* const* out, int nout, long long n,
                      int vec4, int blocks, int batched, hipStream_t St);
 
+/* The kernels' own binary32 arithmetic, element by element over n: op 0
+ * out = 1/a, 1 a/b, 2 a/b for powers of two a, 3 the binary64 and 4 the
+ * binary32 test 1/(2a) <= 200 of the Q weights (0 or 1).  a and b hold n
+ * values each whatever the op; the tests compare them with IEEE arithmetic. */
+void awp_math_probe(int op, const float* a, const float* b, float* out, long long n,
+                    hipStream_t St);
+
 /* ---- The reference's structs at the topography and Lagrange boundary -----
  * The topography and Lagrange launchers take the reference's own structs by
  * pointer.  They are restated here member for member, in the reference's
