@@ -54,20 +54,14 @@ bool awp_grid_ok(int d_i, const char* where);
 // XCD-aware tile order.  The hardware hands workgroup b to XCD (b % 8); this
 // renumbers workgroups so that each XCD receives one contiguous run of logical
 // tiles, which keeps the j/k halo lines neighbouring tiles share inside one
-// L2.  The map is a bijection on [0, nblocks).
-__device__ __forceinline__ int awp_xcd_remap(int b, int nblocks) {
+// L2.  The map is a bijection on [0, nblocks).  Applied to the blocks of one
+// i-chunk of a march at a time, it keeps the XCDs in the same few planes, each
+// with a run of the chunk's tiles (where the chunk's size is no multiple of 8,
+// the runs move on by that remainder from XCD to XCD with every chunk).
+__host__ __device__ __forceinline__ int awp_xcd_remap(int b, int nblocks) {
   const int q = nblocks / AWP_NXCD, r = nblocks % AWP_NXCD;
   const int x = b % AWP_NXCD, s = b / AWP_NXCD;
   return x * q + (x < r ? x : r) + s;
-}
-
-// The same within one i-chunk of a march: of the chunk's n workgroups (n a
-// multiple of the XCDs, the last few without a tile), each XCD takes one run
-// of neighbouring tiles, so the XCDs share halo lines only at the runs' ends
-// but stay in the same few planes.  (awp_xcd_remap over the whole launch gives
-// every XCD chunks of its own, eight streams of planes far apart.)
-__host__ __device__ __forceinline__ int awp_xcd_in_chunk(int r, int n) {
-  return r % AWP_NXCD * (n / AWP_NXCD) + r / AWP_NXCD;
 }
 
 static inline int awp_cdiv(int a, int b) { return (a + b - 1) / b; }

@@ -19,8 +19,7 @@ namespace {
 
 struct VelLaunch {
   int kb, k0, k1, j0, j1, i0;  // kb: k of lane 0 in tile 0; [k0, k1] active
-  int nkt, njt, ichunk, ni, nblocks, remap, jfast;
-  int nper;  // > 0: awp_xcd_in_chunk order, nper workgroups per i-chunk
+  int nkt, njt, ichunk, ni, remap, jfast;
   AwpTile tile;
   int yline;
   long long slice;
@@ -47,14 +46,9 @@ __global__ __launch_bounds__(64 * MAXW) void dvelcx_kernel(
     const typename ST::T* __restrict__ yz, const float* __restrict__ dcrjx,
     const float* __restrict__ dcrjy, const float* __restrict__ dcrjz,
     const float* __restrict__ d1, const VelLaunch L, const WaveScales SC) {
-  int b = (int)blockIdx.x;
-  if (L.nper > 0) {
-    const int tl = awp_xcd_in_chunk(b % L.nper, L.nper);
-    if (tl >= L.nkt * L.njt) return;
-    b = b / L.nper * (L.nkt * L.njt) + tl;
-  } else if (L.remap) {
-    b = awp_xcd_remap(b, L.nblocks);
-  }
+  // Grid: (all blocks, 1), or (an i-chunk's, chunks)
+  const int x = L.remap ? awp_xcd_remap((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
+  const int b = (int)(blockIdx.y * gridDim.x) + x;
   int kt, jt, ic;
   awp_tile3(b, L.nkt, L.njt, L.jfast, kt, jt, ic);
   const int t = (int)threadIdx.x;
@@ -187,24 +181,24 @@ void launch_vel(void* const* f9, void* const* v0, float* dcrjx, float* dcrjy, fl
   typedef typename ST::T T;
   const int nkj = L.nkt * L.njt;
   int nic, ichunk;
-  // Block order.  Where a chunk has 512 waves and more (64 per XCD), the XCDs
-  // stay side by side in one chunk (awp_xcd_in_chunk), with chunks of up to 4
-  // planes in binary32, whose ends the caches still hold, and 16 in 16 bits;
-  // else every XCD has chunks of its own (awp_xcd_remap), so that a small grid's
-  // planes are read through one L2.  In step order (after the stress update), us:
+  // Block order.  Where the ten arrays exceed the 256 MB cache and a chunk has 512
+  // waves and more (64 per XCD), the XCDs stay side by side in one chunk, each
+  // with a run of its tiles, and chunks have up to 4 planes in binary32, whose ends
+  // the caches still hold, and 16 in 16 bits; else every XCD has chunks of its
+  // own, so that a small grid's planes are read through one L2.  In step order
+  // (after the stress update), us:
   //                     512x512x256  256x256x256  768x768x96  320x320x192  128x128x96
-  //   chunks of its own     892          252          840         273         21.2
-  //   side by side          809          241          800         260         22.6
+  //   chunks of its own     892          250          842         273         21.3
+  //   side by side          808          235          803         260         22.6
   // (side by side with chunks of 16: 864, 240, 838, 275; of its own with any
-  // chunk of 4 to 256 planes at 512x512x256: 868 to 905).  300x40x100 19 / 21;
-  // in bfloat16 512x512x256 638 / 629, 243x187x101 58 / 60.
-  const bool side = L.remap && nkj * L.tile.waves >= 512;
+  // chunk of 4 to 256 planes at 512x512x256: 868 to 905).  300x40x100 19 / 21,
+  // 40x300x100 19.2 / 19.8; in bfloat16 512x512x256 638 / 629, 243x187x101 58 / 60.
+  const long long bytes = L.slice * L.ni * (long long)(9 * sizeof(T) + sizeof(float));
+  const bool side = L.remap && nkj * L.tile.waves >= 512 && bytes > 256ll << 20;
   awp_split_march(L.ni, nkj, L.tile.waves, awp_tuning().vel_ichunk, awp_tuning().vel_target_wgs,
                   side && ST::fmt == AWP_FMT_F32 ? 4 : 16, &nic, &ichunk);
   L.ichunk = ichunk;
-  L.nper = side ? awp_cdiv(nkj, AWP_NXCD) * AWP_NXCD : 0;
-  L.nblocks = (side ? L.nper : nkj) * nic;
-  const dim3 grid(L.nblocks), block(64 * L.tile.waves);
+  const dim3 grid(side ? nkj : nkj * nic, side ? nic : 1), block(64 * L.tile.waves);
 #define AWP_VEL_ARGS                                                                             \
   (const T*)f9[3], (const T*)f9[4], (const T*)f9[5], (const T*)f9[6], (const T*)f9[7],           \
       (const T*)f9[8], dcrjx, dcrjy, dcrjz, d_1, L, SC

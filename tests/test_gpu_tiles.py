@@ -54,7 +54,7 @@ def test_surface_ghost_bounds_bit_exact(gpu, oracle_lib, nx, nz, variant, NPC):
 @pytest.mark.parametrize("nx,ny,nz,texture", [(256, 256, 5, "arrays"), (257, 256, 4, "arrays"),
                                               (257, 256, 6, "rule"), (20, 17, 31, "table"),
                                               (21, 18, 66, "arrays"), (20, 19, 96, "rule"),
-                                              (20, 18, 97, "arrays"), (20, 258, 101, "arrays")])
+                                              (20, 18, 97, "arrays"), (274, 258, 97, "arrays")])
 def test_16bit_surfaces_and_columns_bit_exact(gpu, oracle_lib, nx, ny, nz, texture, storage):
     torch, _, _lib = gpu
     from awp_amd import configs
@@ -84,11 +84,13 @@ def test_16bit_surfaces_and_columns_bit_exact(gpu, oracle_lib, nx, ny, nz, textu
     assert np.isfinite(top).all() and np.abs(top).max() > 0
 
 
-# 510, 514, 768 and 516 waves per i-chunk; 257 and 129 tiles leave workgroups without one
-@pytest.mark.parametrize("nx,ny,nz", [(9, 255, 101), (9, 257, 101), (5, 256, 130), (7, 515, 64)])
+# ten arrays of 253 and 259 MiB, chunks of 510, 514 and 516 waves; 257 and 129
+# tiles are no multiple of the XCDs
+@pytest.mark.parametrize("nx,ny,nz", [(186, 257, 65), (190, 257, 65), (192, 255, 65),
+                                      (99, 515, 64)])
 def test_velocity_block_orders_bit_exact(gpu, oracle_lib, nx, ny, nz):
-    """XCDs with i-chunks of their own (chunks below 512 waves) and side by
-    side in one chunk."""
+    """XCDs with i-chunks of their own and (arrays beyond 256 MiB, chunks of 512
+    waves and more) side by side in one chunk."""
     _velocity_stress(gpu, oracle_lib, Dims(nx, ny, nz))
 
 

@@ -76,23 +76,20 @@ ORDER = r"""
 #include <stdio.h>
 #include "awp_common.h"
 int main() {
-  for (int tiles = 1; tiles <= 300; ++tiles) {
-    const int n = awp_cdiv(tiles, AWP_NXCD) * AWP_NXCD;
-    for (int r = 0; r < n; ++r) printf("%d %d %d %d\n", tiles, n, r, awp_xcd_in_chunk(r, n));
-  }
+  for (int n = 1; n <= 300; ++n)
+    for (int b = 0; b < n; ++b) printf("%d %d %d\n", n, b, awp_xcd_remap(b, n));
 }
 """
 
 
-def test_chunk_order_shares_every_chunk_among_the_xcds(tmp_path):
-    """Each tile of an i-chunk is one workgroup's, each XCD (workgroup mod 8)
-    takes one run of neighbouring tiles, and no XCD more than another plus one
-    short run: all of them work on the same planes."""
+def test_xcds_share_the_blocks_in_runs(tmp_path):
+    """n blocks (a launch's or one i-chunk's): each tile is one block's, each
+    XCD (block mod 8) takes one run of neighbouring tiles, and the runs differ
+    by one tile at most."""
     table = run_host(tmp_path, ORDER)
-    for tiles in range(1, 301):
-        _, n, r, t = table[table[:, 0] == tiles].T
-        assert len(r) == n[0] and n[0] - tiles < 8
-        assert sorted(t) == list(range(n[0]))
-        for x in range(8):
-            run = t[r % 8 == x]
-            assert len(run) == n[0] // 8 and (np.diff(run) == 1).all()
+    for n in range(1, 301):
+        _, b, t = table[table[:, 0] == n].T
+        assert sorted(t) == list(range(n))
+        runs = [t[b % 8 == x] for x in range(8)]
+        assert all((np.diff(r) == 1).all() for r in runs)
+        assert max(map(len, runs)) - min(map(len, runs)) <= 1
