@@ -451,6 +451,7 @@ void dstrqc_common(const char* W, void* const* f15, const CStress6& S0, float* l
 #define AWP_STR_LAUNCH(B, FS)                                                               \
   hipLaunchKernelGGL((dstrqc_kernel<B, NEWLIT, OOP, ST, TEX, FS>), dim3(L.nblocks),         \
                      dim3(64 * L.tile.waves), 0, St, AWP_STR_ARGS)
+  // more than 8 waves: only where the tuning forces 16
   if (L.tile.waves > 8) {
     if (fs)
       AWP_STR_LAUNCH(16, true);

@@ -258,6 +258,7 @@ void dvelcx_common(const char* W, void* const* f9, void* const* v0, float* dcrjx
   L.njt = awp_cdiv(L.j1 - L.j0 + 1, L.tile.rows);
   if (L.k1 < L.k0) return;
 #define AWP_VEL_LAUNCH(B) launch_vel<B, ST, DM2>(f9, v0, dcrjx, dcrjy, dcrjz, d_1, St, L, SC)
+  // more than 8 waves: only where the tuning forces 16
   if (L.tile.waves > 8)
     AWP_VEL_LAUNCH(16);
   else
