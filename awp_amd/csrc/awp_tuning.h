@@ -30,7 +30,7 @@ AwpTuning& awp_tuning();
 
 // Chunks of a march over ni planes whose tiling gives nkj workgroups of `waves`
 // waves per chunk, for the Cartesian kernels and the second curvilinear stress
-// pass: 4 to `most` planes towards `target` workgroups of 4 waves (10240 = 40
+// pass: 4 (or `most`, if less) to `most` planes towards `target` workgroups of 4 waves (10240 = 40
 // per CU).  Longer chunks re-read fewer planes at their ends but leave the last
 // round of workgroups nearly empty.  most = 16 for the stress updates: at
 // 243x187x101 chunks of 4 against 16 planes took the stress update (per-cell

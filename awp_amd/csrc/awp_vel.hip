@@ -183,20 +183,29 @@ void launch_vel(void* const* f9, void* const* v0, float* dcrjx, float* dcrjy, fl
   int nic, ichunk;
   // Block order.  Where the ten arrays exceed the 256 MB cache and a chunk has 512
   // waves and more (64 per XCD), the XCDs stay side by side in one chunk, each
-  // with a run of its tiles, and chunks have up to 4 planes in binary32, whose ends
-  // the caches still hold, and 16 in 16 bits; else every XCD has chunks of its
-  // own, so that a small grid's planes are read through one L2.  In step order
-  // (after the stress update), us:
+  // with a run of its tiles; else every XCD has chunks of its own, so that a small
+  // grid's planes are read through one L2.  In step order (after the stress
+  // update), us:
   //                     512x512x256  256x256x256  768x768x96  320x320x192  128x128x96
   //   chunks of its own     892          250          842         273         21.3
-  //   side by side          808          235          803         260         22.6
-  // (side by side with chunks of 16: 864, 240, 838, 275; of its own with any
-  // chunk of 4 to 256 planes at 512x512x256: 868 to 905).  300x40x100 19 / 21,
-  // 40x300x100 19.2 / 19.8; in bfloat16 512x512x256 638 / 629, 243x187x101 58 / 60.
+  //   side by side          808          229          803         262         22.6
+  // (of its own with any chunk of 4 to 256 planes at 512x512x256: 868 to 905).
+  // 300x40x100 19 / 21, 40x300x100 19.2 / 19.8; in bfloat16 512x512x256 638 / 629,
+  // 243x187x101 58 / 60.
+  // Side by side, the chunks of binary32 are short, so that the caches still hold
+  // the planes at their ends: on columns of whole 64-level runs about 14 planes are
+  // in flight over the card (2 planes at 512 waves, 4 at 2048: 256x256x128 122 us
+  // against 127 with 4 and 140 with 16, 512x512x256 817 with 4 against 831 with 2
+  // and 864 with 16), on others 4 (400x300x200 331 against 342 with 2).
   const long long bytes = L.slice * L.ni * (long long)(9 * sizeof(T) + sizeof(float));
-  const bool side = L.remap && nkj * L.tile.waves >= 512 && bytes > 256ll << 20;
+  const int waves = nkj * L.tile.waves;
+  const bool side = L.remap && waves >= 512 && bytes > 256ll << 20;
+  const int most = !side || ST::fmt != AWP_FMT_F32             ? 16
+                   : L.tile.width % 64 != 0 || waves >= 4 * 512 ? 4
+                   : waves < 3 * 512                            ? 2
+                                                                : 3;
   awp_split_march(L.ni, nkj, L.tile.waves, awp_tuning().vel_ichunk, awp_tuning().vel_target_wgs,
-                  side && ST::fmt == AWP_FMT_F32 ? 4 : 16, &nic, &ichunk);
+                  most, &nic, &ichunk);
   L.ichunk = ichunk;
   const dim3 grid(side ? nkj : nkj * nic, side ? nic : 1), block(64 * L.tile.waves);
 #define AWP_VEL_ARGS                                                                             \
